@@ -383,10 +383,7 @@ void bonded_launch(NbSystem &S, const float4 *x, int64_t *force, int stride, boo
   auto *f = reinterpret_cast<unsigned long long *>(force);
   double *part = S.parts_ptr() + S.part.bond_off;
   const int G = S.part.bond_n;
-  if (nt == 0) {
-    if (E || V) launch_fill_f64(part, (size_t)G * kBondPart, s);
-    return;
-  }
+  if (nt == 0) return;  // the reduction counts no rows either
   auto go = [&](auto ev) {
     constexpr int m = decltype(ev)::value;
     if (S.precision == 1)
@@ -405,10 +402,7 @@ void pairs14_launch(NbSystem &S, const float4 *x, int64_t *force, int stride, bo
   auto *f = reinterpret_cast<unsigned long long *>(force);
   double *part = S.parts_ptr() + S.part.p14_off;
   const int G = S.part.p14_n;
-  if (S.nin14 + S.nex14 == 0) {
-    if (E || V) launch_fill_f64(part, (size_t)G * kP14Part, s);
-    return;
-  }
+  if (S.nin14 + S.nex14 == 0) return;  // the reduction counts no rows either
   auto go = [&](auto ev) {
     constexpr int m = decltype(ev)::value;
     if (S.precision == 1)

@@ -221,6 +221,7 @@ struct PartLayout {
   int p14_off = 0, p14_n = 0;
   int bond_off = 0, bond_n = 0;
   int recip_off = 0, recip_n = 0;
+  int recip_used = 0;  // rows the convolution writes (recip_n are reserved)
   int self_off = 0, self_n = 0;
   int total = 0;
 };
@@ -291,10 +292,13 @@ void bonded_launch(NbSystem &sys, const float4 *d_xyzq, int64_t *d_force,
                    int stride, bool energy, bool virial, hipStream_t s);
 void recip_launch(NbSystem &sys, const float4 *d_xyzq, int64_t *d_force,
                   int stride, bool energy, bool virial, hipStream_t s);
-void self_launch(NbSystem &sys, const float4 *d_xyzq, hipStream_t s);
-void reduce_energy_launch(NbSystem &sys, int term_mask, bool energy,
+// Adds up the partials the terms of this call wrote (and the self energy).
+void reduce_energy_launch(NbSystem &sys, const float4 *d_xyzq, int term_mask, bool energy,
                           bool virial, double *d_energy, double *d_virial,
                           hipStream_t s, bool accumulate = false);
+
+// Doubles of NbSystem::red_sums.
+size_t reduce_sums_size(const PartLayout &L, int natom);
 
 // Host topology helper shared by the C ABI.
 void build_exclusions(int natom, int nbond, const int32_t *bonds,

@@ -961,7 +961,7 @@ static void recip_t(NbSystem &S, const float4 *x, int64_t *force, int stride, bo
   if (K1 * P.ncz > S.part.recip_n) throw RuntimeError("reciprocal partial buffer too small");
   double *part = S.parts_ptr() + S.part.recip_off;
   if (EV) {
-    launch_fill_f64(part, (size_t)S.part.recip_n * kRecipPart, s);
+    S.part.recip_used = K1 * P.ncz;
     k_fftz_conv<CT, true, PRIO, BIG><<<K1 * P.ncz, P.ft, P.shz, s>>>(cgrid, P.c, plan_of(S.fz), twz,
                                                                 pre, part);
   } else {

@@ -472,12 +472,13 @@ NbSystem *create_system(const apo_nb_params &p, const apo_nb_topology &t) {
     int nbt = S->nbond + S->nub + S->nangle + S->ndihe + S->nimdihe;
     L.bond_off = off; L.bond_n = std::max(1, (nbt + 255) / 256); off += L.bond_n * kBondPart;
     // z-pass blocks are K1 * ceil(H / W) with W <= 16 set by LDS size; size
-    // for the worst case W = 1 (unused slots are zero-filled)
+    // for the worst case W = 1 (the reduction reads the rows written)
     S->zconv_blocks = S->K[1] * (S->K[0] / 2 + 1);
     L.recip_off = off; L.recip_n = S->zconv_blocks; off += L.recip_n * kRecipPart;
     L.self_off = off; L.self_n = std::max(1, (n + 255) / 256); off += L.self_n;
     L.total = off;
     S->parts.reserve(off);
+    S->red_sums.reserve(reduce_sums_size(L, n));
     APO_HIP(hipDeviceSynchronize());
   } catch (...) {
     delete S;
@@ -580,8 +581,7 @@ void calc_force(NbSystem &S, const float *xyzq, int flags, int64_t *force, int s
     direct_finalize(S, force, stride, s);
     S.toc(7, s, t0);
   }
-  if ((terms & APO_TERM_SELF) && E) self_launch(S, x4, s);
-  if (E || V) reduce_energy_launch(S, terms, E, V, energy, virial, s, acc);
+  if (E || V) reduce_energy_launch(S, x4, terms, E, V, energy, virial, s, acc);
   S.toc(5, s, t_all);
 }
 

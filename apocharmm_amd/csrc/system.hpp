@@ -140,6 +140,7 @@ struct NbSystem {
   // ---- energies / virial --------------------------------------------------------
   PartLayout part;
   DevBuf<double> parts;
+  DevBuf<double> red_sums;  // per-chunk sums of the final reduction
   // when set, the partials live here instead (the no-allocation entry point
   // lends its static device array for the length of one call)
   double *parts_ext = nullptr;

@@ -1,7 +1,9 @@
-// Small device utilities: fills, single-block scans, fixed-point conversion,
-// self energy and the final fixed-order energy/virial reduction.
+// Small device utilities: fills, single-block scans, fixed-point conversion
+// and the final fixed-order energy/virial reduction (self energy included).
 #include <algorithm>
+#include <cmath>
 #include <set>
+#include <type_traits>
 
 #include "apocharmm_amd.h"
 #include "system.hpp"
@@ -154,108 +156,160 @@ void launch_add_energy(const double *src, double *energy, hipStream_t s) {
   APO_LAUNCH_CHECK();
 }
 
-// Block-level fixed-order double reduction (tree over LDS).
-template <int NT>
-__device__ double block_sum(double v, double *sh) {
-  sh[threadIdx.x] = v;
-  __syncthreads();
-  for (int off = NT / 2; off > 0; off >>= 1) {
-    if (threadIdx.x < off) sh[threadIdx.x] += sh[threadIdx.x + off];
-    __syncthreads();
-  }
-  double r = sh[0];
-  __syncthreads();
-  return r;
-}
-
-// Sum of q^2 per block (Ewald self energy, include/cuda_pme_selfe.h:14-53).
-__global__ __launch_bounds__(256) void k_self(const float4 *xyzq, int n, double *part) {
-  __shared__ double sh[256];
-  int i = blockIdx.x * 256 + threadIdx.x;
-  double q = 0.0;
-  if (i < n) q = (double)xyzq[i].w;
-  double s = block_sum<256>(q * q, sh);
-  if (threadIdx.x == 0) part[blockIdx.x] = s;
-}
-
-void self_launch(NbSystem &S, const float4 *x, hipStream_t s) {
-  k_self<<<S.part.self_n, 256, 0, s>>>(x, S.natom, S.parts_ptr() + S.part.self_off);
-  APO_LAUNCH_CHECK();
-}
-
-// Final reduction: every component is summed over its block partials in a
-// fixed order (deterministic bits run to run).
+// Final reduction of the energy and virial partials, two launches: k_reduce_parts
+// sums kReduceRows rows of one region's partials per block (all components of
+// a row together), and k_reduce_final, one block, adds the blocks' sums and
+// writes the energies and the virial.  Both sum in a fixed order, so the bits
+// do not change from run to run.  The Ewald self energy's sum of q^2
+// (include/cuda_pme_selfe.h:14-53) is one more region, read from xyzq.
+// Latency bounds both: the partials are at most a few hundred KB.  A block per
+// 1,024 rows gives each thread four rows in flight and 13 to 35 blocks; one
+// block reading component after component, with the self energy's own launch
+// before it, took 73 us at 2,529 atoms and 92 us at 93,984, the two launches
+// take 8 and 11 us (energy and virial calls 240 -> 179 us and 1,172 -> 1,094).
+constexpr int kReduceThreads = 256, kReduceRows = 1024, kReduceAtoms = 4096;
+constexpr int kReduceWidth = 11;  // widest region (bonded)
+enum { RED_PAIR = 0, RED_P14, RED_BOND, RED_RECIP, RED_SELF, RED_NUM };
+struct ReduceRegion {
+  int off, n, width;  // offset in the partials, rows (atoms for RED_SELF), components per row
+  int start;          // first chunk
+};
 struct ReduceArgs {
-  PartLayout L;
-  int terms;
+  ReduceRegion r[RED_NUM];
+  int nchunk;
   int E, V;
   int acc;  // add into energy / virial instead of overwriting
   double self_fac;
 };
 
-__global__ __launch_bounds__(256) void k_reduce_energy(const double *parts, ReduceArgs a,
-                                                        double *energy, double *virial) {
-  __shared__ double sh[256];
-  const PartLayout &L = a.L;
-  auto region_sum = [&](int off, int nblk, int width, int comp) -> double {
-    double s = 0.0;
-    for (int b = threadIdx.x; b < nblk; b += 256) s += parts[off + b * width + comp];
-    return block_sum<256>(s, sh);
-  };
-  bool dir = a.terms & APO_TERM_DIRECT, p14 = a.terms & APO_TERM_PAIRS14,
-       bnd = a.terms & APO_TERM_BONDED, rec = a.terms & APO_TERM_RECIP,
-       slf = a.terms & APO_TERM_SELF;
-  if (a.E) {
-    double e[APO_NUM_ENERGY] = {0};
-    for (int k = 0; k < 5; k++)
-      e[k] = bnd ? region_sum(L.bond_off, L.bond_n, kBondPart, k) : 0.0;
-    e[APO_E_EWKS] = rec ? region_sum(L.recip_off, L.recip_n, kRecipPart, 0) : 0.0;
-    e[APO_E_EWSE] = slf ? a.self_fac * region_sum(L.self_off, L.self_n, 1, 0) : 0.0;
-    e[APO_E_EWEX] = p14 ? region_sum(L.p14_off, L.p14_n, kP14Part, 2) : 0.0;
-    double el = 0, vd = 0;
-    if (dir) {
-      el += region_sum(L.pair_off, L.pair_n, kPairPart, 0);
-      vd += region_sum(L.pair_off, L.pair_n, kPairPart, 1);
-    }
-    if (p14) {
-      el += region_sum(L.p14_off, L.p14_n, kP14Part, 0);
-      vd += region_sum(L.p14_off, L.p14_n, kP14Part, 1);
-    }
-    e[APO_E_ELEC] = el;
-    e[APO_E_VDW] = vd;
-    double tot = 0;
-    for (int k = 0; k < APO_E_EPOT; k++) tot += e[k];
-    e[APO_E_EPOT] = tot;
-    if (threadIdx.x == 0)
-      for (int k = 0; k < APO_NUM_ENERGY; k++) energy[k] = a.acc ? energy[k] + e[k] : e[k];
+static_assert(kPairPart <= kReduceWidth && kP14Part <= kReduceWidth &&
+                  kBondPart <= kReduceWidth && kRecipPart <= kReduceWidth,
+              "reduction width");
+
+template <int W, typename Load>
+__device__ __forceinline__ void reduce_chunk(int r0, int r1, Load &&load, double *out) {
+  __shared__ double sh[kReduceThreads / 64][W];
+  double v[W];
+#pragma unroll
+  for (int k = 0; k < W; k++) v[k] = 0.0;
+  for (int r = r0 + threadIdx.x; r < r1; r += kReduceThreads)
+#pragma unroll
+    for (int k = 0; k < W; k++) v[k] += load(r, k);
+#pragma unroll
+  for (int k = 0; k < W; k++) {
+    for (int off = 32; off > 0; off >>= 1) v[k] += __shfl_xor(v[k], off);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6][k] = v[k];
   }
-  if (a.V) {
-    double v6[6] = {0};
-    for (int c = 0; c < 6; c++) {
-      double s = 0;
-      if (dir) s += region_sum(L.pair_off, L.pair_n, kPairPart, 2 + c);
-      if (p14) s += region_sum(L.p14_off, L.p14_n, kP14Part, 3 + c);
-      if (bnd) s += region_sum(L.bond_off, L.bond_n, kBondPart, 5 + c);
-      if (rec) s += region_sum(L.recip_off, L.recip_n, kRecipPart, 1 + c);
-      v6[c] = s;
-    }
-    if (threadIdx.x == 0) {
-      const double w[9] = {v6[0], v6[1], v6[2], v6[1], v6[3], v6[4], v6[2], v6[4], v6[5]};
-      for (int k = 0; k < 9; k++) virial[k] = a.acc ? virial[k] + w[k] : w[k];
-    }
+  __syncthreads();
+  if (threadIdx.x < W) {
+    double s = 0.0;
+    for (int w = 0; w < kReduceThreads / 64; w++) s += sh[w][threadIdx.x];
+    out[threadIdx.x] = s;
   }
 }
 
-void reduce_energy_launch(NbSystem &S, int terms, bool E, bool V, double *energy,
+__global__ __launch_bounds__(kReduceThreads) void k_reduce_parts(const double *__restrict__ parts,
+                                                                 const float4 *__restrict__ xyzq,
+                                                                 ReduceArgs a,
+                                                                 double *__restrict__ sums) {
+  const int c = blockIdx.x;
+  int g = 0;
+  while (g + 1 < RED_NUM && a.r[g + 1].start <= c) g++;
+  const ReduceRegion R = a.r[g];
+  double *out = sums + (size_t)c * kReduceWidth;
+  const int per = g == RED_SELF ? kReduceAtoms : kReduceRows;
+  const int r0 = (c - R.start) * per, r1 = min(r0 + per, R.n);
+  const double *p = parts + R.off;
+  auto row = [&](auto w) {
+    constexpr int W = decltype(w)::value;
+    reduce_chunk<W>(r0, r1, [&](int r, int k) { return p[(size_t)r * W + k]; }, out);
+  };
+  if (g == RED_PAIR) row(std::integral_constant<int, kPairPart>{});
+  else if (g == RED_P14) row(std::integral_constant<int, kP14Part>{});
+  else if (g == RED_BOND) row(std::integral_constant<int, kBondPart>{});
+  else if (g == RED_RECIP) row(std::integral_constant<int, kRecipPart>{});
+  else
+    reduce_chunk<1>(r0, r1, [&](int r, int) {
+      const double q = (double)xyzq[r].w;
+      return q * q;
+    }, out);
+}
+
+// Four lanes per (region, component) add that component's chunk sums.
+__global__ __launch_bounds__(256) void k_reduce_final(const double *__restrict__ sums, ReduceArgs a,
+                                                      double *__restrict__ energy,
+                                                      double *__restrict__ virial) {
+  static_assert(4 * RED_NUM * kReduceWidth <= 256, "one thread group per component");
+  __shared__ double t[RED_NUM][kReduceWidth];
+  const int id = threadIdx.x >> 2, sub = threadIdx.x & 3;
+  const int g = id / kReduceWidth, k = id % kReduceWidth;
+  double s = 0.0;
+  if (g < RED_NUM && k < a.r[g].width) {
+    const int c1 = g + 1 < RED_NUM ? a.r[g + 1].start : a.nchunk;
+    for (int c = a.r[g].start + sub; c < c1; c += 4) s += sums[(size_t)c * kReduceWidth + k];
+  }
+  s += __shfl_xor(s, 1);
+  s += __shfl_xor(s, 2);
+  if (g < RED_NUM && sub == 0) t[g][k] = s;
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  if (a.E) {
+    double e[APO_NUM_ENERGY] = {0};
+    for (int c = 0; c < 5; c++) e[c] = t[RED_BOND][c];
+    e[APO_E_EWKS] = t[RED_RECIP][0];
+    e[APO_E_EWSE] = a.self_fac * t[RED_SELF][0];
+    e[APO_E_EWEX] = t[RED_P14][2];
+    e[APO_E_ELEC] = t[RED_PAIR][0] + t[RED_P14][0];
+    e[APO_E_VDW] = t[RED_PAIR][1] + t[RED_P14][1];
+    double tot = 0;
+    for (int c = 0; c < APO_E_EPOT; c++) tot += e[c];
+    e[APO_E_EPOT] = tot;
+    for (int c = 0; c < APO_NUM_ENERGY; c++) energy[c] = a.acc ? energy[c] + e[c] : e[c];
+  }
+  if (a.V) {
+    double v6[6];
+    for (int c = 0; c < 6; c++)
+      v6[c] = t[RED_PAIR][2 + c] + t[RED_P14][3 + c] + t[RED_BOND][5 + c] + t[RED_RECIP][1 + c];
+    const double w[9] = {v6[0], v6[1], v6[2], v6[1], v6[3], v6[4], v6[2], v6[4], v6[5]};
+    for (int c = 0; c < 9; c++) virial[c] = a.acc ? virial[c] + w[c] : w[c];
+  }
+}
+
+// chunk sums of the largest reduction this system can ask for
+size_t reduce_sums_size(const PartLayout &L, int natom) {
+  auto chunks = [](int n, int per) { return (size_t)((n + per - 1) / per); };
+  return kReduceWidth * (chunks(L.pair_n, kReduceRows) + chunks(L.p14_n, kReduceRows) +
+                         chunks(L.bond_n, kReduceRows) + chunks(L.recip_n, kReduceRows) +
+                         chunks(natom, kReduceAtoms));
+}
+
+void reduce_energy_launch(NbSystem &S, const float4 *x, int terms, bool E, bool V, double *energy,
                           double *virial, hipStream_t s, bool accumulate) {
+  const PartLayout &L = S.part;
+  const bool bonded = S.nbond + S.nub + S.nangle + S.ndihe + S.nimdihe > 0;
   ReduceArgs a;
-  a.L = S.part;
-  a.terms = terms;
+  a.nchunk = 0;
+  auto region = [&](int g, bool on, int off, int n, int width, int per) {
+    a.r[g] = ReduceRegion{off, on ? n : 0, width, a.nchunk};
+    a.nchunk += (a.r[g].n + per - 1) / per;
+  };
+  // rows the kernels of this call wrote; a term that is off or empty has none
+  region(RED_PAIR, terms & APO_TERM_DIRECT, L.pair_off, L.pair_n, kPairPart, kReduceRows);
+  region(RED_P14, (terms & APO_TERM_PAIRS14) && S.nin14 + S.nex14 > 0, L.p14_off, L.p14_n,
+         kP14Part, kReduceRows);
+  region(RED_BOND, (terms & APO_TERM_BONDED) && bonded, L.bond_off, L.bond_n, kBondPart,
+         kReduceRows);
+  region(RED_RECIP, terms & APO_TERM_RECIP, L.recip_off, L.recip_used, kRecipPart, kReduceRows);
+  region(RED_SELF, (terms & APO_TERM_SELF) && E, 0, S.natom, 1, kReduceAtoms);
   a.E = E;
   a.V = V;
   a.acc = accumulate ? 1 : 0;
   a.self_fac = -S.kappa * kCcelec / std::sqrt(kPi);
-  k_reduce_energy<<<1, 256, 0, s>>>(S.parts_ptr(), a, energy, virial);
+  if (a.nchunk) {
+    k_reduce_parts<<<a.nchunk, kReduceThreads, 0, s>>>(S.parts_ptr(), x, a, S.red_sums.get());
+    APO_LAUNCH_CHECK();
+  }
+  k_reduce_final<<<1, 256, 0, s>>>(S.red_sums.get(), a, energy, virial);
   APO_LAUNCH_CHECK();
 }
 
