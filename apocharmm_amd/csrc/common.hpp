@@ -185,18 +185,29 @@ template <typename A> struct BatchLaunch {
   }
 };
 
-// Pair-kernel constants (VFSW + Ewald), CT = float (mixed) or double (FP64).
-// Switching constants follow src/CudaPMEDirectForce.cu:321-331.
+// VFSW + Ewald constants in A, CT = float (mixed) or double (FP64): the 1-4 /
+// exclusion terms.  Switching constants follow src/CudaPMEDirectForce.cu:321-331.
 template <typename CT> struct PairConsts {
-  CT sx, sy, sz;          // box / 2^32: fixed-point coordinate unit
-  // cubic boxes: the pair kernel forms r^2 in fixed-point units and converts
-  // once (s2 = sx^2); roff2u = roff^2 in those units
-  CT s2, roff2u;
-  CT roff2, ron2, rlist2;
+  CT ron2;
   CT k6, k12, dv6, dv12, roffinv3, roffinv6;
-  CT kappa, kappa2, k2log2e, two_kappa_sqrtpi;
-  CT erfc_p;              // t = 1/(1 + erfc_p * kappa r)
-  CT erfc_c[9];           // erfc(x) ~ exp(-x^2) * sum_k c_k t^k
+  CT kappa, kappa2, two_kappa_sqrtpi;
+};
+
+// Constants of the pair kernel, which works in units of h = the interval of
+// its Coulomb table (NbSystem::tab_h): a distance in these units is the table
+// index and the offset inside the interval without another multiply.
+// Lengths below are in h, energies in kcal/mol; the vdW tables the kernel
+// reads (vdwtab, vdwsq, ljtype, vdwpqa) are in the same units.
+template <typename CT> struct PairUnits {
+  CT sx, sy, sz;  // 32-bit fixed-point unit of each axis
+  CT s2;          // ISO (cubic box): sx^2, converts r^2 formed in fixed-point units
+  // cutoff the kernel compares r^2 with, and the gradient's factor to
+  // kcal/mol/A: in h, and in fixed-point units for ISO
+  CT roff2, roff2u, flush, flush_u;
+  CT ron2;
+  CT k6, k12, dv6, dv12, roffinv3, roffinv6;
+  CT kappa;
+  int ntab;       // intervals of the Coulomb table (ntab + 1 entries)
 };
 struct PairArgs {
   const int4 *posq;
@@ -205,11 +216,12 @@ struct PairArgs {
   const int *iorder;  // processing order of the items
   const uint32_t *ent;
   const int *cand_j, *meta;
+  const float4 *ewtab;
   const float2 *vdwtab, *vdwsq;
   const float2 *ljtype;  // per-type (sqrt(eps), Rmin/2) when the table follows the rule
   const float4 *vdwpqa;  // switched vdW coefficients (P, Q, A12) per type pair, few types
   int ntypes;
-  PairConsts<float> P;
+  PairUnits<float> P;
   float qfac;
   unsigned long long *fsort;
   int ss;

@@ -1,7 +1,8 @@
 // calc_force without device allocation (apo_nb_calc_force_noalloc).
 //
 // The energy / virial partial sums of one force call (per-block FP64 partials
-// of the pair, 1-4, bonded and reciprocal terms, reduced by k_reduce_parts) go to `scratch`, a file-scope device array of
+// of the pair, 1-4, bonded and reciprocal terms, reduced by k_reduce_parts) go
+// to `scratch`, a file-scope device array of
 // kScratchDoubles doubles instead of the system's own buffer, and the call
 // never grows the neighbor-list buffers.  Every slot the reduction reads is
 // written by the same call, so nothing carries over between calls; calls that

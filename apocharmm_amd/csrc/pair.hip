@@ -14,15 +14,25 @@
 //    wraps to the minimum image exactly, then converts to float;
 //  * forces accumulate in FP32 within a step/item and are rounded to int64
 //    2^-40 fixed point per flush, so results are bitwise reproducible.
+#include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "system.hpp"
 
 namespace apo {
 
 template <typename CT> struct Vec2;
-template <> struct Vec2<float> { using T = float2; };
-template <> struct Vec2<double> { using T = double2; };
+template <> struct Vec2<float> {
+  using T = float2;
+  using Ew = float4;  // Coulomb table: kEw of these per entry
+  static constexpr int kEw = 1;
+};
+template <> struct Vec2<double> {
+  using T = double2;
+  using Ew = double2;
+  static constexpr int kEw = 3;
+};
 
 __device__ __forceinline__ unsigned long long fx_round(float v) {
   return (unsigned long long)(long long)__builtin_rintf(v * 1099511627776.0f);
@@ -31,22 +41,25 @@ __device__ __forceinline__ unsigned long long fx_round(double v) {
   return (unsigned long long)(long long)__builtin_rint(v * 1099511627776.0);
 }
 
-// Coulomb part: returns r dU/dr; u = U.
-__device__ __forceinline__ float ewald_pair(float r2, float r, float rinv, float qq,
-                                            const PairConsts<float> &P, float &u) {
-  const float e2 = __builtin_amdgcn_exp2f(-P.k2log2e * r2);  // exp(-k^2 r^2)
-  const float t = __builtin_amdgcn_rcpf(fmaf(P.erfc_p, r, 1.0f));
-  float p = P.erfc_c[8];
-#pragma unroll
-  for (int k = 7; k >= 0; k--) p = fmaf(p, t, P.erfc_c[k]);
-  u = qq * (e2 * p) * rinv;
-  return -qq * P.two_kappa_sqrtpi * e2 - u;
+// Coulomb factor f(r) = erfc(k r) + 2 k r / sqrt(pi) exp(-k^2 r^2) from the
+// per-interval polynomials in LDS (NbSystem::ewtab): r in units of the
+// interval, r <= ntab + 1 (the last entry serves r that rounds up to r_off).
+// In FP32 this is one 16-byte LDS read and six instructions where exp2, rcp and
+// a degree-8 erfc polynomial took about twenty issue slots (VALU instructions
+// of one launch at 93,984 atoms 73.2 M -> 62.9 M).  Kernel alone: 140 -> 134 us
+// there, 57 -> 49 with the virial at 26,988 atoms, FP64 with energies and virial
+// 207 -> 154 at 11,748.  What bounds it then is the latency of one pair's chain
+// (rsq, table read, cubic) over the four waves a SIMD holds.
+__device__ __forceinline__ float coulomb_factor(const float4 *tab, float r) {
+  const float4 c = tab[(unsigned)r];
+  const float u = __builtin_amdgcn_fractf(r);
+  return fmaf(fmaf(fmaf(c.w, u, c.z), u, c.y), u, c.x);
 }
-__device__ __forceinline__ double ewald_pair(double r2, double r, double rinv, double qq,
-                                             const PairConsts<double> &P, double &u) {
-  const double e2 = exp(-P.kappa2 * r2);
-  u = qq * erfc(P.kappa * r) * rinv;
-  return -qq * P.two_kappa_sqrtpi * e2 - u;
+__device__ __forceinline__ double coulomb_factor(const double2 *tab, double r) {
+  const unsigned k = (unsigned)r;
+  const double u = r - (double)k;
+  const double2 a = tab[3 * k], b = tab[3 * k + 1], c = tab[3 * k + 2];
+  return fma(fma(fma(fma(fma(c.y, u, c.x), u, b.y), u, b.x), u, a.y), u, a.x);
 }
 
 __device__ __forceinline__ float rsqrt_ct(float x) { return __builtin_amdgcn_rsqf(x); }
@@ -102,10 +115,17 @@ template <typename T2> static int pair_tab_mode(int ntypes, bool combine) {
   if ((size_t)ntypes * (ntypes + 1) / 2 * sizeof(T2) <= kMaxTriLdsBytes) return TAB_TRI;
   return combine && sizeof(T2) == sizeof(float2) ? TAB_COMBINE : TAB_GLOBAL;
 }
-template <typename T2> static size_t pair_tab_lds_bytes(int mode, int ntypes) {
-  if (mode == TAB_PQA) return 2 * (size_t)ntypes * ntypes * sizeof(float4);
-  return mode == TAB_SQUARE ? (size_t)ntypes * ntypes * sizeof(T2)
-                            : (mode == TAB_TRI ? (size_t)ntypes * (ntypes + 1) / 2 * sizeof(T2) : 0);
+// bytes of the Coulomb table, which precedes the vdW table in LDS
+template <typename CT> __host__ __device__ __forceinline__ int ew_lds_bytes(int ntab) {
+  return (ntab + 1) * Vec2<CT>::kEw * (int)sizeof(typename Vec2<CT>::Ew);
+}
+template <typename T2> static size_t pair_tab_lds_bytes(int mode, int ntypes, int ntab) {
+  using CT = std::conditional_t<sizeof(T2) == sizeof(float2), float, double>;
+  const size_t ew = ew_lds_bytes<CT>(ntab);
+  if (mode == TAB_PQA) return ew + 2 * (size_t)ntypes * ntypes * sizeof(float4);
+  return ew + (mode == TAB_SQUARE
+                   ? (size_t)ntypes * ntypes * sizeof(T2)
+                   : (mode == TAB_TRI ? (size_t)ntypes * (ntypes + 1) / 2 * sizeof(T2) : 0));
 }
 
 // One wave64 = one work item: an i-group of kGroup consecutive sorted slots
@@ -117,10 +137,11 @@ template <typename T2> static size_t pair_tab_lds_bytes(int mode, int ntypes) {
 // reduced once per item; j-forces are flushed per step.
 // TAB: where the vdW table is read (TAB_GLOBAL / TAB_SQUARE / TAB_TRI /
 // TAB_COMBINE / TAB_PQA).
+// Lengths are in units of the Coulomb table's interval (PairUnits); forces are
+// scaled to A when they are flushed.
 // ISO (cubic box, mixed precision): the coordinate differences stay in
 // fixed-point units, r^2 is compared with the cutoff in those units and
-// converted once per pair, and the forces accumulate per unit and are scaled
-// to A when they are flushed.
+// converted once per pair, and the forces accumulate per unit.
 // PRUNE (list pruning fused into an MD step, mixed precision): the kernel
 // runs on the build's list and also writes the pruned copy the next steps
 // read: each entry gains the skip bits of its pairs at or beyond the prune
@@ -135,10 +156,11 @@ __device__ __forceinline__ void pair_body(
     int bid, int nb, const int4 *__restrict__ posq, const int *__restrict__ types,
     const int4 *__restrict__ items, const int *__restrict__ iorder, const uint32_t *__restrict__ ent,
     const int *__restrict__ cand_j, const int *__restrict__ meta,
+    const typename Vec2<CT>::Ew *__restrict__ ewtab,
     const typename Vec2<CT>::T *__restrict__ vdwtab, const typename Vec2<CT>::T *__restrict__ vdwsq,
     const float2 *__restrict__ ljtype, const float4 *__restrict__ vdwpqa, int ntypes,
-    const PairConsts<CT> &P, CT qfac, unsigned long long *__restrict__ fsort, int ss,
-    double *__restrict__ part, const PairConsts<double> &PE,
+    const PairUnits<CT> &P, CT qfac, unsigned long long *__restrict__ fsort, int ss,
+    double *__restrict__ part, const PairUnits<double> &PE,
     const double2 *__restrict__ vdwtab_e, uint32_t *__restrict__ ent_out,
     int4 *__restrict__ items_out, CT rp2t) {
   static_assert(!ISO || sizeof(CT) == sizeof(float), "fixed-point-unit distances are FP32 only");
@@ -146,22 +168,27 @@ __device__ __forceinline__ void pair_body(
                 "fused pruning is an MD-step variant");
   static_assert(TAB != TAB_PQA || sizeof(CT) == sizeof(float), "the PQA table is FP32 only");
   using T2 = typename Vec2<CT>::T;
+  using Ew = typename Vec2<CT>::Ew;
   extern __shared__ char smem_pair[];
-  T2 *sh_tab = reinterpret_cast<T2 *>(smem_pair);
-  float4 *sh_pqa = reinterpret_cast<float4 *>(smem_pair);
+  Ew *sh_ew = reinterpret_cast<Ew *>(smem_pair);
+  const int ew_bytes = ew_lds_bytes<CT>(P.ntab);
+  T2 *sh_tab = reinterpret_cast<T2 *>(smem_pair + ew_bytes);
+  float4 *sh_pqa = reinterpret_cast<float4 *>(smem_pair + ew_bytes);
   const int nt2 = ntypes * ntypes;
-  if (TAB == TAB_PQA) {
-    for (int k = threadIdx.x; k < 2 * nt2; k += 64) sh_pqa[k] = vdwpqa[k];
-    __syncthreads();
-  } else if (TAB == TAB_SQUARE) {
-    for (int k = threadIdx.x; k < ntypes * ntypes; k += 64) sh_tab[k] = vdwsq[k];
-    __syncthreads();
-  } else if (TAB == TAB_TRI) {
-    for (int k = threadIdx.x; k < ntypes * (ntypes + 1) / 2; k += 64) sh_tab[k] = vdwtab[k];
-    __syncthreads();
-  }
   const int lane = threadIdx.x;
   const int nitem = meta[3];
+  if (bid < nitem) {
+    for (int k = lane; k < (P.ntab + 1) * Vec2<CT>::kEw; k += 64) sh_ew[k] = ewtab[k];
+    if (TAB == TAB_PQA) {
+      for (int k = lane; k < 2 * nt2; k += 64) sh_pqa[k] = vdwpqa[k];
+    } else if (TAB == TAB_SQUARE) {
+      for (int k = lane; k < nt2; k += 64) sh_tab[k] = vdwsq[k];
+    } else if (TAB == TAB_TRI) {
+      for (int k = lane; k < ntypes * (ntypes + 1) / 2; k += 64) sh_tab[k] = vdwtab[k];
+    }
+    __syncthreads();
+  }
+  const CT flush = ISO ? P.flush_u : P.flush;
   double acc[kPairPart];
 #pragma unroll
   for (int k = 0; k < kPairPart; k++) acc[k] = 0.0;
@@ -250,32 +277,20 @@ __device__ __forceinline__ void pair_body(
           const CT r2 = ISO ? r2t * P.s2 : r2t;
           const CT rinv = rsqrt_ct(r2);
           const CT rinv2 = rinv * rinv;
-          const CT qq = qi[k] * qj;
-          CT fij;
+          const CT rinv3 = rinv2 * rinv;
+          const CT rinv6 = rinv3 * rinv3;
+          // Coulomb: r dU/dr = -qq f(r) / r
+          const CT qf = qi[k] * qj * coulomb_factor(sh_ew, r2 * rinv);
+          CT fv;
           if constexpr (TAB == TAB_PQA) {
-            // Coulomb: r dU/dr = -qq exp(-k^2 r^2) (2 k / sqrt(pi) + P(t) / r);
             // vdW: P r^-6 - Q r^-3 - A12 r^-12 with the region's coefficients
-            const CT r = r2 * rinv;
-            const CT e2 = __builtin_amdgcn_exp2f(-P.k2log2e * r2);
-            const CT t = __builtin_amdgcn_rcpf(fmaf(P.erfc_p, r, 1.0f));
-            CT p = P.erfc_c[8];
-#pragma unroll
-            for (int c = 7; c >= 0; c--) p = fmaf(p, t, P.erfc_c[c]);
-            const CT w = fmaf(p, rinv, P.two_kappa_sqrtpi);
-            const CT rinv3 = rinv2 * rinv;
-            const CT rinv6 = rinv3 * rinv3;
             const CT rinv12 = rinv6 * rinv6;
             const float4 c = *reinterpret_cast<const float4 *>(
                 reinterpret_cast<const char *>(sh_pqa) + rowi[k] + tjb + (r2 > P.ron2 ? 16 : 0));
-            CT fv = c.x * rinv6;
+            fv = c.x * rinv6;
             fv = fmaf(-c.y, rinv3, fv);
             fv = fmaf(-c.z, rinv12, fv);
-            fij = fmaf(-(qq * e2), w, fv) * rinv2;
           } else {
-            const CT r = r2 * rinv;
-            CT u_el;
-            const CT f_el = ewald_pair(r2, r, rinv, qq, P, u_el);
-            (void)u_el;
             T2 c;
             if (TAB == TAB_SQUARE) {
               c = sh_tab[rowi[k] + tj];
@@ -289,8 +304,6 @@ __device__ __forceinline__ void pair_body(
               const int aa = ti > tj ? ti : tj, bb = ti > tj ? tj : ti;
               c = TAB == TAB_TRI ? sh_tab[aa * (aa + 1) / 2 + bb] : vdwtab[aa * (aa + 1) / 2 + bb];
             }
-            const CT rinv3 = rinv * rinv2;
-            const CT rinv6 = rinv3 * rinv3;
             // force switch: in the switched region (r > r_on) the c6/c12
             // terms are k6 c6 r^-3 (r^-3 - r_off^-3) and k12 c12 r^-6 (r^-6 -
             // r_off^-6); selects between per-lane values and an fma with a -1/0
@@ -300,10 +313,10 @@ __device__ __forceinline__ void pair_body(
             const CT t6 = fma(mo, P.roffinv3, rinv3), t12 = fma(mo, P.roffinv6, rinv6);
             const CT c6k = c.x * P.k6, c12k = c.y * P.k12;
             const CT c6 = outer ? c6k : c.x, c12 = outer ? c12k : c.y;
-            const CT f_vdw = c6 * t6 * rinv3 - c12 * t12 * rinv6;
-            fij = (f_vdw + f_el) * rinv2;
+            fv = c6 * t6 * rinv3 - c12 * t12 * rinv6;
           }
-          // ISO: gradients in A^-1 x unit, scaled when flushed
+          const CT fij = fma(-qf, rinv, fv) * rinv2;
+          // gradients per h (ISO: per fixed-point unit), scaled when flushed
           fjx = fma(-fij, dx, fjx);
           fjy = fma(-fij, dy, fjy);
           fjz = fma(-fij, dz, fjz);
@@ -320,8 +333,8 @@ __device__ __forceinline__ void pair_body(
             const double ez = (double)(int)(piz[k] - pj.z) * PE.sz;
             const double er2 = ex * ex + ey * ey + ez * ez;
             const double er = sqrt(er2), erinv = 1.0 / er;
-            el += (double)qi[k] * (double)charge_of<CT>(pj.w) * kCcelec * erfc(PE.kappa * er) *
-                  erinv;
+            el += (double)qi[k] * (double)charge_of<CT>(pj.w) * (kCcelec * PE.flush) *
+                  erfc(PE.kappa * er) * erinv;
             const int ti = TAB == TAB_SQUARE ? rowi[k] / ntypes
                                              : (TAB == TAB_PQA ? rowi[k] / (ntypes * 32) : rowi[k]);
             const int aa = ti > tj ? ti : tj, bb = ti > tj ? tj : ti;
@@ -354,16 +367,16 @@ __device__ __forceinline__ void pair_body(
       }
       // j-forces that stayed zero (no pair inside r_off) cost no memory traffic
       if (fjx != (CT)0 || fjy != (CT)0 || fjz != (CT)0) {
-        atomicAdd(&fsort[jl], fx_round(ISO ? fjx * P.sx : fjx));
-        atomicAdd(&fsort[ss + jl], fx_round(ISO ? fjy * P.sx : fjy));
-        atomicAdd(&fsort[2 * (size_t)ss + jl], fx_round(ISO ? fjz * P.sx : fjz));
+        atomicAdd(&fsort[jl], fx_round(fjx * flush));
+        atomicAdd(&fsort[ss + jl], fx_round(fjy * flush));
+        atomicAdd(&fsort[2 * (size_t)ss + jl], fx_round(fjz * flush));
       }
       if (CALC_E) {
         acc[0] += el;
         acc[1] += ev;
       }
       if (CALC_V) {
-        // ISO: the products are in unit^2 x (energy / A^2)
+        // ISO: the products are in unit^2 x (energy / h^2)
         const double vs = ISO ? (double)P.s2 : 1.0;
         acc[2] += (double)v0 * vs;
         acc[3] += (double)v1 * vs;
@@ -383,9 +396,9 @@ __device__ __forceinline__ void pair_body(
     if ((lane & 3) == 0) {
       const int il = ibase + (lane >> 2);
       if (fi[0] != (CT)0 || fi[1] != (CT)0 || fi[2] != (CT)0) {
-        atomicAdd(&fsort[il], fx_round(ISO ? fi[0] * P.sx : fi[0]));
-        atomicAdd(&fsort[ss + il], fx_round(ISO ? fi[1] * P.sx : fi[1]));
-        atomicAdd(&fsort[2 * (size_t)ss + il], fx_round(ISO ? fi[2] * P.sx : fi[2]));
+        atomicAdd(&fsort[il], fx_round(fi[0] * flush));
+        atomicAdd(&fsort[ss + il], fx_round(fi[1] * flush));
+        atomicAdd(&fsort[2 * (size_t)ss + il], fx_round(fi[2] * flush));
       }
     }
   }
@@ -406,10 +419,11 @@ template <typename CT, bool CALC_E, bool CALC_V, int TAB, bool ISO, bool PRUNE>
 __global__ __launch_bounds__(64) void k_pair(
     const int4 *__restrict__ posq, const int *__restrict__ types, const int4 *__restrict__ items,
     const int *__restrict__ iorder, const uint32_t *__restrict__ ent, const int *__restrict__ cand_j, const int *__restrict__ meta,
+    const typename Vec2<CT>::Ew *__restrict__ ewtab,
     const typename Vec2<CT>::T *__restrict__ vdwtab, const typename Vec2<CT>::T *__restrict__ vdwsq,
     const float2 *__restrict__ ljtype, const float4 *__restrict__ vdwpqa, int ntypes,
-    const PairConsts<CT> P, CT qfac, unsigned long long *__restrict__ fsort, int ss,
-    double *__restrict__ part, const PairConsts<double> PE, const double2 *__restrict__ vdwtab_e,
+    const PairUnits<CT> P, CT qfac, unsigned long long *__restrict__ fsort, int ss,
+    double *__restrict__ part, const PairUnits<double> PE, const double2 *__restrict__ vdwtab_e,
     uint32_t *__restrict__ ent_out, int4 *__restrict__ items_out, CT rp2t) {
   // Register floor of 112 VGPRs (an empty asm statement that names v111): a
   // SIMD then holds at most four pair waves (448 of its 512 VGPRs) and keeps
@@ -419,7 +433,7 @@ __global__ __launch_bounds__(64) void k_pair(
   // kernel's own allocation is 92-107 VGPRs, so no spill follows.
   asm volatile("" ::: "v111");
   pair_body<CT, CALC_E, CALC_V, TAB, ISO, PRUNE>(blockIdx.x, gridDim.x, posq, types, items, iorder, ent,
-                                                 cand_j, meta, vdwtab, vdwsq, ljtype, vdwpqa,
+                                                 cand_j, meta, ewtab, vdwtab, vdwsq, ljtype, vdwpqa,
                                                  ntypes, P, qfac, fsort, ss, part, PE, vdwtab_e,
                                                  ent_out, items_out, rp2t);
 }
@@ -431,10 +445,10 @@ __global__ __launch_bounds__(64) void kb_pair(const PairArgs *__restrict__ tab,
                                               const int *__restrict__ bstart, int nsys) {
   const int s = batch_system(bstart, nsys);
   const PairArgs &a = tab[s];
-  const PairConsts<double> no_energy{};
+  const PairUnits<double> no_energy{};
   pair_body<float, false, false, TAB, ISO, false>(
       blockIdx.x - bstart[s], bstart[s + 1] - bstart[s], a.posq, a.types, a.items, a.iorder, a.ent,
-      a.cand_j, a.meta, a.vdwtab, a.vdwsq, a.ljtype, a.vdwpqa, a.ntypes, a.P, a.qfac, a.fsort,
+      a.cand_j, a.meta, a.ewtab, a.vdwtab, a.vdwsq, a.ljtype, a.vdwpqa, a.ntypes, a.P, a.qfac, a.fsort,
       a.ss, nullptr, no_energy, nullptr, nullptr, nullptr, 0.0f);
 }
 
@@ -445,6 +459,7 @@ struct PairLaunch {
   const int *iorder;
   const uint32_t *ent;
   const int *cand_j, *meta;
+  const void *ewtab;  // the precision's Coulomb table
   const float2 *ljtype;
   const float4 *vdwpqa;
   int ntypes;
@@ -464,26 +479,27 @@ struct PairLaunch {
 
 template <typename CT, bool E, bool V, int TAB, bool ISO>
 static void go_pair(const PairLaunch &L, const typename Vec2<CT>::T *tab,
-                    const typename Vec2<CT>::T *sq, const PairConsts<CT> &P, CT qfac,
-                    const PairConsts<double> &PE) {
+                    const typename Vec2<CT>::T *sq, const PairUnits<CT> &P, CT qfac,
+                    const PairUnits<double> &PE) {
+  const auto *ew = static_cast<const typename Vec2<CT>::Ew *>(L.ewtab);
   if constexpr (sizeof(CT) == sizeof(float) && !E && !V) {
     if (L.ent_out) {
       k_pair<CT, false, false, TAB, ISO, true><<<L.blocks, 64, L.lds, L.s>>>(
-          L.posq, L.types, L.items, L.iorder, L.ent, L.cand_j, L.meta, tab, sq, L.ljtype, L.vdwpqa,
+          L.posq, L.types, L.items, L.iorder, L.ent, L.cand_j, L.meta, ew, tab, sq, L.ljtype, L.vdwpqa,
           L.ntypes, P, qfac, L.fsort, L.ss, L.part, PE, L.vdwtab_e, L.ent_out, L.items_out,
           L.rp2t);
       return;
     }
   }
   k_pair<CT, E, V, TAB, ISO, false><<<L.blocks, 64, L.lds, L.s>>>(
-      L.posq, L.types, L.items, L.iorder, L.ent, L.cand_j, L.meta, tab, sq, L.ljtype, L.vdwpqa,
+      L.posq, L.types, L.items, L.iorder, L.ent, L.cand_j, L.meta, ew, tab, sq, L.ljtype, L.vdwpqa,
       L.ntypes, P,
       qfac, L.fsort, L.ss, L.part, PE, L.vdwtab_e, nullptr, nullptr, (CT)0);
 }
 template <typename CT, bool E, bool V, bool ISO>
 static void go_pair_tab(int mode, const PairLaunch &L, const typename Vec2<CT>::T *tab,
-                        const typename Vec2<CT>::T *sq, const PairConsts<CT> &P, CT qfac,
-                        const PairConsts<double> &PE) {
+                        const typename Vec2<CT>::T *sq, const PairUnits<CT> &P, CT qfac,
+                        const PairUnits<double> &PE) {
   if constexpr (sizeof(CT) == sizeof(float)) {
     if (mode == TAB_PQA) return go_pair<CT, E, V, TAB_PQA, ISO>(L, tab, sq, P, qfac, PE);
     if (mode == TAB_COMBINE) return go_pair<CT, E, V, TAB_COMBINE, ISO>(L, tab, sq, P, qfac, PE);
@@ -494,8 +510,8 @@ static void go_pair_tab(int mode, const PairLaunch &L, const typename Vec2<CT>::
 }
 template <typename CT, bool E, bool V>
 static void go_pair_iso(bool iso, int mode, const PairLaunch &L, const typename Vec2<CT>::T *tab,
-                        const typename Vec2<CT>::T *sq, const PairConsts<CT> &P, CT qfac,
-                        const PairConsts<double> &PE) {
+                        const typename Vec2<CT>::T *sq, const PairUnits<CT> &P, CT qfac,
+                        const PairUnits<double> &PE) {
   if constexpr (sizeof(CT) == sizeof(float))
     if (iso) return go_pair_tab<CT, E, V, true>(mode, L, tab, sq, P, qfac, PE);
   go_pair_tab<CT, E, V, false>(mode, L, tab, sq, P, qfac, PE);
@@ -511,8 +527,9 @@ static bool pair_iso(const NbSystem &S) {
 // the pruned copy (mixed-precision MD steps only)
 template <typename CT>
 static void launch_pair_t(NbSystem &S, const typename Vec2<CT>::T *tab,
-                          const typename Vec2<CT>::T *sq, const PairConsts<CT> &P, CT qfac, bool E,
-                          bool V, hipStream_t s, bool pruned, bool prune_out) {
+                          const typename Vec2<CT>::T *sq, const void *ewtab,
+                          const PairUnits<CT> &P, CT qfac, bool E, bool V, hipStream_t s,
+                          bool pruned, bool prune_out) {
   const int mode = pair_tab_mode<typename Vec2<CT>::T>(S.ntypes, S.lj_combine);
   pruned = pruned && !prune_out;
   const bool iso = pair_iso(S);
@@ -523,6 +540,7 @@ static void launch_pair_t(NbSystem &S, const typename Vec2<CT>::T *tab,
                pruned ? S.ent_p.get() : S.ent.get(),
                S.cand_j.get(),
                S.meta.get(),
+               ewtab,
                S.ljtype.get(),
                S.vdwpqa.get(),
                S.ntypes,
@@ -531,21 +549,21 @@ static void launch_pair_t(NbSystem &S, const typename Vec2<CT>::T *tab,
                S.parts_ptr() + S.part.pair_off,
                S.vdwtab_d.get(),
                S.pair_blocks,
-               pair_tab_lds_bytes<typename Vec2<CT>::T>(mode, S.ntypes),
+               pair_tab_lds_bytes<typename Vec2<CT>::T>(mode, S.ntypes, S.tab_n),
                s,
                prune_out ? S.ent_p.get() : nullptr,
                prune_out ? S.items_p.get() : nullptr,
                (float)(iso ? (double)S.prune_r2 / ((S.box[0] / 4294967296.0) *
                                                    (S.box[0] / 4294967296.0))
-                           : (double)S.prune_r2)};
+                           : (double)S.prune_r2 / (S.tab_h * S.tab_h))};
   if (E && V)
-    go_pair_iso<CT, true, true>(iso, mode, L, tab, sq, P, qfac, S.pc_d);
+    go_pair_iso<CT, true, true>(iso, mode, L, tab, sq, P, qfac, S.pu_d);
   else if (E)
-    go_pair_iso<CT, true, false>(iso, mode, L, tab, sq, P, qfac, S.pc_d);
+    go_pair_iso<CT, true, false>(iso, mode, L, tab, sq, P, qfac, S.pu_d);
   else if (V)
-    go_pair_iso<CT, false, true>(iso, mode, L, tab, sq, P, qfac, S.pc_d);
+    go_pair_iso<CT, false, true>(iso, mode, L, tab, sq, P, qfac, S.pu_d);
   else
-    go_pair_iso<CT, false, false>(iso, mode, L, tab, sq, P, qfac, S.pc_d);
+    go_pair_iso<CT, false, false>(iso, mode, L, tab, sq, P, qfac, S.pu_d);
   APO_LAUNCH_CHECK();
 }
 
@@ -553,11 +571,11 @@ void direct_launch(NbSystem &S, bool E, bool V, hipStream_t s, bool pruned, bool
   if (prune_out && (S.precision != 0 || E || V))
     throw InvalidArgument("fused list pruning runs in mixed-precision MD steps only");
   if (S.precision == 1)
-    launch_pair_t<double>(S, S.vdwtab_d.get(), S.vdwsq_d.get(), S.pc_d, kCcelec, E, V, s, pruned,
-                          false);
+    launch_pair_t<double>(S, S.vdwtab_d.get(), S.vdwsq_d.get(), S.ewtab_d.get(), S.pu_d,
+                          kCcelec / S.tab_h, E, V, s, pruned, false);
   else
-    launch_pair_t<float>(S, S.vdwtab.get(), S.vdwsq.get(), S.pc_f, (float)kCcelec, E, V, s,
-                         pruned, prune_out);
+    launch_pair_t<float>(S, S.vdwtab.get(), S.vdwsq.get(), S.ewtab.get(), S.pu_f,
+                         (float)(kCcelec / S.tab_h), E, V, s, pruned, prune_out);
 }
 
 // Sorted -> global order (addSortedForce, src/CudaPMEDirectForce.cu:1375-1386).
@@ -591,15 +609,18 @@ void batch_add_pair(BatchLaunch<PairArgs> &b, NbSystem &S, int blocks) {
   if (S.precision != 0) throw InvalidArgument("fused batches run the mixed-precision path");
   PairArgs a{S.posq.get(), S.type_s.get(), S.items.get(), S.item_order.get(), S.ent.get(),
              S.cand_j.get(),
-             S.meta.get(), S.vdwtab.get(), S.vdwsq.get(), S.ljtype.get(), S.vdwpqa.get(),
-             S.ntypes, S.pc_f, (float)kCcelec,
+             S.meta.get(), S.ewtab.get(), S.vdwtab.get(), S.vdwsq.get(), S.ljtype.get(),
+             S.vdwpqa.get(), S.ntypes, S.pu_f, (float)(kCcelec / S.tab_h),
              reinterpret_cast<unsigned long long *>(S.fsort.get()), S.ssort};
-  // LDS of every LDS layout: the launch uses the one every system allows
-  b.add(a, blocks, std::max({pair_tab_lds_bytes<float2>(TAB_SQUARE, S.ntypes),
-                             pair_tab_lds_bytes<float2>(TAB_TRI, S.ntypes),
-                             S.ntypes <= kMaxTypesPqa
-                                 ? pair_tab_lds_bytes<float2>(TAB_PQA, S.ntypes)
-                                 : (size_t)0}));
+  // LDS of every layout this system allows: the launch uses one that every
+  // system of the batch allows
+  const size_t tri = pair_tab_lds_bytes<float2>(TAB_TRI, S.ntypes, S.tab_n);
+  size_t lds = pair_tab_lds_bytes<float2>(TAB_GLOBAL, S.ntypes, S.tab_n);
+  if (tri <= lds + kMaxTriLdsBytes) lds = tri;
+  for (int m : {TAB_SQUARE, TAB_PQA})
+    if (S.ntypes <= (m == TAB_PQA ? kMaxTypesPqa : kMaxTypesLds))
+      lds = std::max(lds, pair_tab_lds_bytes<float2>(m, S.ntypes, S.tab_n));
+  b.add(a, blocks, lds);
 }
 template <bool ISO>
 static void batch_pair_t(BatchLaunch<PairArgs> &b, int mode, hipStream_t s) {
@@ -611,9 +632,9 @@ static void batch_pair_t(BatchLaunch<PairArgs> &b, int mode, hipStream_t s) {
   else if (mode == TAB_TRI)
     kb_pair<TAB_TRI, ISO><<<b.blocks(), 64, b.lds, s>>>(b.d_args.get(), b.d_start.get(), b.nsys());
   else if (mode == TAB_COMBINE)
-    kb_pair<TAB_COMBINE, ISO><<<b.blocks(), 64, 0, s>>>(b.d_args.get(), b.d_start.get(), b.nsys());
+    kb_pair<TAB_COMBINE, ISO><<<b.blocks(), 64, b.lds, s>>>(b.d_args.get(), b.d_start.get(), b.nsys());
   else
-    kb_pair<TAB_GLOBAL, ISO><<<b.blocks(), 64, 0, s>>>(b.d_args.get(), b.d_start.get(), b.nsys());
+    kb_pair<TAB_GLOBAL, ISO><<<b.blocks(), 64, b.lds, s>>>(b.d_args.get(), b.d_start.get(), b.nsys());
 }
 // mode: the table layout every system of the batch allows (pair_tab_mode);
 // iso: every system's box is cubic

@@ -10,62 +10,58 @@
 namespace apo {
 
 // ---------------------------------------------------------------------------
-// erfc approximation for the FP32 pair kernel.
-// erfc(x) = exp(-x^2) erfcx(x); erfcx is interpolated at Chebyshev nodes in
-// t = 1/(1 + p x) on [0, xfit] (xfit >= kappa*r_off), then expanded to a
-// monomial series in t evaluated by Horner in the kernel.  Project-fitted at
-// set-up for the system's own interval (no third-party constants).
+// Coulomb table of the pair kernel: f(r) = erfc(k r) + 2 k r / sqrt(pi)
+// exp(-k^2 r^2) as one polynomial per interval, interpolated at Chebyshev
+// nodes in double at set-up for the system's own k and r_off.
 // ---------------------------------------------------------------------------
-static double erfcx_host(double x) { return std::erfc(x) * std::exp(x * x); }
+static double coulomb_f(double x) {  // x = k r
+  return std::erfc(x) + 2.0 / std::sqrt(kPi) * x * std::exp(-x * x);
+}
 
-static void fit_erfc(double xfit, double p, double *coef /*9*/) {
-  const int deg = 8, nn = deg + 1;
-  double tmin = 1.0 / (1.0 + p * xfit);
-  // Chebyshev coefficients of f(u), u in [-1,1] <-> t = tmin + (u+1)(1-tmin)/2
-  double c[nn];
-  for (int k = 0; k < nn; k++) {
-    double s = 0;
-    for (int j = 0; j < nn; j++) {
-      double u = std::cos(kPi * (j + 0.5) / nn);
-      double t = tmin + (u + 1.0) * (1.0 - tmin) * 0.5;
-      double x = (1.0 / t - 1.0) / p;
-      s += erfcx_host(x) * std::cos(kPi * k * (j + 0.5) / nn);
-    }
-    c[k] = (k == 0 ? 1.0 : 2.0) * s / nn;
+// Coefficients c[0..deg] in u on [0, 1] of the polynomial through fn at the
+// deg + 1 Chebyshev nodes (Newton's divided differences, then expanded).
+template <typename F> static void fit_interval(F &&fn, int deg, double *c) {
+  double u[8], d[8];
+  for (int k = 0; k <= deg; k++) {
+    u[k] = 0.5 - 0.5 * std::cos(kPi * (k + 0.5) / (deg + 1));
+    d[k] = fn(u[k]);
   }
-  // Chebyshev -> monomial in u (T_{k+1} = 2u T_k - T_{k-1})
-  double Tprev[nn] = {0}, Tcur[nn] = {0}, pu[nn] = {0};
-  Tprev[0] = 1.0;            // T0
-  Tcur[1] = 1.0;             // T1
-  pu[0] += c[0];
-  for (int i = 0; i < nn; i++) pu[i] += c[1] * Tcur[i];
-  for (int k = 2; k < nn; k++) {
-    double Tn[nn] = {0};
-    for (int i = 0; i < nn; i++) {
-      if (i > 0) Tn[i] += 2.0 * Tcur[i - 1];
-      Tn[i] -= Tprev[i];
-    }
-    for (int i = 0; i < nn; i++) {
-      pu[i] += c[k] * Tn[i];
-      Tprev[i] = Tcur[i];
-      Tcur[i] = Tn[i];
-    }
+  for (int j = 1; j <= deg; j++)
+    for (int k = deg; k >= j; k--) d[k] = (d[k] - d[k - 1]) / (u[k] - u[k - j]);
+  for (int k = 0; k <= deg; k++) c[k] = 0.0;
+  for (int k = deg; k >= 0; k--) {  // c <- c (u - u_k) + d_k
+    for (int i = deg; i > 0; i--) c[i] = c[i - 1] - u[k] * c[i];
+    c[0] = d[k] - u[k] * c[0];
   }
-  // compose with u = a t + b
-  double a = 2.0 / (1.0 - tmin), b = -2.0 * tmin / (1.0 - tmin) - 1.0;
-  double pt[nn] = {0};
-  double powab[nn] = {0};  // (a t + b)^k coefficients
-  powab[0] = 1.0;
-  for (int k = 0; k < nn; k++) {
-    for (int i = 0; i < nn; i++) pt[i] += pu[k] * powab[i];
-    double nxt[nn] = {0};
-    for (int i = 0; i < nn; i++) {
-      nxt[i] += b * powab[i];
-      if (i + 1 < nn) nxt[i + 1] += a * powab[i];
-    }
-    std::memcpy(powab, nxt, sizeof(nxt));
+}
+
+// Interval edge: the largest power of two with k h <= 1/20 (1/8 A, 96
+// intervals at k = 0.34, r_off = 12), where the cubic's interpolation error,
+// (k h)^4 f^(4) / 3072 < 1e-8 of f(0), is well below FP32 rounding and degree 5
+// reaches 1e-12 in FP64.  At least 1/64 A (r^-12 of a pair in units of h stays
+// in FP32 range), 64 to 512 intervals (1 to 8 KB of LDS in FP32).  A power of
+// two changes no mantissa against A, so neither the unit factor's rounding nor
+// the reciprocal square root's error at the distances that dominate the force
+// moves (with h = r_off / 128 the direct forces' error was 8 % larger).
+void NbSystem::make_pair_tables() {
+  int e = (int)std::min(20.0, std::max(-6.0, std::floor(std::log2(1.0 / (20.0 * kappa)))));
+  while (std::ldexp(1.0, e) * 64.0 > ctofnb) e--;
+  while (e < -6 || std::ldexp(1.0, e) * 512.0 < ctofnb) e++;
+  tab_h = std::ldexp(1.0, e);
+  tab_n = (int)std::ceil(ctofnb / tab_h);
+  const double xh = kappa * tab_h;
+  std::vector<float4> t(tab_n + 1);
+  std::vector<double2> td(3 * (size_t)(tab_n + 1));
+  for (int k = 0; k <= tab_n; k++) {
+    auto fn = [&](double u) { return coulomb_f(xh * (k + u)); };
+    double c[6];
+    fit_interval(fn, 3, c);
+    t[k] = make_float4((float)c[0], (float)c[1], (float)c[2], (float)c[3]);
+    fit_interval(fn, 5, c);
+    for (int i = 0; i < 3; i++) td[3 * (size_t)k + i] = make_double2(c[2 * i], c[2 * i + 1]);
   }
-  for (int i = 0; i < nn; i++) coef[i] = pt[i];
+  ewtab.upload(t, 0);
+  ewtab_d.upload(td, 0);
 }
 
 void NbSystem::make_pair_consts() {
@@ -84,20 +80,10 @@ void NbSystem::make_pair_consts() {
     dv6 = -1.0 / roff6;
     dv12 = -1.0 / (roff6 * roff6);
   }
-  double s32 = 4294967296.0;
-  double ep = 0.47, coef[9];
-  fit_erfc(std::max(kappa * roff * 1.01, 4.0), ep, coef);
+  const double s32 = 4294967296.0;
   auto fill = [&](auto &pc) {
-    using T = std::remove_reference_t<decltype(pc.sx)>;
-    pc.sx = (T)(box[0] / s32);
-    pc.sy = (T)(box[1] / s32);
-    pc.sz = (T)(box[2] / s32);
-    const double u = box[0] / s32;
-    pc.s2 = (T)(u * u);
-    pc.roff2u = (T)(roff * roff / (u * u));
-    pc.roff2 = (T)(roff * roff);
+    using T = std::remove_reference_t<decltype(pc.ron2)>;
     pc.ron2 = (T)(ron * ron);
-    pc.rlist2 = (T)(cutnb * cutnb);
     pc.k6 = (T)k6;
     pc.k12 = (T)k12;
     pc.dv6 = (T)dv6;
@@ -106,13 +92,34 @@ void NbSystem::make_pair_consts() {
     pc.roffinv6 = (T)(1.0 / roff6);
     pc.kappa = (T)kappa;
     pc.kappa2 = (T)(kappa * kappa);
-    pc.k2log2e = (T)(kappa * kappa * 1.4426950408889634);
     pc.two_kappa_sqrtpi = (T)(2.0 * kappa / std::sqrt(kPi));
-    pc.erfc_p = (T)(ep * kappa);
-    for (int i = 0; i < 9; i++) pc.erfc_c[i] = (T)coef[i];
   };
   fill(pc_f);
   fill(pc_d);
+  const double h = tab_h, h3 = h * h * h, h6 = h3 * h3;
+  auto units = [&](auto &pu) {
+    using T = std::remove_reference_t<decltype(pu.ron2)>;
+    pu.sx = (T)(box[0] / s32 / h);
+    pu.sy = (T)(box[1] / s32 / h);
+    pu.sz = (T)(box[2] / s32 / h);
+    const double u = box[0] / s32;  // A
+    pu.s2 = (T)(u / h * u / h);
+    pu.roff2 = (T)(roff * roff / (h * h));
+    pu.roff2u = (T)(roff * roff / (u * u));
+    pu.flush = (T)(1.0 / h);
+    pu.flush_u = (T)(u / h / h);
+    pu.ron2 = (T)(ron * ron / (h * h));
+    pu.k6 = (T)k6;
+    pu.k12 = (T)k12;
+    pu.dv6 = (T)(dv6 * h6);
+    pu.dv12 = (T)(dv12 * h6 * h6);
+    pu.roffinv3 = (T)(h3 / roff3);
+    pu.roffinv6 = (T)(h6 / roff6);
+    pu.kappa = (T)(kappa * h);
+    pu.ntab = tab_n;
+  };
+  units(pu_f);
+  units(pu_d);
 }
 
 // ---------------------------------------------------------------------------
@@ -293,12 +300,16 @@ NbSystem *create_system(const apo_nb_params &p, const apo_nb_topology &t) {
     std::vector<float2> tab(npair), tab14(npair);
     std::vector<double2> tabd(npair), tab14d(npair);
     const float *t14 = t.vdwtab14 ? t.vdwtab14 : t.vdwtab;
+    S->make_pair_tables();
+    S->make_pair_consts();
+    const double hi3 = 1.0 / (S->tab_h * S->tab_h * S->tab_h), hi6 = hi3 * hi3;
     for (int k = 0; k < npair; k++) {
       // stored as (6 c6, 12 c12) like setup_vdwparam
-      // (src/CudaPMEDirectForce.cu:534-540)
-      tab[k] = make_float2(6.0f * t.vdwtab[2 * k], 12.0f * t.vdwtab[2 * k + 1]);
+      // (src/CudaPMEDirectForce.cu:534-540); the pair kernel's in units of tab_h
+      tabd[k] = make_double2(6.0 * (double)t.vdwtab[2 * k] * hi6,
+                             12.0 * (double)t.vdwtab[2 * k + 1] * hi6 * hi6);
+      tab[k] = make_float2((float)tabd[k].x, (float)tabd[k].y);
       tab14[k] = make_float2(6.0f * t14[2 * k], 12.0f * t14[2 * k + 1]);
-      tabd[k] = make_double2(6.0 * (double)t.vdwtab[2 * k], 12.0 * (double)t.vdwtab[2 * k + 1]);
       tab14d[k] = make_double2(6.0 * (double)t14[2 * k], 12.0 * (double)t14[2 * k + 1]);
     }
     if (t.ntypes <= 32) {
@@ -344,7 +355,7 @@ NbSystem *create_system(const apo_nb_params &p, const apo_nb_topology &t) {
         }
       S->lj_combine = ok;
       std::vector<float2> lt(nt);
-      for (int a = 0; a < nt; a++) lt[a] = make_float2((float)se[a], (float)rh[a]);
+      for (int a = 0; a < nt; a++) lt[a] = make_float2((float)se[a], (float)(rh[a] / S->tab_h));
       S->ljtype.upload(lt, 0);
     }
     S->vdwtab.upload(tab, 0);
@@ -415,13 +426,12 @@ NbSystem *create_system(const apo_nb_params &p, const apo_nb_topology &t) {
     S->dihe.upload(mkd(t.dihe, t.dihe_par, t.ndihe), 0);
     S->imdihe.upload(mkd(t.imdihe, t.imdihe_par, t.nimdihe), 0);
 
-    S->make_pair_consts();
     if (t.ntypes <= kMaxTypesPqa) {
       // (P, Q, A12) of the inner and outer switch regions per type pair,
       // formed in FP64 from the (6 c6, 12 c12) table
       const int nt = t.ntypes;
-      const double r3 = 1.0 / (S->ctofnb * S->ctofnb * S->ctofnb), r6 = r3 * r3;
-      const double k6 = S->pc_d.k6, k12 = S->pc_d.k12;
+      const double r3 = S->pu_d.roffinv3, r6 = S->pu_d.roffinv6;
+      const double k6 = S->pu_d.k6, k12 = S->pu_d.k12;
       std::vector<float4> pqa(2 * (size_t)nt * nt);
       for (int a = 0; a < nt; a++)
         for (int b = 0; b < nt; b++) {

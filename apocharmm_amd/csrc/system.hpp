@@ -36,8 +36,16 @@ struct NbSystem {
   // ---- topology ------------------------------------------------------------
   int ntypes = 0;
   DevBuf<int> vdwtype;
-  DevBuf<float2> vdwtab;      // (6*c6, 12*c12)
-  DevBuf<float2> vdwtab14;
+  // Coulomb part of the pair kernel: f(r) = erfc(k r) + 2 k r / sqrt(pi)
+  // exp(-k^2 r^2), so that r dU/dr = -qq f / r, as polynomials over tab_n
+  // equal intervals of edge tab_h (pair.hip); cubic in FP32, degree 5 in FP64
+  double tab_h = 0;
+  int tab_n = 0;
+  DevBuf<float4> ewtab;
+  DevBuf<double2> ewtab_d;  // 3 per entry
+  // vdW tables of the pair kernel, in units of tab_h (6*c6, 12*c12)
+  DevBuf<float2> vdwtab;
+  DevBuf<float2> vdwtab14;    // 1-4 pairs, in A
   DevBuf<double2> vdwtab_d;   // FP64 instantiation
   DevBuf<double2> vdwtab14_d;
   DevBuf<float2> vdwsq;       // square (ntypes x ntypes) copy for <= 32 types
@@ -171,8 +179,11 @@ struct NbSystem {
 
   PairConsts<float> pc_f;
   PairConsts<double> pc_d;
+  PairUnits<float> pu_f;
+  PairUnits<double> pu_d;
 
   void make_pair_consts();
+  void make_pair_tables();
   void setup_pme();
   void setup_columns();
 };
