@@ -63,7 +63,14 @@ __device__ __forceinline__ double coulomb_factor(const double2 *tab, double r) {
 }
 
 __device__ __forceinline__ float rsqrt_ct(float x) { return __builtin_amdgcn_rsqf(x); }
-__device__ __forceinline__ double rsqrt_ct(double x) { return 1.0 / sqrt(x); }
+// hardware estimate, then one third-order step: y (1 + e/2 + 3 e^2/8) with
+// e = 1 - x y^2 leaves 5 e^3/16, below FP64 rounding for any estimate good to
+// 2^-18
+__device__ __forceinline__ double rsqrt_ct(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = fma(-x * y, y, 1.0);
+  return fma(y * e, fma(0.375, e, 0.5), y);
+}
 
 template <typename CT> __device__ __forceinline__ CT charge_of(int bits);
 template <> __device__ __forceinline__ float charge_of<float>(int bits) { return __int_as_float(bits); }
@@ -119,13 +126,24 @@ template <typename T2> static int pair_tab_mode(int ntypes, bool combine) {
 template <typename CT> __host__ __device__ __forceinline__ int ew_lds_bytes(int ntab) {
   return (ntab + 1) * Vec2<CT>::kEw * (int)sizeof(typename Vec2<CT>::Ew);
 }
-template <typename T2> static size_t pair_tab_lds_bytes(int mode, int ntypes, int ntab) {
+// bytes of the vdW table in LDS, padded to 16
+template <typename T2> __host__ __device__ __forceinline__ int vdw_lds_bytes(int mode, int ntypes) {
+  const int b = mode == TAB_PQA      ? 2 * ntypes * ntypes * (int)sizeof(float4)
+                : mode == TAB_SQUARE ? ntypes * ntypes * (int)sizeof(T2)
+                : mode == TAB_TRI    ? ntypes * (ntypes + 1) / 2 * (int)sizeof(T2)
+                                     : 0;
+  return (b + 15) & ~15;
+}
+// energy calls add the erfc table and, with TAB_PQA, the vdW energies
+template <typename T2>
+static size_t pair_tab_lds_bytes(int mode, int ntypes, int ntab, bool energy = false) {
   using CT = std::conditional_t<sizeof(T2) == sizeof(float2), float, double>;
-  const size_t ew = ew_lds_bytes<CT>(ntab);
-  if (mode == TAB_PQA) return ew + 2 * (size_t)ntypes * ntypes * sizeof(float4);
-  return ew + (mode == TAB_SQUARE
-                   ? (size_t)ntypes * ntypes * sizeof(T2)
-                   : (mode == TAB_TRI ? (size_t)ntypes * (ntypes + 1) / 2 * sizeof(T2) : 0));
+  size_t b = (size_t)ew_lds_bytes<CT>(ntab) + vdw_lds_bytes<T2>(mode, ntypes);
+  if (energy) {
+    b += ew_lds_bytes<double>(ntab);
+    if (mode == TAB_PQA) b += 4 * (size_t)ntypes * ntypes * sizeof(double2);
+  }
+  return b;
 }
 
 // One wave64 = one work item: an i-group of kGroup consecutive sorted slots
@@ -161,6 +179,7 @@ __device__ __forceinline__ void pair_body(
     const float2 *__restrict__ ljtype, const float4 *__restrict__ vdwpqa, int ntypes,
     const PairUnits<CT> &P, CT qfac, unsigned long long *__restrict__ fsort, int ss,
     double *__restrict__ part, const PairUnits<double> &PE,
+    const double2 *__restrict__ erfctab, const double2 *__restrict__ vdwen,
     const double2 *__restrict__ vdwtab_e, uint32_t *__restrict__ ent_out,
     int4 *__restrict__ items_out, CT rp2t) {
   static_assert(!ISO || sizeof(CT) == sizeof(float), "fixed-point-unit distances are FP32 only");
@@ -174,6 +193,9 @@ __device__ __forceinline__ void pair_body(
   const int ew_bytes = ew_lds_bytes<CT>(P.ntab);
   T2 *sh_tab = reinterpret_cast<T2 *>(smem_pair + ew_bytes);
   float4 *sh_pqa = reinterpret_cast<float4 *>(smem_pair + ew_bytes);
+  double2 *sh_erfc =
+      reinterpret_cast<double2 *>(smem_pair + ew_bytes + vdw_lds_bytes<T2>(TAB, ntypes));
+  double2 *sh_en = sh_erfc + 3 * (P.ntab + 1);
   const int nt2 = ntypes * ntypes;
   const int lane = threadIdx.x;
   const int nitem = meta[3];
@@ -185,6 +207,11 @@ __device__ __forceinline__ void pair_body(
       for (int k = lane; k < nt2; k += 64) sh_tab[k] = vdwsq[k];
     } else if (TAB == TAB_TRI) {
       for (int k = lane; k < ntypes * (ntypes + 1) / 2; k += 64) sh_tab[k] = vdwtab[k];
+    }
+    if (CALC_E) {
+      for (int k = lane; k < 3 * (P.ntab + 1); k += 64) sh_erfc[k] = erfctab[k];
+      if (TAB == TAB_PQA)
+        for (int k = lane; k < 4 * nt2; k += 64) sh_en[k] = vdwen[k];
     }
     __syncthreads();
   }
@@ -259,6 +286,7 @@ __device__ __forceinline__ void pair_body(
       CT fjx = 0, fjy = 0, fjz = 0;
       // energies accumulate per pair in FP64 (large cancelling sums); the
       // virial per step in CT
+      const double qje = (double)charge_of<CT>(pj.w) * (kCcelec * PE.flush);
       double el = 0, ev = 0;
       CT v0 = 0, v1 = 0, v2 = 0, v3 = 0, v4 = 0, v5 = 0;
 #pragma unroll
@@ -327,25 +355,43 @@ __device__ __forceinline__ void pair_body(
             // energies of energy steps in FP64 from the same fixed-point
             // geometry: a pair energy is ~1e2 larger than the sums it
             // cancels into, and FP32 pair arithmetic (~2e-7 relative) would
-            // dominate the energy error
-            const double ex = (double)(int)(pix[k] - pj.x) * PE.sx;
-            const double ey = (double)(int)(piy[k] - pj.y) * PE.sy;
-            const double ez = (double)(int)(piz[k] - pj.z) * PE.sz;
-            const double er2 = ex * ex + ey * ey + ez * ez;
-            const double er = sqrt(er2), erinv = 1.0 / er;
-            el += (double)qi[k] * (double)charge_of<CT>(pj.w) * (kCcelec * PE.flush) *
-                  erfc(PE.kappa * er) * erinv;
-            const int ti = TAB == TAB_SQUARE ? rowi[k] / ntypes
-                                             : (TAB == TAB_PQA ? rowi[k] / (ntypes * 32) : rowi[k]);
-            const int aa = ti > tj ? ti : tj, bb = ti > tj ? tj : ti;
-            const double2 ce = vdwtab_e[aa * (aa + 1) / 2 + bb];
+            // dominate the energy error.  FP64 issue bounds this block:
+            // erfc(k r) from a degree-5 table (errors below 1e-12), the
+            // reciprocal root by one third-order step and, with TAB_PQA, one
+            // polynomial in r^-3 per region replace libm's erfc, a square root
+            // and a divide (kernel with energies and virial, alone: 616 -> 246
+            // us at 93,984 atoms, 191 -> 104 in DHFR, 42 -> 23 at 2,529; all
+            // FP64 154 -> 68 at 11,748)
+            double er2, erinv;
+            if constexpr (sizeof(CT) == sizeof(double)) {
+              er2 = r2;
+              erinv = rinv;
+            } else {
+              const double ex = (double)(int)(pix[k] - pj.x) * PE.sx;
+              const double ey = (double)(int)(piy[k] - pj.y) * PE.sy;
+              const double ez = (double)(int)(piz[k] - pj.z) * PE.sz;
+              er2 = fma(ez, ez, fma(ey, ey, ex * ex));
+              erinv = rsqrt_ct(er2);
+            }
+            el = fma((double)qi[k] * qje, coulomb_factor(sh_erfc, er2 * erinv) * erinv, el);
             const double er3 = erinv * erinv * erinv, er6 = er3 * er3;
             const bool eo = er2 > PE.ron2;
-            const double e6 = eo ? er3 - PE.roffinv3 : er3, e12 = eo ? er6 - PE.roffinv6 : er6;
-            const double A6 = eo ? PE.k6 : 1.0, A12 = eo ? PE.k12 : 1.0;
-            const double C6 = eo ? 0.0 : PE.dv6, C12 = eo ? 0.0 : PE.dv12;
-            ev += ce.y * (1.0 / 12.0) * (A12 * e12 * e12 + C12) -
-                  ce.x * (1.0 / 6.0) * (A6 * e6 * e6 + C6);
+            if constexpr (TAB == TAB_PQA) {
+              // U = E12 r^-12 - E6 r^-6 + E3 r^-3 + E0 with the region's values
+              const double2 *c = reinterpret_cast<const double2 *>(
+                  reinterpret_cast<const char *>(sh_en) + 2 * (rowi[k] + tjb) + (eo ? 32 : 0));
+              const double2 c0 = c[0], c1 = c[1];
+              ev += fma(fma(c0.x, er6, -c0.y), er6, fma(c1.x, er3, c1.y));
+            } else {
+              const int ti = TAB == TAB_SQUARE ? rowi[k] / ntypes : rowi[k];
+              const int aa = ti > tj ? ti : tj, bb = ti > tj ? tj : ti;
+              const double2 ce = vdwtab_e[aa * (aa + 1) / 2 + bb];
+              const double e6 = eo ? er3 - PE.roffinv3 : er3, e12 = eo ? er6 - PE.roffinv6 : er6;
+              const double A6 = eo ? PE.k6 : 1.0, A12 = eo ? PE.k12 : 1.0;
+              const double C6 = eo ? 0.0 : PE.dv6, C12 = eo ? 0.0 : PE.dv12;
+              ev += ce.y * (1.0 / 12.0) * (A12 * e12 * e12 + C12) -
+                    ce.x * (1.0 / 6.0) * (A6 * e6 * e6 + C6);
+            }
           }
           if (CALC_V) {
             const CT gx = fij * dx, gy = fij * dy, gz = fij * dz;
@@ -415,15 +461,18 @@ __device__ __forceinline__ void pair_body(
   }
 }
 
+// energy calls in mixed precision: three waves per SIMD (168 VGPRs; 179 without
+// the bound, which leaves two)
 template <typename CT, bool CALC_E, bool CALC_V, int TAB, bool ISO, bool PRUNE>
-__global__ __launch_bounds__(64) void k_pair(
+__global__ __launch_bounds__(64, CALC_E && sizeof(CT) == sizeof(float) ? 3 : 1) void k_pair(
     const int4 *__restrict__ posq, const int *__restrict__ types, const int4 *__restrict__ items,
     const int *__restrict__ iorder, const uint32_t *__restrict__ ent, const int *__restrict__ cand_j, const int *__restrict__ meta,
     const typename Vec2<CT>::Ew *__restrict__ ewtab,
     const typename Vec2<CT>::T *__restrict__ vdwtab, const typename Vec2<CT>::T *__restrict__ vdwsq,
     const float2 *__restrict__ ljtype, const float4 *__restrict__ vdwpqa, int ntypes,
     const PairUnits<CT> P, CT qfac, unsigned long long *__restrict__ fsort, int ss,
-    double *__restrict__ part, const PairUnits<double> PE, const double2 *__restrict__ vdwtab_e,
+    double *__restrict__ part, const PairUnits<double> PE, const double2 *__restrict__ erfctab,
+    const double2 *__restrict__ vdwen, const double2 *__restrict__ vdwtab_e,
     uint32_t *__restrict__ ent_out, int4 *__restrict__ items_out, CT rp2t) {
   // Register floor of 112 VGPRs (an empty asm statement that names v111): a
   // SIMD then holds at most four pair waves (448 of its 512 VGPRs) and keeps
@@ -434,7 +483,7 @@ __global__ __launch_bounds__(64) void k_pair(
   asm volatile("" ::: "v111");
   pair_body<CT, CALC_E, CALC_V, TAB, ISO, PRUNE>(blockIdx.x, gridDim.x, posq, types, items, iorder, ent,
                                                  cand_j, meta, ewtab, vdwtab, vdwsq, ljtype, vdwpqa,
-                                                 ntypes, P, qfac, fsort, ss, part, PE, vdwtab_e,
+                                                 ntypes, P, qfac, fsort, ss, part, PE, erfctab, vdwen, vdwtab_e,
                                                  ent_out, items_out, rp2t);
 }
 
@@ -449,7 +498,7 @@ __global__ __launch_bounds__(64) void kb_pair(const PairArgs *__restrict__ tab,
   pair_body<float, false, false, TAB, ISO, false>(
       blockIdx.x - bstart[s], bstart[s + 1] - bstart[s], a.posq, a.types, a.items, a.iorder, a.ent,
       a.cand_j, a.meta, a.ewtab, a.vdwtab, a.vdwsq, a.ljtype, a.vdwpqa, a.ntypes, a.P, a.qfac, a.fsort,
-      a.ss, nullptr, no_energy, nullptr, nullptr, nullptr, 0.0f);
+      a.ss, nullptr, no_energy, nullptr, nullptr, nullptr, nullptr, nullptr, 0.0f);
 }
 
 struct PairLaunch {
@@ -466,7 +515,7 @@ struct PairLaunch {
   unsigned long long *fsort;
   int ss;
   double *part;
-  const double2 *vdwtab_e;
+  const double2 *erfctab, *vdwen, *vdwtab_e;  // energy calls
   int blocks;
   size_t lds;
   hipStream_t s;
@@ -486,7 +535,7 @@ static void go_pair(const PairLaunch &L, const typename Vec2<CT>::T *tab,
     if (L.ent_out) {
       k_pair<CT, false, false, TAB, ISO, true><<<L.blocks, 64, L.lds, L.s>>>(
           L.posq, L.types, L.items, L.iorder, L.ent, L.cand_j, L.meta, ew, tab, sq, L.ljtype, L.vdwpqa,
-          L.ntypes, P, qfac, L.fsort, L.ss, L.part, PE, L.vdwtab_e, L.ent_out, L.items_out,
+          L.ntypes, P, qfac, L.fsort, L.ss, L.part, PE, L.erfctab, L.vdwen, L.vdwtab_e, L.ent_out, L.items_out,
           L.rp2t);
       return;
     }
@@ -494,7 +543,7 @@ static void go_pair(const PairLaunch &L, const typename Vec2<CT>::T *tab,
   k_pair<CT, E, V, TAB, ISO, false><<<L.blocks, 64, L.lds, L.s>>>(
       L.posq, L.types, L.items, L.iorder, L.ent, L.cand_j, L.meta, ew, tab, sq, L.ljtype, L.vdwpqa,
       L.ntypes, P,
-      qfac, L.fsort, L.ss, L.part, PE, L.vdwtab_e, nullptr, nullptr, (CT)0);
+      qfac, L.fsort, L.ss, L.part, PE, L.erfctab, L.vdwen, L.vdwtab_e, nullptr, nullptr, (CT)0);
 }
 template <typename CT, bool E, bool V, bool ISO>
 static void go_pair_tab(int mode, const PairLaunch &L, const typename Vec2<CT>::T *tab,
@@ -547,9 +596,11 @@ static void launch_pair_t(NbSystem &S, const typename Vec2<CT>::T *tab,
                reinterpret_cast<unsigned long long *>(S.fsort.get()),
                S.ssort,
                S.parts_ptr() + S.part.pair_off,
+               S.erfctab.get(),
+               S.vdwen.get(),
                S.vdwtab_d.get(),
                S.pair_blocks,
-               pair_tab_lds_bytes<typename Vec2<CT>::T>(mode, S.ntypes, S.tab_n),
+               pair_tab_lds_bytes<typename Vec2<CT>::T>(mode, S.ntypes, S.tab_n, E),
                s,
                prune_out ? S.ent_p.get() : nullptr,
                prune_out ? S.items_p.get() : nullptr,

@@ -51,7 +51,7 @@ void NbSystem::make_pair_tables() {
   tab_n = (int)std::ceil(ctofnb / tab_h);
   const double xh = kappa * tab_h;
   std::vector<float4> t(tab_n + 1);
-  std::vector<double2> td(3 * (size_t)(tab_n + 1));
+  std::vector<double2> td(3 * (size_t)(tab_n + 1)), te(td.size());
   for (int k = 0; k <= tab_n; k++) {
     auto fn = [&](double u) { return coulomb_f(xh * (k + u)); };
     double c[6];
@@ -59,9 +59,12 @@ void NbSystem::make_pair_tables() {
     t[k] = make_float4((float)c[0], (float)c[1], (float)c[2], (float)c[3]);
     fit_interval(fn, 5, c);
     for (int i = 0; i < 3; i++) td[3 * (size_t)k + i] = make_double2(c[2 * i], c[2 * i + 1]);
+    fit_interval([&](double u) { return std::erfc(xh * (k + u)); }, 5, c);
+    for (int i = 0; i < 3; i++) te[3 * (size_t)k + i] = make_double2(c[2 * i], c[2 * i + 1]);
   }
   ewtab.upload(t, 0);
   ewtab_d.upload(td, 0);
+  erfctab.upload(te, 0);
 }
 
 void NbSystem::make_pair_consts() {
@@ -443,6 +446,21 @@ NbSystem *create_system(const apo_nb_params &p, const apo_nb_topology &t) {
                                    (float)(k12 * c12), 0.f);
         }
       S->vdwpqa.upload(pqa, 0);
+      // energies of the same regions: c12 (r^-12 + dv12) - c6 (r^-6 + dv6)
+      // and k12 c12 (r^-6 - r_off^-6)^2 - k6 c6 (r^-3 - r_off^-3)^2, expanded
+      std::vector<double2> en(4 * (size_t)nt * nt);
+      for (int a = 0; a < nt; a++)
+        for (int b = 0; b < nt; b++) {
+          const int hi = a > b ? a : b, lo = a > b ? b : a;
+          const double c6 = tabd[hi * (hi + 1) / 2 + lo].x / 6.0;
+          const double c12 = tabd[hi * (hi + 1) / 2 + lo].y / 12.0;
+          const size_t k = 4 * ((size_t)a * nt + b);
+          en[k] = make_double2(c12, c6);
+          en[k + 1] = make_double2(0.0, c12 * S->pu_d.dv12 - c6 * S->pu_d.dv6);
+          en[k + 2] = make_double2(k12 * c12, k6 * c6 + 2.0 * k12 * c12 * r6);
+          en[k + 3] = make_double2(2.0 * k6 * c6 * r3, k12 * c12 * r6 * r6 - k6 * c6 * r3 * r3);
+        }
+      S->vdwen.upload(en, 0);
     }
     S->setup_columns();
     S->setup_pme();

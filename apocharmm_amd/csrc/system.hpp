@@ -43,6 +43,7 @@ struct NbSystem {
   int tab_n = 0;
   DevBuf<float4> ewtab;
   DevBuf<double2> ewtab_d;  // 3 per entry
+  DevBuf<double2> erfctab;  // erfc(k r) likewise, for the pair energies
   // vdW tables of the pair kernel, in units of tab_h (6*c6, 12*c12)
   DevBuf<float2> vdwtab;
   DevBuf<float2> vdwtab14;    // 1-4 pairs, in A
@@ -60,6 +61,9 @@ struct NbSystem {
   // with (P, Q, A12) = (6c6, 0, 12c12) inside r_on and (k6 6c6 + k12 12c12
   // r_off^-6, k6 6c6 r_off^-3, k12 12c12) beyond it; [ti][tj][inner | outer]
   DevBuf<float4> vdwpqa;
+  // ... and its energies U = E12 r^-12 - E6 r^-6 + E3 r^-3 + E0, in FP64:
+  // [ti][tj][inner | outer] (E12, E6), (E3, E0)
+  DevBuf<double2> vdwen;
   DevBuf<int> excl_ptr, excl_idx;
   int nin14 = 0, nex14 = 0;
   DevBuf<int2> in14, ex14;
