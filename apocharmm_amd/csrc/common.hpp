@@ -302,8 +302,10 @@ void pairs14_launch(NbSystem &sys, const float4 *d_xyzq, int64_t *d_force,
                     int stride, bool energy, bool virial, hipStream_t s);
 void bonded_launch(NbSystem &sys, const float4 *d_xyzq, int64_t *d_force,
                    int stride, bool energy, bool virial, hipStream_t s);
+// fold: the gather also adds the sorted pair gradient (direct_finalize), whose
+// kernel must precede this call on the same stream
 void recip_launch(NbSystem &sys, const float4 *d_xyzq, int64_t *d_force,
-                  int stride, bool energy, bool virial, hipStream_t s);
+                  int stride, bool energy, bool virial, hipStream_t s, bool fold = false);
 // Adds up the partials the terms of this call wrote (and the self energy).
 void reduce_energy_launch(NbSystem &sys, const float4 *d_xyzq, int term_mask, bool energy,
                           bool virial, double *d_energy, double *d_virial,

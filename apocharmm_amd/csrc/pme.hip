@@ -576,12 +576,16 @@ void k_spread_fftx(const int4 *__restrict__ posq,
 // Gather in cell order: 16 lanes per atom; the gradient goes straight into
 // the global-order output with int64 atomics (three per atom), so the gather
 // can run while the pair kernel and the bonded terms write the same atoms.
+// fsort (stride ss), when given, is the finished sorted pair gradient: the
+// atom's entry is added in the same atomics.
 template <typename CT>
 __device__ __forceinline__ void gather_body(int bid, const int4 *__restrict__ posq,
                                             const int *__restrict__ meta,
                                             const int *__restrict__ loc2glo, const GridGeom &g,
                                             double qunscale, const CT *__restrict__ phi,
-                                            unsigned long long *__restrict__ force, int stride) {
+                                            unsigned long long *__restrict__ force, int stride,
+                                            const unsigned long long *__restrict__ fsort = nullptr,
+                                            int ss = 0) {
   const int gt = bid * 256 + threadIdx.x;
   const int loc = gt >> 4, row = gt & 15;
   const bool valid = loc < meta[0] * kCell;
@@ -619,14 +623,22 @@ __device__ __forceinline__ void gather_body(int bid, const int4 *__restrict__ po
     f2 += __shfl_xor(f2, off);
     f3 += __shfl_xor(f3, off);
   }
-  if (valid && q != 0.0 && row == 0) {
+  if (valid && row == 0 && (q != 0.0 || fsort)) {
     const int gi = loc2glo[loc];
     if (gi >= 0) {
       const double qc = q * kCcelec;
       auto fx = [](double v) { return (unsigned long long)(long long)__builtin_rint(v); };
-      atomicAdd(&force[gi], fx(qc * g.inv0 * g.K0 * (double)f1 * kForceScale));
-      atomicAdd(&force[stride + gi], fx(qc * g.inv1 * g.K1 * (double)f2 * kForceScale));
-      atomicAdd(&force[2 * (size_t)stride + gi], fx(qc * g.inv2 * g.K2 * (double)f3 * kForceScale));
+      unsigned long long gx = fx(qc * g.inv0 * g.K0 * (double)f1 * kForceScale),
+                         gy = fx(qc * g.inv1 * g.K1 * (double)f2 * kForceScale),
+                         gz = fx(qc * g.inv2 * g.K2 * (double)f3 * kForceScale);
+      if (fsort) {
+        gx += fsort[loc];
+        gy += fsort[ss + loc];
+        gz += fsort[2 * (size_t)ss + loc];
+      }
+      atomicAdd(&force[gi], gx);
+      atomicAdd(&force[stride + gi], gy);
+      atomicAdd(&force[2 * (size_t)stride + gi], gz);
     }
   }
 }
@@ -636,9 +648,11 @@ __global__ __launch_bounds__(256) void k_gather_sorted(const int4 *__restrict__ 
                                                        const int *__restrict__ loc2glo, GridGeom g,
                                                        double qunscale, const CT *__restrict__ phi,
                                                        unsigned long long *__restrict__ force,
-                                                       int stride) {
+                                                       int stride,
+                                                       const unsigned long long *__restrict__ fsort,
+                                                       int ss) {
   if constexpr (PRIO) pme_wave_priority();
-  gather_body<CT>(blockIdx.x, posq, meta, loc2glo, g, qunscale, phi, force, stride);
+  gather_body<CT>(blockIdx.x, posq, meta, loc2glo, g, qunscale, phi, force, stride, fsort, ss);
 }
 
 
@@ -944,7 +958,7 @@ template <typename CT, bool PRIO, bool BIG>
 static void recip_t(NbSystem &S, const float4 *x, int64_t *force, int stride, bool EV,
                     typename Cx<CT>::T *cgrid, CT *phi, const typename Cx<CT>::T *twx,
                     const typename Cx<CT>::T *twy, const typename Cx<CT>::T *twz, const CT *pre,
-                    hipStream_t s) {
+                    hipStream_t s, bool fold) {
   (void)x;
   const PmeShapes<CT> P = pme_shapes<CT>(S);
   const int K1 = S.K[1], K2 = S.K[2], H = S.K[0] / 2 + 1;
@@ -978,13 +992,14 @@ static void recip_t(NbSystem &S, const float4 *x, int64_t *force, int stride, bo
   S.tic(3, s, t0);
   k_gather_sorted<CT, PRIO><<<(S.ssort * 16 + 255) / 256, 256, 0, s>>>(
       S.posq.get(), S.meta.get(), S.loc2glo.get(), P.g, qunscale, phi,
-      reinterpret_cast<unsigned long long *>(force), stride);
+      reinterpret_cast<unsigned long long *>(force), stride,
+      fold ? reinterpret_cast<const unsigned long long *>(S.fsort.get()) : nullptr, S.ssort);
   APO_LAUNCH_CHECK();
   S.toc(3, s, t0);
 }
 
 void recip_launch(NbSystem &S, const float4 *x, int64_t *force, int stride, bool E, bool V,
-                  hipStream_t s) {
+                  hipStream_t s, bool fold) {
   // the issue priority is a template parameter: as a kernel argument, every
   // wave waited for its load before issuing the kernel's own first loads
   auto run = [&](auto prio, auto big) {
@@ -992,10 +1007,10 @@ void recip_launch(NbSystem &S, const float4 *x, int64_t *force, int stride, bool
     if (S.precision == 1)
       recip_t<double, P, B>(S, x, force, stride, E || V, S.cgrid_d.get(), S.phi_d.get(),
                             S.fx.tw64.get(), S.fy.tw64.get(), S.fz.tw64.get(), S.prefac_d.get(),
-                            s);
+                            s, fold);
     else
       recip_t<float, P, B>(S, x, force, stride, E || V, S.cgrid.get(), S.phi.get(),
-                           S.fx.tw.get(), S.fy.tw.get(), S.fz.tw.get(), S.prefac.get(), s);
+                           S.fx.tw.get(), S.fy.tw.get(), S.fz.tw.get(), S.prefac.get(), s, fold);
   };
   const bool big = plan_big(S.fx) || plan_big(S.fy) || plan_big(S.fz);
   if (S.pme_prio) {

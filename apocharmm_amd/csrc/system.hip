@@ -525,6 +525,26 @@ void set_box(NbSystem &S, const double *b) {
   S.generation++;
 }
 
+// Whether an eager call (not being captured) runs its branches on the caller's
+// stream one after the other instead of forking PME and the bonded terms onto
+// side streams.  The four event records and waits of the fork cost the host
+// about 50 us; the overlap they buy is the shorter of the pair kernel and the
+// PME chain, which passes that near 25,000 atoms (forces; one stream / fork:
+// 83 / 127 us at 5,553 atoms, 133 / 132 at 21,525, 165 / 156 at 37,086, 307 /
+// 273 at 93,984) and near 40,000 with energies or the virial (145 / 185, 216 /
+// 225, 269 / 270, 459 / 426).  A captured call forks at every size: a graph
+// replays the events at no host cost.
+static bool one_stream(const NbSystem &S, hipStream_t s, bool ev) {
+  if (S.single_stream) return true;
+  if (S.natom >= (ev ? 40000 : 25000)) return false;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &cap) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return cap == hipStreamCaptureStatusNone;
+}
+
 void calc_force(NbSystem &S, const float *xyzq, int flags, int64_t *force, int stride,
                 double *energy, double *virial, hipStream_t s) {
   if (!xyzq || !force) throw InvalidArgument("xyzq and force must be device pointers");
@@ -549,7 +569,7 @@ void calc_force(NbSystem &S, const float *xyzq, int flags, int64_t *force, int s
   // `force`:  bonded + 1-4 (side[1], int64 atomics into force) | pair kernel
   // (caller's stream, atomics into the sorted buffer) | PME spread, FFT,
   // gather (side[0], atomics into force).
-  const bool fork = !S.single_stream;
+  const bool fork = !one_stream(S, s, E || V);
   hipStream_t sb = fork ? S.side[1] : s, sp = fork ? S.side[0] : s;
   bool rebuilt = false;
   if (dir || rec) {
@@ -587,9 +607,13 @@ void calc_force(NbSystem &S, const float *xyzq, int flags, int64_t *force, int s
     direct_launch(S, E, V, s, pruned, fused);
     S.toc(0, s, t0);
   };
-  if (dir && S.pair_first) pair_branch();
+  // on one stream the pair kernel runs first, and the gather, which then
+  // comes after every pair force, also folds the sorted gradient into `force`
+  const bool fold = !fork && dir && rec && !(flags & kCalcNoFinalize);
+  const bool pair_first = S.pair_first || fold;
+  if (dir && pair_first) pair_branch();
   if (rec) {
-    recip_launch(S, x4, force, stride, E, V, sp);
+    recip_launch(S, x4, force, stride, E, V, sp, fold);
     if (fork) APO_HIP(hipEventRecord(S.ev_pme, sp));
   }
   // bonded after PME (measured: launched first, its blocks delay the sort
@@ -601,10 +625,10 @@ void calc_force(NbSystem &S, const float *xyzq, int flags, int64_t *force, int s
     S.toc(6, sb, t1);
     if (fork) APO_HIP(hipEventRecord(S.ev_bond, sb));
   }
-  if (dir && !S.pair_first) pair_branch();
+  if (dir && !pair_first) pair_branch();
   if (fork && rec) APO_HIP(hipStreamWaitEvent(s, S.ev_pme, 0));
   if (fork && bnd) APO_HIP(hipStreamWaitEvent(s, S.ev_bond, 0));
-  if ((dir || rec) && !(flags & kCalcNoFinalize)) {
+  if ((dir || rec) && !fold && !(flags & kCalcNoFinalize)) {
     S.tic(7, s, t0);
     direct_finalize(S, force, stride, s);
     S.toc(7, s, t0);
