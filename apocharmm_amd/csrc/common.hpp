@@ -294,14 +294,15 @@ constexpr int kCalcNoFinalize = 1 << 26;
 // pruned: the pair kernel reads the pruned list copy; prune_out: it reads the
 // build's list and writes the pruned copy for the next steps (fused pruning,
 // mixed-precision MD steps)
-void direct_launch(NbSystem &sys, bool energy, bool virial, hipStream_t s, bool pruned = false,
+// pairs14, bonded: those lists run in the same launch (force calls only)
+void direct_launch(NbSystem &sys, const float4 *d_xyzq, int64_t *d_force, int stride, bool energy,
+                   bool virial, bool pairs14, bool bonded, hipStream_t s, bool pruned = false,
                    bool prune_out = false);
 void direct_finalize(NbSystem &sys, int64_t *d_force, int stride,
                      hipStream_t s);
-void pairs14_launch(NbSystem &sys, const float4 *d_xyzq, int64_t *d_force,
-                    int stride, bool energy, bool virial, hipStream_t s);
-void bonded_launch(NbSystem &sys, const float4 *d_xyzq, int64_t *d_force,
-                   int stride, bool energy, bool virial, hipStream_t s);
+// 1-4 / exclusion pairs and bonded terms (each when asked for), one launch
+void bonded_launch(NbSystem &sys, const float4 *d_xyzq, int64_t *d_force, int stride, bool energy,
+                   bool virial, bool pairs14, bool bonded, hipStream_t s);
 // fold: the gather also adds the sorted pair gradient (direct_finalize), whose
 // kernel must precede this call on the same stream
 void recip_launch(NbSystem &sys, const float4 *d_xyzq, int64_t *d_force,

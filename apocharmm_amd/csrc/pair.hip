@@ -18,6 +18,7 @@
 #include <cmath>
 #include <type_traits>
 
+#include "bonded_terms.hpp"
 #include "system.hpp"
 
 namespace apo {
@@ -473,7 +474,8 @@ __global__ __launch_bounds__(64, CALC_E && sizeof(CT) == sizeof(float) ? 3 : 1) 
     const PairUnits<CT> P, CT qfac, unsigned long long *__restrict__ fsort, int ss,
     double *__restrict__ part, const PairUnits<double> PE, const double2 *__restrict__ erfctab,
     const double2 *__restrict__ vdwen, const double2 *__restrict__ vdwtab_e,
-    uint32_t *__restrict__ ent_out, int4 *__restrict__ items_out, CT rp2t) {
+    uint32_t *__restrict__ ent_out, int4 *__restrict__ items_out, CT rp2t, int nblocks,
+    Bonded14<CT> B) {
   // Register floor of 112 VGPRs (an empty asm statement that names v111): a
   // SIMD then holds at most four pair waves (448 of its 512 VGPRs) and keeps
   // room for one wave of the PME passes (44-54 VGPRs), which otherwise waited
@@ -481,7 +483,14 @@ __global__ __launch_bounds__(64, CALC_E && sizeof(CT) == sizeof(float) ? 3 : 1) 
   // convolution 102 -> 86 us inside the step, step 705 -> 714 ns/day).  The
   // kernel's own allocation is 92-107 VGPRs, so no spill follows.
   asm volatile("" ::: "v111");
-  pair_body<CT, CALC_E, CALC_V, TAB, ISO, PRUNE>(blockIdx.x, gridDim.x, posq, types, items, iorder, ent,
+  if constexpr (!CALC_E && !CALC_V) {
+    if ((int)blockIdx.x >= nblocks) {
+      bonded14_body<CT, false, false, 64>(blockIdx.x - nblocks, B, nullptr, PairConsts<double>{},
+                                          nullptr, nullptr);
+      return;
+    }
+  }
+  pair_body<CT, CALC_E, CALC_V, TAB, ISO, PRUNE>(blockIdx.x, nblocks, posq, types, items, iorder, ent,
                                                  cand_j, meta, ewtab, vdwtab, vdwsq, ljtype, vdwpqa,
                                                  ntypes, P, qfac, fsort, ss, part, PE, erfctab, vdwen, vdwtab_e,
                                                  ent_out, items_out, rp2t);
@@ -524,6 +533,16 @@ struct PairLaunch {
   uint32_t *ent_out;
   int4 *items_out;
   float rp2t;
+  const NbSystem *S;
+  const struct PairBonded *bnd;  // or null
+};
+
+// bonded terms to run in the same launch (force calls)
+struct PairBonded {
+  const float4 *x;
+  int64_t *force;
+  int stride;
+  bool pairs14, bonded;
 };
 
 template <typename CT, bool E, bool V, int TAB, bool ISO>
@@ -531,19 +550,24 @@ static void go_pair(const PairLaunch &L, const typename Vec2<CT>::T *tab,
                     const typename Vec2<CT>::T *sq, const PairUnits<CT> &P, CT qfac,
                     const PairUnits<double> &PE) {
   const auto *ew = static_cast<const typename Vec2<CT>::Ew *>(L.ewtab);
+  Bonded14<CT> B{};
+  if (!E && !V && L.bnd)
+    B = bonded14_args<CT>(*L.S, L.bnd->x, L.bnd->force, L.bnd->stride, L.bnd->pairs14,
+                          L.bnd->bonded, 64);
+  const int grid = L.blocks + B.n14 + B.nb;
   if constexpr (sizeof(CT) == sizeof(float) && !E && !V) {
     if (L.ent_out) {
-      k_pair<CT, false, false, TAB, ISO, true><<<L.blocks, 64, L.lds, L.s>>>(
+      k_pair<CT, false, false, TAB, ISO, true><<<grid, 64, L.lds, L.s>>>(
           L.posq, L.types, L.items, L.iorder, L.ent, L.cand_j, L.meta, ew, tab, sq, L.ljtype, L.vdwpqa,
           L.ntypes, P, qfac, L.fsort, L.ss, L.part, PE, L.erfctab, L.vdwen, L.vdwtab_e, L.ent_out, L.items_out,
-          L.rp2t);
+          L.rp2t, L.blocks, B);
       return;
     }
   }
-  k_pair<CT, E, V, TAB, ISO, false><<<L.blocks, 64, L.lds, L.s>>>(
+  k_pair<CT, E, V, TAB, ISO, false><<<grid, 64, L.lds, L.s>>>(
       L.posq, L.types, L.items, L.iorder, L.ent, L.cand_j, L.meta, ew, tab, sq, L.ljtype, L.vdwpqa,
       L.ntypes, P,
-      qfac, L.fsort, L.ss, L.part, PE, L.erfctab, L.vdwen, L.vdwtab_e, nullptr, nullptr, (CT)0);
+      qfac, L.fsort, L.ss, L.part, PE, L.erfctab, L.vdwen, L.vdwtab_e, nullptr, nullptr, (CT)0, L.blocks, B);
 }
 template <typename CT, bool E, bool V, bool ISO>
 static void go_pair_tab(int mode, const PairLaunch &L, const typename Vec2<CT>::T *tab,
@@ -578,7 +602,7 @@ template <typename CT>
 static void launch_pair_t(NbSystem &S, const typename Vec2<CT>::T *tab,
                           const typename Vec2<CT>::T *sq, const void *ewtab,
                           const PairUnits<CT> &P, CT qfac, bool E, bool V, hipStream_t s,
-                          bool pruned, bool prune_out) {
+                          bool pruned, bool prune_out, const PairBonded *bnd) {
   const int mode = pair_tab_mode<typename Vec2<CT>::T>(S.ntypes, S.lj_combine);
   pruned = pruned && !prune_out;
   const bool iso = pair_iso(S);
@@ -606,7 +630,9 @@ static void launch_pair_t(NbSystem &S, const typename Vec2<CT>::T *tab,
                prune_out ? S.items_p.get() : nullptr,
                (float)(iso ? (double)S.prune_r2 / ((S.box[0] / 4294967296.0) *
                                                    (S.box[0] / 4294967296.0))
-                           : (double)S.prune_r2 / (S.tab_h * S.tab_h))};
+                           : (double)S.prune_r2 / (S.tab_h * S.tab_h)),
+               &S,
+               bnd};
   if (E && V)
     go_pair_iso<CT, true, true>(iso, mode, L, tab, sq, P, qfac, S.pu_d);
   else if (E)
@@ -618,15 +644,17 @@ static void launch_pair_t(NbSystem &S, const typename Vec2<CT>::T *tab,
   APO_LAUNCH_CHECK();
 }
 
-void direct_launch(NbSystem &S, bool E, bool V, hipStream_t s, bool pruned, bool prune_out) {
+void direct_launch(NbSystem &S, const float4 *x, int64_t *force, int stride, bool E, bool V,
+                   bool pairs14, bool bonded, hipStream_t s, bool pruned, bool prune_out) {
+  const PairBonded bnd{x, force, stride, pairs14, bonded};
   if (prune_out && (S.precision != 0 || E || V))
     throw InvalidArgument("fused list pruning runs in mixed-precision MD steps only");
   if (S.precision == 1)
     launch_pair_t<double>(S, S.vdwtab_d.get(), S.vdwsq_d.get(), S.ewtab_d.get(), S.pu_d,
-                          kCcelec / S.tab_h, E, V, s, pruned, false);
+                          kCcelec / S.tab_h, E, V, s, pruned, false, &bnd);
   else
     launch_pair_t<float>(S, S.vdwtab.get(), S.vdwsq.get(), S.ewtab.get(), S.pu_f,
-                         (float)(kCcelec / S.tab_h), E, V, s, pruned, prune_out);
+                         (float)(kCcelec / S.tab_h), E, V, s, pruned, prune_out, &bnd);
 }
 
 // Sorted -> global order (addSortedForce, src/CudaPMEDirectForce.cu:1375-1386).

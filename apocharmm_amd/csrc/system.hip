@@ -290,7 +290,7 @@ NbSystem *create_system(const apo_nb_params &p, const apo_nb_topology &t) {
     APO_HIP(hipGetDeviceProperties(&prop, S->device));
     S->ncu = prop.multiProcessorCount > 0 ? prop.multiProcessorCount : 256;
     for (hipStream_t &st : S->side) APO_HIP(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
-    for (hipEvent_t *e : {&S->ev_fork, &S->ev_sorted, &S->ev_pme, &S->ev_bond})
+    for (hipEvent_t *e : {&S->ev_sorted, &S->ev_side, &S->ev_bond})
       APO_HIP(hipEventCreateWithFlags(e, hipEventDisableTiming));
 
     const int n = t.natom;
@@ -525,24 +525,42 @@ void set_box(NbSystem &S, const double *b) {
   S.generation++;
 }
 
-// Whether an eager call (not being captured) runs its branches on the caller's
-// stream one after the other instead of forking PME and the bonded terms onto
-// side streams.  The four event records and waits of the fork cost the host
-// about 50 us; the overlap they buy is the shorter of the pair kernel and the
-// PME chain, which passes that near 25,000 atoms (forces; one stream / fork:
-// 83 / 127 us at 5,553 atoms, 133 / 132 at 21,525, 165 / 156 at 37,086, 307 /
-// 273 at 93,984) and near 40,000 with energies or the virial (145 / 185, 216 /
-// 225, 269 / 270, 459 / 426).  A captured call forks at every size: a graph
-// replays the events at no host cost.
-static bool one_stream(const NbSystem &S, hipStream_t s, bool ev) {
-  if (S.single_stream) return true;
-  if (S.natom >= (ev ? 40000 : 25000)) return false;
+// How a call runs its three branches: the pair kernel, the PME chain and the
+// bonded and 1-4 terms.
+//  * one_stream: one after the other on the caller's stream (small eager calls);
+//  * otherwise the PME chain stays on the caller's stream, behind the sort, so
+//    that the spread's blocks are resident before the pair kernel on the side
+//    stream takes the wave slots (the other way round the spread starved:
+//    force call 277 -> 253 us at 93,984 atoms);
+//  * merge: the bonded terms' blocks run in the pair kernel's launch;
+//  * bonded2: they have a side stream of their own (captured calls, where the
+//    events cost the host nothing).
+// Each event record or wait costs the host about 6 us, and what a fork buys is
+// the shorter of the pair kernel and the PME chain: eager calls fork, with one
+// side stream, from kForkAtoms up (one stream / fork: 127 / 131 us at 21,525
+// atoms, 146 / 148 at 28,731, 159 / 152 at 37,086, 181 / 165 at 45,852; with the
+// virial 176 / 188 at 26,988) and with energies, whose pair kernel is longer,
+// from kForkAtomsE (211 / 217, 243 / 233, 265 / 245, 287 / 279 at those sizes).  Merging saves a launch and fills the
+// drain of the pair items, but its latency-bound waves take pair-wave slots: in
+// captured steps it pays up to kMergeAtoms (apart / merged, 40 MD steps: 3,369 /
+// 3,186 us at 3,708 atoms, 3,324 / 3,243 at 8,061, 3,583 / 3,630 at 11,748),
+// on one stream at every size (130 -> 128 us at 23,558).
+constexpr int kForkAtoms = 33000, kForkAtomsE = 25000, kMergeAtoms = 10000;
+struct BranchPlan {
+  bool fork, merge, bonded2;
+};
+static BranchPlan plan_branches(const NbSystem &S, hipStream_t s, bool dir, bool rec, bool bnd,
+                                bool E, bool V) {
+  BranchPlan p{false, false, false};
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(s, &cap) != hipSuccess) {
-    (void)hipGetLastError();
-    return false;
-  }
-  return cap == hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &cap) != hipSuccess) (void)hipGetLastError();
+  const bool captured = cap != hipStreamCaptureStatusNone;
+  p.fork = dir && rec && !S.single_stream &&
+           (captured || S.natom >= (E ? kForkAtomsE : kForkAtoms));
+  // kernel timers on: a launch of their own, so that slot 6 times them
+  p.merge = bnd && dir && !E && !V && !S.prof_on && (!p.fork || S.natom < kMergeAtoms);
+  p.bonded2 = p.fork && captured && bnd && !p.merge;
+  return p;
 }
 
 void calc_force(NbSystem &S, const float *xyzq, int flags, int64_t *force, int stride,
@@ -565,12 +583,15 @@ void calc_force(NbSystem &S, const float *xyzq, int flags, int64_t *force, int s
   const bool acc = flags & APO_ACCUMULATE;
   if (!(dir || rec) && !acc) launch_fill_i64(force, 3 * (size_t)stride, s);
   const bool bnd = terms & (APO_TERM_PAIRS14 | APO_TERM_BONDED);
-  // Three branches that meet before the sorted pair gradient is folded into
-  // `force`:  bonded + 1-4 (side[1], int64 atomics into force) | pair kernel
-  // (caller's stream, atomics into the sorted buffer) | PME spread, FFT,
-  // gather (side[0], atomics into force).
-  const bool fork = !one_stream(S, s, E || V);
-  hipStream_t sb = fork ? S.side[1] : s, sp = fork ? S.side[0] : s;
+  const BranchPlan plan = plan_branches(S, s, dir, rec, bnd, E, V);
+  // The branches meet before the sorted pair gradient is folded into `force`:
+  // the pair kernel adds into the sorted buffer, the others into force, all in
+  // int64, so their order changes no bit.  pair_first (a launch setting of
+  // captured steps) swaps the streams: a graph keeps the first captured child
+  // of the sort on the caller's queue and dispatches it first.
+  const bool swap = plan.fork && S.pair_first;
+  hipStream_t side = plan.fork ? S.side[0] : s;  // the branch that forks
+  hipStream_t sp = swap ? side : s, sd = swap ? s : side;
   bool rebuilt = false;
   if (dir || rec) {
     // both the pair kernel and PME work on the cell-sorted coordinates
@@ -584,17 +605,17 @@ void calc_force(NbSystem &S, const float *xyzq, int flags, int64_t *force, int s
     nblist_sort_coords(S, x4, s, acc ? nullptr : force, acc ? 0 : 3 * (size_t)stride);
     S.toc(7, s, t0);
   }
-  // Both side branches fork right after the sort.  The capture order of the
-  // three branches is a launch setting (pair_first): a graph keeps the first
-  // captured child of the sort on the caller's queue and dispatches it first.
-  if (fork && rec) {
+  if (plan.fork) {
     APO_HIP(hipEventRecord(S.ev_sorted, s));
-    APO_HIP(hipStreamWaitEvent(sp, S.ev_sorted, 0));
+    APO_HIP(hipStreamWaitEvent(side, S.ev_sorted, 0));
+    if (plan.bonded2) APO_HIP(hipStreamWaitEvent(S.side[1], S.ev_sorted, 0));
   }
-  if (fork && bnd) {
-    APO_HIP(hipEventRecord(S.ev_fork, s));
-    APO_HIP(hipStreamWaitEvent(sb, S.ev_fork, 0));
-  }
+  auto bonded_branch = [&](hipStream_t st) {
+    S.tic(6, st, t1);
+    bonded_launch(S, x4, force, stride, E, V, terms & APO_TERM_PAIRS14, terms & APO_TERM_BONDED,
+                  st);
+    S.toc(6, st, t1);
+  };
   auto pair_branch = [&] {
     // a pruned list is refreshed after every build and when asked: by the
     // pair kernel itself in mixed-precision steps without energies (it tests
@@ -602,32 +623,38 @@ void calc_force(NbSystem &S, const float *xyzq, int flags, int64_t *force, int s
     const bool pruned = flags & kCalcUsePruned;
     const bool refresh = pruned && (rebuilt || (flags & kCalcPrune));
     const bool fused = refresh && S.precision == 0 && !E && !V;
-    if (refresh && !fused) nblist_prune(S, s);
-    S.tic(0, s, t0);
-    direct_launch(S, E, V, s, pruned, fused);
-    S.toc(0, s, t0);
+    if (refresh && !fused) nblist_prune(S, sd);
+    S.tic(0, sd, t0);
+    direct_launch(S, x4, force, stride, E, V, plan.merge && (terms & APO_TERM_PAIRS14),
+                  plan.merge && (terms & APO_TERM_BONDED), sd, pruned, fused);
+    S.toc(0, sd, t0);
   };
   // on one stream the pair kernel runs first, and the gather, which then
   // comes after every pair force, also folds the sorted gradient into `force`
-  const bool fold = !fork && dir && rec && !(flags & kCalcNoFinalize);
+  const bool fold = !plan.fork && dir && rec && !(flags & kCalcNoFinalize);
   const bool pair_first = S.pair_first || fold;
-  if (dir && pair_first) pair_branch();
-  if (rec) {
-    recip_launch(S, x4, force, stride, E, V, sp, fold);
-    if (fork) APO_HIP(hipEventRecord(S.ev_pme, sp));
+  const bool own = bnd && !plan.merge;  // the bonded terms' own launch
+  // ... before the pair kernel, whose slots it would wait for behind it; energy
+  // calls' pair kernel is the longest branch, so there it follows the gather
+  const bool with_pair = own && !plan.bonded2 && dir && !(E || V);
+  if (dir && pair_first) {
+    if (with_pair) bonded_branch(sd);
+    pair_branch();
   }
-  // bonded after PME (measured: launched first, its blocks delay the sort
-  // and the PME chain)
-  if (bnd) {
-    S.tic(6, sb, t1);
-    if (terms & APO_TERM_PAIRS14) pairs14_launch(S, x4, force, stride, E, V, sb);
-    if (terms & APO_TERM_BONDED) bonded_launch(S, x4, force, stride, E, V, sb);
-    S.toc(6, sb, t1);
-    if (fork) APO_HIP(hipEventRecord(S.ev_bond, sb));
+  if (rec) recip_launch(S, x4, force, stride, E, V, sp, fold);
+  if (own && !with_pair) {
+    bonded_branch(plan.bonded2 ? S.side[1] : sp);
+    if (plan.bonded2) APO_HIP(hipEventRecord(S.ev_bond, S.side[1]));
   }
-  if (dir && !pair_first) pair_branch();
-  if (fork && rec) APO_HIP(hipStreamWaitEvent(s, S.ev_pme, 0));
-  if (fork && bnd) APO_HIP(hipStreamWaitEvent(s, S.ev_bond, 0));
+  if (dir && !pair_first) {
+    if (with_pair) bonded_branch(sd);
+    pair_branch();
+  }
+  if (plan.fork) {
+    APO_HIP(hipEventRecord(S.ev_side, side));
+    APO_HIP(hipStreamWaitEvent(s, S.ev_side, 0));
+    if (plan.bonded2) APO_HIP(hipStreamWaitEvent(s, S.ev_bond, 0));
+  }
   if ((dir || rec) && !fold && !(flags & kCalcNoFinalize)) {
     S.tic(7, s, t0);
     direct_finalize(S, force, stride, s);
@@ -683,12 +710,12 @@ void NbSystem::profile_flush() {
 
 NbSystem::~NbSystem() {
   // list builds write the pinned h_meta from whatever stream the caller gave
-  // them, and PME / bonded work runs on the side streams: drain the device
+  // them, and branches run on the side streams: drain the device
   // before any of them is released
   (void)hipDeviceSynchronize();
   if (h_meta) (void)hipHostFree(h_meta);
   for (auto e : ev_pool) (void)hipEventDestroy(e);
-  for (hipEvent_t e : {ev_fork, ev_sorted, ev_pme, ev_bond})
+  for (hipEvent_t e : {ev_sorted, ev_side, ev_bond})
     if (e) (void)hipEventDestroy(e);
   for (hipStream_t st : side)
     if (st) (void)hipStreamDestroy(st);

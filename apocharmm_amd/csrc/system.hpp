@@ -160,11 +160,11 @@ struct NbSystem {
   // false: list builds must fit the current capacities (no allocation)
   bool may_allocate = true;
 
-  // calc_force runs PME and the bonded/1-4 terms on two side streams that
-  // fork from and join back into the caller's stream
+  // calc_force runs its branches on the caller's stream and up to two side
+  // streams that fork from and join back into it (plan_branches, system.hip)
   hipStream_t side[2] = {nullptr, nullptr};
   bool single_stream = false;  // everything on the caller's stream (batched systems)
-  hipEvent_t ev_fork = nullptr, ev_sorted = nullptr, ev_pme = nullptr, ev_bond = nullptr;
+  hipEvent_t ev_sorted = nullptr, ev_side = nullptr, ev_bond = nullptr;
 
   // HIP-event kernel timers (apo_nb_profile)
   struct TimerRec { int slot; hipEvent_t a, b; };
