@@ -396,19 +396,42 @@ __device__ inline float wave_max(float v) {
 // SETTLE to each water from LDS, and every wave finishes its atoms.  The
 // per-atom arithmetic does not depend on the split.
 constexpr int kStepThreads = 3 * kStepBlock;
+// this block's kinetic energies and displacement maxima
+__device__ __forceinline__ void step_partials(int bid, double ke0, double ke1, float d2, float s2,
+                                              double2 *__restrict__ part,
+                                              float2 *__restrict__ dpart) {
+  __shared__ double red_ke[2][3];
+  __shared__ float red_d[2][3];
+  const int k = threadIdx.x / kStepBlock;
+  ke0 = wave_sum(ke0);
+  ke1 = wave_sum(ke1);
+  d2 = wave_max(d2);
+  s2 = wave_max(s2);
+  if ((threadIdx.x & (kStepBlock - 1)) == 0) {
+    red_ke[0][k] = ke0;
+    red_ke[1][k] = ke1;
+    red_d[0][k] = d2;
+    red_d[1][k] = s2;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    part[bid] = make_double2(red_ke[0][0] + red_ke[0][1] + red_ke[0][2],
+                             red_ke[1][0] + red_ke[1][1] + red_ke[1][2]);
+    dpart[bid] = make_float2(fmaxf(fmaxf(red_d[0][0], red_d[0][1]), red_d[0][2]),
+                             fmaxf(fmaxf(red_d[1][0], red_d[1][1]), red_d[1][2]));
+  }
+}
 __device__ __forceinline__ void lt_step_body(int bid, const LtState &S, const LtCoef &C,
                                              const unsigned long long *__restrict__ stepc,
                                              double2 *__restrict__ part,
                                              float2 *__restrict__ dpart) {
   __shared__ double old_x[3][3][kStepBlock], new_x[3][3][kStepBlock];
-  __shared__ double red_ke[2][3];
-  __shared__ float red_d[2][3];
   const int lane = threadIdx.x & (kStepBlock - 1), k = threadIdx.x / kStepBlock;
   const int u = bid * kStepBlock + lane;
   const unsigned long long step = stepc[0];
   const bool water = u < S.nwater;
   // units: the waters, then the atoms in no water and no SHAKE group (the
-  // SHAKE groups are stepped by k_lt_shake)
+  // SHAKE groups are stepped by lt_shake_body)
   const bool single = !water && k == 0 && u < S.nwater + S.nsingle;
   const int i = water ? S.waters[3 * u + k] : (single ? S.singles[u - S.nwater] : -1);
   double3 r = make_double3(0, 0, 0), p = r, xn = r;
@@ -452,32 +475,87 @@ __device__ __forceinline__ void lt_step_body(int bid, const LtState &S, const Lt
     lt_finish(S, C, i, r, xn, p, ke0, ke1);
     disp_track(S, i, r, xn, d2, s2);
   }
-  ke0 = wave_sum(ke0);
-  ke1 = wave_sum(ke1);
-  d2 = wave_max(d2);
-  s2 = wave_max(s2);
-  if (lane == 0) {
-    red_ke[0][k] = ke0;
-    red_ke[1][k] = ke1;
-    red_d[0][k] = d2;
-    red_d[1][k] = s2;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    part[bid] = make_double2(red_ke[0][0] + red_ke[0][1] + red_ke[0][2],
-                             red_ke[1][0] + red_ke[1][1] + red_ke[1][2]);
-    dpart[bid] = make_float2(fmaxf(fmaxf(red_d[0][0], red_d[0][1]), red_d[0][2]),
-                             fmaxf(fmaxf(red_d[1][0], red_d[1][1]), red_d[1][2]));
-  }
+  step_partials(bid, ke0, ke1, d2, s2, part, dpart);
 }
+// The SHAKE groups of a step, four lanes per group: lane a draws the random
+// force and takes the unconstrained step of atom a (heavy atom, 1-3
+// hydrogens), the quad shares its atoms and each lane solves the group, then
+// finishes its own atom.  Latency bounds a group (random numbers, three or
+// four Newton iterations in FP64), so the blocks run in the water kernel's
+// launch, after its blocks, with their partials after its partials: 790 groups
+// took 34 us in a launch of their own with one lane stepping a group's atoms in
+// turn; water and SHAKE blocks together take 13 (MD of DHFR, 40 steps: 5,817 ->
+// 4,945 us).
+constexpr int kShakeGroups = kStepThreads / 4;  // groups per block
+__device__ __forceinline__ double3 shfl3(double3 v, int lane) {
+  return make_double3(__shfl(v.x, lane, 64), __shfl(v.y, lane, 64), __shfl(v.z, lane, 64));
+}
+__device__ __forceinline__ void lt_shake_body(int bid, int pbid, const LtState &S, const LtCoef &C,
+                                              const unsigned long long *__restrict__ stepc,
+                                              double2 *__restrict__ part,
+                                              float2 *__restrict__ dpart) {
+  const int lane = threadIdx.x & 63, q = threadIdx.x & 3, lead = lane & ~3;
+  const int u = bid * kShakeGroups + (threadIdx.x >> 2);
+  const unsigned long long step = stepc[0];
+  int4 g = make_int4(-1, -1, -1, -1);
+  if (u < S.nshake) g = S.shake[u];
+  const int i = q == 0 ? g.x : (q == 1 ? g.y : (q == 2 ? g.z : g.w));
+  double3 r = make_double3(0, 0, 0), p = r, xn = r;
+  double im = 0.0, ke0 = 0.0, ke1 = 0.0;
+  float d2 = 0.f, s2 = 0.f;
+  if (i >= 0) {
+    r = ld3(S.x, S.n, i);
+    p = ld3(S.dp, S.n, i);
+    im = S.invmass[i];
+    xn = lt_position(S, C, step, i, r, p);
+  }
+  double imq[4];
+  double3 rq[4], nq[4];
+#pragma unroll
+  for (int a = 0; a < 4; a++) {
+    imq[a] = __shfl(im, lead + a, 64);
+    rq[a] = shfl3(r, lead + a);
+    nq[a] = shfl3(xn, lead + a);
+  }
+  if (u < S.nshake) {
+    const double r2 = S.shake_r2[u];
+    with_group_size(g, [&](auto mc) {
+      constexpr int M = decltype(mc)::value;
+      double ima[M + 1];
+      double3 ref[M + 1], nw[M + 1];
+#pragma unroll
+      for (int a = 0; a <= M; a++) {
+        ima[a] = imq[a];
+        ref[a] = rq[a];
+        nw[a] = nq[a];
+      }
+      shake_group<M>(r2, ima, ref, nw);
+#pragma unroll
+      for (int a = 0; a <= M; a++)
+        if (q == a) xn = nw[a];
+    });
+  }
+  if (i >= 0) {
+    lt_finish(S, C, i, r, xn, p, ke0, ke1);
+    disp_track(S, i, r, xn, d2, s2);
+  }
+  step_partials(pbid, ke0, ke1, d2, s2, part, dpart);
+}
+
 // pend: raised for the kinetic-energy reduction of this step, which the next
-// coordinate sort runs (thermo.hpp)
+// coordinate sort runs (thermo.hpp).  SHAKE: blocks from nstep on take the
+// SHAKE groups (a variant, so that the group solve's registers do not limit
+// the water blocks of systems without groups).
+template <bool SHAKE>
 __global__ __launch_bounds__(kStepThreads) void k_lt_step(LtState S, LtCoef C,
                                                           const unsigned long long *__restrict__ stepc,
                                                           double2 *__restrict__ part,
-                                                          float2 *__restrict__ dpart,
+                                                          float2 *__restrict__ dpart, int nstep,
                                                           unsigned long long *__restrict__ pend) {
-  lt_step_body(blockIdx.x, S, C, stepc, part, dpart);
+  if (SHAKE && (int)blockIdx.x >= nstep)
+    lt_shake_body(blockIdx.x - nstep, blockIdx.x, S, C, stepc, part, dpart);
+  else
+    lt_step_body(blockIdx.x, S, C, stepc, part, dpart);
   if (blockIdx.x == 0 && threadIdx.x == 0) *pend = 1ull;
 }
 struct LtStepArgs {
@@ -486,73 +564,18 @@ struct LtStepArgs {
   const unsigned long long *stepc;
   double2 *part;
   float2 *dpart;
+  int nstep;
 };
+template <bool SHAKE>
 __global__ __launch_bounds__(kStepThreads) void kb_lt_step(const LtStepArgs *__restrict__ tab,
                                                          const int *__restrict__ bstart, int nsys) {
   const int s = batch_system(bstart, nsys);
   const LtStepArgs &a = tab[s];
-  lt_step_body(blockIdx.x - bstart[s], a.S, a.C, a.stepc, a.part, a.dpart);
-}
-
-
-// The SHAKE groups of a step: one lane steps, constrains and finishes each
-// group's atoms (heavy atom and 1-3 hydrogens).  Its own launch (one wave per
-// block), so that the registers of the group solve do not limit the
-// occupancy of the water kernel; the blocks' kinetic-energy and displacement
-// partials follow the water kernel's (k_lt_finalize sums both).
-constexpr int kShakeBlock = 64;
-__device__ __forceinline__ void lt_shake_body(int bid, const LtState &S, const LtCoef &C,
-                                              const unsigned long long *__restrict__ stepc,
-                                              double2 *__restrict__ part,
-                                              float2 *__restrict__ dpart) {
-  const int u = bid * kShakeBlock + threadIdx.x;
-  const unsigned long long step = stepc[0];
-  double ke0 = 0.0, ke1 = 0.0;
-  float d2 = 0.f, s2 = 0.f;
-  if (u < S.nshake) {
-    const int4 g = S.shake[u];
-    const double r2 = S.shake_r2[u];
-    with_group_size(g, [&](auto mc) {
-      constexpr int M = decltype(mc)::value;
-      const int at[4] = {g.x, g.y, g.z, g.w};
-      double im[M + 1];
-      double3 ref[M + 1], dp4[M + 1], nw[M + 1];
-#pragma unroll
-      for (int a = 0; a <= M; a++) {
-        im[a] = S.invmass[at[a]];
-        ref[a] = ld3(S.x, S.n, at[a]);
-        dp4[a] = ld3(S.dp, S.n, at[a]);
-        nw[a] = lt_position(S, C, step, at[a], ref[a], dp4[a]);
-      }
-      shake_group<M>(r2, im, ref, nw);
-#pragma unroll
-      for (int a = 0; a <= M; a++) {
-        lt_finish(S, C, at[a], ref[a], nw[a], dp4[a], ke0, ke1);
-        disp_track(S, at[a], ref[a], nw[a], d2, s2);
-      }
-    });
-  }
-  ke0 = wave_sum(ke0);
-  ke1 = wave_sum(ke1);
-  d2 = wave_max(d2);
-  s2 = wave_max(s2);
-  if (threadIdx.x == 0) {
-    part[bid] = make_double2(ke0, ke1);
-    dpart[bid] = make_float2(d2, s2);
-  }
-}
-__global__ __launch_bounds__(kShakeBlock) void k_lt_shake(LtState S, LtCoef C,
-                                                          const unsigned long long *__restrict__ stepc,
-                                                          double2 *__restrict__ part,
-                                                          float2 *__restrict__ dpart) {
-  lt_shake_body(blockIdx.x, S, C, stepc, part, dpart);
-}
-__global__ __launch_bounds__(kShakeBlock) void kb_lt_shake(const LtStepArgs *__restrict__ tab,
-                                                           const int *__restrict__ bstart,
-                                                           int nsys) {
-  const int s = batch_system(bstart, nsys);
-  const LtStepArgs &a = tab[s];
-  lt_shake_body(blockIdx.x - bstart[s], a.S, a.C, a.stepc, a.part, a.dpart);
+  const int bid = blockIdx.x - bstart[s];
+  if (SHAKE && bid >= a.nstep)
+    lt_shake_body(bid - a.nstep, bid, a.S, a.C, a.stepc, a.part, a.dpart);
+  else
+    lt_step_body(bid, a.S, a.C, a.stepc, a.part, a.dpart);
 }
 
 __global__ __launch_bounds__(256) void k_lt_finalize(const double2 *__restrict__ part, int npart,
@@ -776,8 +799,8 @@ struct LtSystem {
   bool use_graph = true;
   double ndof = 0;
   int nwater = 0, nshake = 0, nsingle = 0, nunit_blocks = 0;
-  int nstep_blocks = 0;   // k_lt_step blocks (waters and free atoms)
-  int nshake_blocks = 0;  // k_lt_shake blocks; their partials follow k_lt_step's
+  int nstep_blocks = 0;   // k_lt_step blocks for waters and free atoms
+  int nshake_blocks = 0;  // its blocks for the SHAKE groups, after those
   DevBuf<int4> shake;
   DevBuf<double> shake_r2;
   DevBuf<double> x, dp, v, invmass;
@@ -908,12 +931,14 @@ struct LtSystem {
   void update(hipStream_t s) {
     hipEvent_t t0 = nullptr;
     nb->tic(8, s, t0);
-    k_lt_step<<<nstep_blocks, kStepThreads, 0, s>>>(state(true), C, counters.get(), ke_part.get(),
-                                                  dpart.get(), counters.get() + 3);
-    if (nshake_blocks)
-      k_lt_shake<<<nshake_blocks, kShakeBlock, 0, s>>>(state(true), C, counters.get(),
-                                                      ke_part.get() + nstep_blocks,
-                                                      dpart.get() + nstep_blocks);
+    auto go = [&](auto shake) {
+      k_lt_step<decltype(shake)::value>
+          <<<nstep_blocks + nshake_blocks, kStepThreads, 0, s>>>(
+              state(true), C, counters.get(), ke_part.get(), dpart.get(), nstep_blocks,
+              counters.get() + 3);
+    };
+    if (nshake_blocks) go(std::true_type{});
+    else go(std::false_type{});
     // with the fixed cadence the next force call's coordinate sort reduces
     // this step's kinetic energy (fin_args), and propagate() closes with a
     // reduction of the last step; the displacement check reads every step's
@@ -1285,7 +1310,7 @@ LtSystem *create_lt(NbSystem *nb, const apo_lt_params &p, const double *xyz, con
       sg[g] = make_int4(a[0], a[1], a[2], a[3]);
     }
     // groups ordered by hydrogen count (stable), so that the lanes of a wave
-    // of k_lt_shake mostly take the same solver instantiation
+    // of lt_shake_body mostly take the same solver instantiation
     {
       auto nh = [](const int4 &q) { return q.w >= 0 ? 3 : (q.z >= 0 ? 2 : 1); };
       std::vector<int> order(p.nshake);
@@ -1309,7 +1334,7 @@ LtSystem *create_lt(NbSystem *nb, const apo_lt_params &p, const double *xyz, con
     L->nsingle = (int)singles.size();
     L->nunit_blocks = nblk(L->nwater + L->nshake + L->nsingle, kStepBlock);
     L->nstep_blocks = std::max(1, nblk(L->nwater + L->nsingle, kStepBlock));
-    L->nshake_blocks = nblk(L->nshake, kShakeBlock);
+    L->nshake_blocks = nblk(L->nshake, kShakeGroups);
     L->com_blocks = nblk(n, kStepBlock);
     // P1: 3N - 3, less 3 per SETTLE water and 1 per SHAKE bond
     // (CharmmContext::useHolonomicConstraints, src/CharmmContext.cu:919-945)
@@ -1453,7 +1478,8 @@ struct LtBatch {
   // fused step: one launch per kernel type for all systems
   BatchLaunch<SortArgs> sort;
   BatchLaunch<PairArgs> pair;
-  BatchLaunch<LtStepArgs> lstep, lshake;
+  BatchLaunch<LtStepArgs> lstep;
+  bool has_shake = false;
   BatchLaunch<LtFinArgs> lfin;
   PmeBatch *pme = nullptr;
   BondedBatch *bond = nullptr;
@@ -1495,7 +1521,7 @@ struct LtBatch {
     sort.clear();
     pair.clear();
     lstep.clear();
-    lshake.clear();
+    has_shake = false;
     lfin.clear();
     pme_batch_clear(*pme);
     bonded_batch_clear(*bond);
@@ -1528,12 +1554,9 @@ struct LtBatch {
       pme_batch_add(*pme, S, g, L->gstride, fft_rows, fft_cols, fft_threads);
       bonded_batch_add(*bond, S, x, g, L->gstride);
       lstep.add(LtStepArgs{L->state(true), L->C, L->counters.get(), L->ke_part.get(),
-                           L->dpart.get()},
-                L->nstep_blocks);
-      if (L->nshake_blocks)
-        lshake.add(LtStepArgs{L->state(true), L->C, L->counters.get(),
-                              L->ke_part.get() + L->nstep_blocks, L->dpart.get() + L->nstep_blocks},
-                   L->nshake_blocks);
+                           L->dpart.get(), L->nstep_blocks},
+                L->nstep_blocks + L->nshake_blocks);
+      has_shake = has_shake || L->nshake_blocks > 0;
       lfin.add(LtFinArgs{L->ke_part.get(), L->nstep_blocks + L->nshake_blocks, L->ndof, L->thermo.get(),
                          L->counters.get(), L->dpart.get(), S.meta.get(), L->h_disp, nullptr},
                1);
@@ -1541,7 +1564,6 @@ struct LtBatch {
     sort.upload(m);
     pair.upload(m);
     lstep.upload(m);
-    lshake.upload(m);
     lfin.upload(m);
     pme_batch_upload(*pme, m);
     bonded_batch_upload(*bond, m);
@@ -1550,18 +1572,18 @@ struct LtBatch {
     for (size_t i = 0; i < sys.size(); i++) tab_gens[i] = sys[i]->nb->generation;
   }
 
-  // force path of every system + integrator update: 12 launches in all (13
-  // with SHAKE groups).
+  // force path of every system + integrator update: 12 launches in all.
   // After the sort, the PME chain and the bonded terms fork onto side
   // streams and the pair kernel runs on s; all three write int64 sums, so
   // their overlap changes no bit.
   void fused_step(hipStream_t s) {
     force_step(s);
-    kb_lt_step<<<lstep.blocks(), kStepThreads, 0, s>>>(lstep.d_args.get(), lstep.d_start.get(),
-                                                     lstep.nsys());
-    if (lshake.nsys())
-      kb_lt_shake<<<lshake.blocks(), kShakeBlock, 0, s>>>(lshake.d_args.get(),
-                                                         lshake.d_start.get(), lshake.nsys());
+    if (has_shake)
+      kb_lt_step<true><<<lstep.blocks(), kStepThreads, 0, s>>>(lstep.d_args.get(),
+                                                               lstep.d_start.get(), lstep.nsys());
+    else
+      kb_lt_step<false><<<lstep.blocks(), kStepThreads, 0, s>>>(lstep.d_args.get(),
+                                                                lstep.d_start.get(), lstep.nsys());
     kb_lt_finalize<<<lfin.nsys(), 256, 0, s>>>(lfin.d_args.get());
     APO_LAUNCH_CHECK();
   }
