@@ -363,7 +363,15 @@ __device__ __forceinline__ double readlane_f64(double v, int k) {
   return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
 }
 
-template <typename CT, bool BIG>
+// Whether stencil row p >= -3 (from the slab's first row) lies in a slab of B
+// rows.  WRAP: the axis is shorter than slab and stencil together (K < B + 3),
+// so rows below the slab can come round to it.
+template <bool WRAP> __device__ __forceinline__ bool in_slab(int p, int K, int B) {
+  if (WRAP && p < 0) p += K;
+  return p >= 0 && p < B;
+}
+
+template <typename CT, bool BIG, bool WRAP>
 __device__ __forceinline__ void spread_fftx_body(int bid, const int4 *__restrict__ posq,
                                                  const float4 *__restrict__ bb,
                                                  const int *__restrict__ meta, const BrickGeom &g,
@@ -480,8 +488,8 @@ __device__ __forceinline__ void spread_fftx_body(int bid, const int4 *__restrict
             rtx[4 * r + t] = qs * theta6(c, wx);
             rty[4 * r + t] = theta6(c, wy);
             rtz[4 * r + t] = theta6(c, wz);
-            if (dy + t >= 0 && dy + t < by) ymask |= 1u << t;
-            if (dz + t >= 0 && dz + t < bz) zmask |= 1u << t;
+            if (in_slab<WRAP>(dy + t, g.K1, by)) ymask |= 1u << t;
+            if (in_slab<WRAP>(dz + t, g.K2, bz)) zmask |= 1u << t;
           }
           rpos[r] = ix | ((dy + 3) << 16) | ((dz + 3) << 24);
         }
@@ -511,8 +519,10 @@ __device__ __forceinline__ void spread_fftx_body(int bid, const int4 *__restrict
           const int rr = ent & 31, sy = (ent >> 5) & 3, sz = ent >> 7;
           const int pos = rpos[rr];
           const int px0 = pos & 0xffff;
-          const int py = ((pos >> 16) & 0xff) - 3 + sy;
-          const int pz = (int)((unsigned)pos >> 24) - 3 + sz;
+          int py = ((pos >> 16) & 0xff) - 3 + sy;
+          int pz = (int)((unsigned)pos >> 24) - 3 + sz;
+          if (WRAP && py < 0) py += g.K1;
+          if (WRAP && pz < 0) pz += g.K2;
           unsigned long long *row = slab + (size_t)(pz * by + py) * ss;
           const double wyv = rty[4 * rr + sy], wzv = rtz[4 * rr + sz];
 #pragma unroll
@@ -561,7 +571,7 @@ __device__ __forceinline__ void spread_fftx_body(int bid, const int4 *__restrict
     if (z < g.K2 && y + 1 < g.K1) out[o + H] = B;
   }
 }
-template <typename CT, bool PRIO, bool BIG>
+template <typename CT, bool PRIO, bool BIG, bool WRAP = false>
 __global__ __launch_bounds__(kSpreadThreads) APO_SPREAD_WAVES_ATTR
 void k_spread_fftx(const int4 *__restrict__ posq,
                                                      const float4 *__restrict__ bb,
@@ -570,7 +580,7 @@ void k_spread_fftx(const int4 *__restrict__ posq,
                                                      const typename Cx<CT>::T *__restrict__ twg,
                                                      typename Cx<CT>::T *__restrict__ out) {
   if constexpr (PRIO) pme_wave_priority();
-  spread_fftx_body<CT, BIG>(blockIdx.x, posq, bb, meta, g, qunscale, p, twg, out);
+  spread_fftx_body<CT, BIG, WRAP>(blockIdx.x, posq, bb, meta, g, qunscale, p, twg, out);
 }
 
 // Gather in cell order: 16 lanes per atom; the gradient goes straight into
@@ -895,6 +905,7 @@ template <typename CT> struct PmeShapes {
   GridGeom g;
   BrickGeom bg;
   int nslabs, nrows, npair, rb, wy, ncy, wz, ncz;
+  bool wrap;  // an axis shorter than a slab and a stencil (in_slab)
   int ft;  // threads per block of the y, z and x-inverse passes
   size_t shs, shx, shy, shz;
   ConvArgs c;
@@ -934,6 +945,7 @@ static PmeShapes<CT> pme_shapes(const NbSystem &S, int rows = kFftRowsPerBlock,
   P.bg = BrickGeom{K0, K1, K2, by, bz, (K1 + by - 1) / by, (K2 + bz - 1) / bz, (float)S.box[0],
                    (float)S.box[1], (float)S.box[2]};
   P.nslabs = P.bg.nby * P.bg.nbz;
+  P.wrap = K1 < by + 3 || K2 < bz + 3;
   P.shs = slab_lds<C2>(K0, by, bz);
   P.nrows = K1 * K2;
   P.rb = (int)std::max<size_t>(
@@ -965,8 +977,12 @@ static void recip_t(NbSystem &S, const float4 *x, int64_t *force, int stride, bo
   const double qunscale = 1.0;  // sorted coordinates carry the raw charge
   hipEvent_t t0 = nullptr;
   S.tic(1, s, t0);
-  k_spread_fftx<CT, PRIO, BIG><<<P.nslabs, kSpreadThreads, P.shs, s>>>(
-      S.posq.get(), S.cell_bb.get(), S.meta.get(), P.bg, qunscale, plan_of(S.fx), twx, cgrid);
+  auto spread = [&](auto *k) {
+    k<<<P.nslabs, kSpreadThreads, P.shs, s>>>(S.posq.get(), S.cell_bb.get(), S.meta.get(), P.bg,
+                                              qunscale, plan_of(S.fx), twx, cgrid);
+  };
+  if (P.wrap) spread(k_spread_fftx<CT, false, true, true>);
+  else spread(k_spread_fftx<CT, PRIO, BIG>);
   APO_LAUNCH_CHECK();
   S.toc(1, s, t0);
   S.tic(2, s, t0);
@@ -1062,14 +1078,14 @@ struct GatherArgs {
   int stride;
 };
 
-template <bool BIG>
+template <bool BIG, bool WRAP = false>
 __global__ __launch_bounds__(kSpreadThreads) APO_SPREAD_WAVES_ATTR
 void kb_spread_fftx(const SpreadArgs *__restrict__ tab,
                                                       const int *__restrict__ bstart, int nsys) {
   const int s = batch_system(bstart, nsys);
   const SpreadArgs &a = tab[s];
-  spread_fftx_body<float, BIG>(blockIdx.x - bstart[s], a.posq, a.bb, a.meta, a.g, 1.0, a.p, a.tw,
-                          a.cout);
+  spread_fftx_body<float, BIG, WRAP>(blockIdx.x - bstart[s], a.posq, a.bb, a.meta, a.g, 1.0, a.p,
+                                     a.tw, a.cout);
 }
 template <bool BIG>
 __global__ __launch_bounds__(256) void kb_fftx_inv(const FftxArgs *__restrict__ tab,
@@ -1109,6 +1125,7 @@ struct PmeBatch {
   BatchLaunch<GatherArgs> gather;
   int ft = kFftThreads;  // threads per block of the y, z and x-inverse passes
   bool big = false;      // some system's plans need radices above 5 (plan_big)
+  bool wrap = false;     // some system's spread wraps (PmeShapes::wrap)
 };
 
 PmeBatch *pme_batch_create() { return new PmeBatch(); }
@@ -1119,7 +1136,7 @@ void pme_batch_clear(PmeBatch &b) {
   b.fy.clear();
   b.fz.clear();
   b.gather.clear();
-  b.big = false;
+  b.big = b.wrap = false;
 }
 
 void pme_batch_add(PmeBatch &b, NbSystem &S, int64_t *force, int stride, int fft_rows,
@@ -1127,6 +1144,7 @@ void pme_batch_add(PmeBatch &b, NbSystem &S, int64_t *force, int stride, int fft
   if (S.precision != 0) throw InvalidArgument("fused batches run the mixed-precision path");
   const PmeShapes<float> P = pme_shapes<float>(S, fft_rows, fft_cols, fft_threads, true);
   b.ft = P.ft;
+  b.wrap = b.wrap || P.wrap;
   b.big = b.big || plan_big(S.fx) || plan_big(S.fy) || plan_big(S.fz);
   if (S.K[1] * P.ncz > S.part.recip_n) throw RuntimeError("reciprocal partial buffer too small");
   const int H = S.K[0] / 2 + 1;
@@ -1156,8 +1174,13 @@ void pme_batch_upload(PmeBatch &b, hipStream_t s) {
 // launch each for all systems (cell boxes must be current).  Without the gather the
 // launches write only the batch's grids (the autotuner times them so).
 template <bool BIG> static void pme_batch_launch_t(PmeBatch &b, hipStream_t s, bool gather) {
-  kb_spread_fftx<BIG><<<b.spread.blocks(), kSpreadThreads, b.spread.lds, s>>>(
-      b.spread.d_args.get(), b.spread.d_start.get(), b.spread.nsys());
+  auto spread = [&](auto *k) {
+    k<<<b.spread.blocks(), kSpreadThreads, b.spread.lds, s>>>(b.spread.d_args.get(),
+                                                              b.spread.d_start.get(),
+                                                              b.spread.nsys());
+  };
+  if (b.wrap) spread(kb_spread_fftx<true, true>);
+  else spread(kb_spread_fftx<BIG>);
   kb_ffty<BIG><<<b.fy.blocks(), b.ft, b.fy.lds, s>>>(b.fy.d_args.get(), b.fy.d_start.get(),
                                                     b.fy.nsys(), 0);
   kb_fftz_conv<BIG><<<b.fz.blocks(), b.ft, b.fz.lds, s>>>(b.fz.d_args.get(), b.fz.d_start.get(),
