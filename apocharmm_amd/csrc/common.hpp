@@ -274,6 +274,8 @@ void launch_add_energy(const double *src, double *energy, hipStream_t s);
 void nblist_build(NbSystem &sys, const float4 *d_xyzq, hipStream_t s, bool sizing);
 void list_export_check(NbSystem &sys, hipStream_t s, bool allow_growth);
 void list_reserve(NbSystem &sys, int ncand, int nent, int nitem);
+// LDS of one pair-kernel wave (force calls).
+size_t pair_wave_lds(const NbSystem &sys);
 // Sorts the coordinates into cell order (and the cell boxes); when force is
 // given, also zeroes its nforce entries.
 void nblist_sort_coords(NbSystem &sys, const float4 *d_xyzq, hipStream_t s,
@@ -304,9 +306,10 @@ void direct_finalize(NbSystem &sys, int64_t *d_force, int stride,
 void bonded_launch(NbSystem &sys, const float4 *d_xyzq, int64_t *d_force, int stride, bool energy,
                    bool virial, bool pairs14, bool bonded, hipStream_t s);
 // fold: the gather also adds the sorted pair gradient (direct_finalize), whose
-// kernel must precede this call on the same stream
+// kernel must precede this call on the same stream; shared: the pair kernel
+// runs beside the chain
 void recip_launch(NbSystem &sys, const float4 *d_xyzq, int64_t *d_force,
-                  int stride, bool energy, bool virial, hipStream_t s, bool fold = false);
+                  int stride, bool energy, bool virial, hipStream_t s, bool fold, bool shared);
 // Adds up the partials the terms of this call wrote (and the self energy).
 void reduce_energy_launch(NbSystem &sys, const float4 *d_xyzq, int term_mask, bool energy,
                           bool virial, double *d_energy, double *d_virial,

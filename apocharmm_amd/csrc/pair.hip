@@ -644,6 +644,14 @@ static void launch_pair_t(NbSystem &S, const typename Vec2<CT>::T *tab,
   APO_LAUNCH_CHECK();
 }
 
+size_t pair_wave_lds(const NbSystem &S) {
+  return S.precision == 1
+             ? pair_tab_lds_bytes<double2>(pair_tab_mode<double2>(S.ntypes, S.lj_combine),
+                                           S.ntypes, S.tab_n)
+             : pair_tab_lds_bytes<float2>(pair_tab_mode<float2>(S.ntypes, S.lj_combine), S.ntypes,
+                                          S.tab_n);
+}
+
 void direct_launch(NbSystem &S, const float4 *x, int64_t *force, int stride, bool E, bool V,
                    bool pairs14, bool bonded, hipStream_t s, bool pruned, bool prune_out) {
   const PairBonded bnd{x, force, stride, pairs14, bonded};

@@ -18,6 +18,7 @@
 #include <algorithm>
 #include <cmath>
 #include <type_traits>
+#include <utility>
 
 #include "system.hpp"
 
@@ -40,11 +41,11 @@ __device__ __forceinline__ unsigned magic_dev(int d) {
   return d > 1 ? 0xffffffffu / (unsigned)d + 1u : 0u;
 }
 
-// Whether a transform length needs a radix above 5 (the FFT kernels' variant
-// with the radix-7, 11 and 13 stages).
+// Whether a transform length needs radix 7, 11 or 13 (the FFT kernels' variant
+// with those stages).
 static bool plan_big(const FftDim &d) {
   for (int i = 0; i < d.nrad; i++)
-    if (d.rad[i] > 5) return true;
+    if (d.rad[i] == 7 || d.rad[i] == 11 || d.rad[i] == 13) return true;
   return false;
 }
 
@@ -73,10 +74,16 @@ static FftPlan plan_of(const FftDim &d) {
   return p;
 }
 
+// Every multiply-add of the transforms is written as an fma and contraction is
+// off, so that a transform gives the same bits in whichever kernel it is
+// inlined (a batch's trajectories are bitwise the lone ones).
+__device__ __forceinline__ float fma_ct(float a, float b, float c) { return fmaf(a, b, c); }
+__device__ __forceinline__ double fma_ct(double a, double b, double c) { return fma(a, b, c); }
 template <typename C2> __device__ __forceinline__ C2 cmul(C2 a, C2 b) {
+#pragma clang fp contract(off)
   C2 r;
-  r.x = a.x * b.x - a.y * b.y;
-  r.y = a.x * b.y + a.y * b.x;
+  r.x = fma_ct(a.x, b.x, -(a.y * b.y));
+  r.y = fma_ct(a.x, b.y, a.y * b.x);
   return r;
 }
 template <typename C2> __device__ __forceinline__ C2 cadd(C2 a, C2 b) {
@@ -97,9 +104,53 @@ template <typename C2> __device__ __forceinline__ C2 twid(const C2 *tw, int e, b
   return w;
 }
 
-// Small DFT of length R on registers (forward: e^{-2 pi i r q / R}).
-template <typename C2, int R>
-__device__ __forceinline__ void small_dft(C2 (&v)[R], const C2 *tw, int n, bool inv) {
+// cos and sin of 2 pi r / R, r = 1..(R - 1) / 2, for the odd radices
+constexpr int odd_row(int R) { return R == 3 ? 0 : R == 5 ? 1 : R == 7 ? 2 : R == 11 ? 3 : 4; }
+constexpr double kOddCos[5][6] = {
+    {-0.5},
+    {0.30901699437494745, -0.80901699437494734},
+    {0.62348980185873359, -0.22252093395631434, -0.90096886790241903},
+    {0.84125353283118121, 0.41541501300188644, -0.142314838273285, -0.65486073394528499, -0.95949297361449737},
+    {0.88545602565320991, 0.56806474673115592, 0.12053668025532301, -0.35460488704253545, -0.74851074817110119, -0.97094181742605201}};
+constexpr double kOddSin[5][6] = {
+    {0.86602540378443871},
+    {0.95105651629515353, 0.58778525229247325},
+    {0.7818314824680298, 0.97492791218182362, 0.43388373911755823},
+    {0.54064081745559756, 0.90963199535451833, 0.9898214418809328, 0.75574957435425827, 0.28173255684142967},
+    {0.46472317204376851, 0.82298386589365635, 0.99270887409805397, 0.93501624268541483, 0.66312265824079519, 0.23931566428755768}};
+constexpr double odd_cos(int R, int r) {  // r mod R
+  r %= R;
+  return r == 0 ? 1.0 : kOddCos[odd_row(R)][(r <= R / 2 ? r : R - r) - 1];
+}
+constexpr double odd_sin(int R, int r) {
+  r %= R;
+  return r == 0 ? 0.0
+                : (r <= R / 2 ? kOddSin[odd_row(R)][r - 1] : -kOddSin[odd_row(R)][R - r - 1]);
+}
+// cos and sin of 2 pi q / R for the even radices 6, 8 and 10, from those of R / 2
+constexpr double kSqrtHalf = 0.70710678118654752440;
+constexpr double even_cos(int R, int q) {  // 0 <= q < R / 2
+  if (R == 8) return q == 0 ? 1.0 : q == 1 ? kSqrtHalf : q == 2 ? 0.0 : -kSqrtHalf;
+  // 2 pi q / (2 m) = pi q / m: -cos(pi q / m + pi) with m odd
+  return q % 2 == 0 ? odd_cos(R / 2, q / 2) : -odd_cos(R / 2, (q + R / 2) / 2);
+}
+constexpr double even_sin(int R, int q) {
+  if (R == 8) return q == 0 ? 0.0 : q == 2 ? 1.0 : kSqrtHalf;
+  return q % 2 == 0 ? odd_sin(R / 2, q / 2) : -odd_sin(R / 2, (q + R / 2) / 2);
+}
+
+template <int N> struct IntC { static constexpr int value = N; };
+template <int... I, typename F>
+__device__ __forceinline__ void unrolled(std::integer_sequence<int, I...>, F &&f) {
+  (f(IntC<I>{}), ...);
+}
+
+// Small DFT of length R on registers (forward: e^{-2 pi i r q / R}), with its
+// constants in the instructions: the odd radices on sums and differences of
+// mirrored inputs, the even ones above 4 as two of half the length.
+template <typename C2, int R> __device__ __forceinline__ void small_dft(C2 (&v)[R], bool inv) {
+#pragma clang fp contract(off)
+  using T = decltype(v[0].x + v[0].x);
   if constexpr (R == 2) {
     C2 a = v[0], b = v[1];
     v[0] = cadd(a, b);
@@ -114,42 +165,104 @@ __device__ __forceinline__ void small_dft(C2 (&v)[R], const C2 *tw, int n, bool 
     v[2] = csub(s0, s2);
     v[1] = cadd(s1, js3);
     v[3] = csub(s1, js3);
-  } else {
-    C2 o[R];
-    const int st = n / R;
+  } else if constexpr (R % 2 == 0) {
+    constexpr int m = R / 2;
+    C2 e[m], o[m];
 #pragma unroll
-    for (int q = 0; q < R; q++) {
-      C2 s = v[0];
-#pragma unroll
-      for (int r = 1; r < R; r++) s = cadd(s, cmul(v[r], twid(tw, ((r * q) % R) * st, inv)));
-      o[q] = s;
+    for (int q = 0; q < m; q++) {
+      e[q] = v[2 * q];
+      o[q] = v[2 * q + 1];
     }
+    small_dft<C2, m>(e, inv);
+    small_dft<C2, m>(o, inv);
+    v[0] = cadd(e[0], o[0]);
+    v[m] = csub(e[0], o[0]);
+    unrolled(std::make_integer_sequence<int, m - 1>{}, [&](auto qc) {
+      constexpr int q = decltype(qc)::value + 1;
+      constexpr T c = (T)even_cos(R, q), sn = (T)even_sin(R, q);
+      C2 w;
+      w.x = c;
+      w.y = inv ? sn : -sn;
+      const C2 t = cmul(o[q], w);
+      v[q] = cadd(e[q], t);
+      v[q + m] = csub(e[q], t);
+    });
+  } else {
+    // a_q = v0 + sum_r cos(2 pi r q / R) (v_r + v_{R-r}),
+    // b_q = sum_r sin(2 pi r q / R) (v_r - v_{R-r}): outputs a_q -+ i b_q
+    constexpr int h = (R - 1) / 2;
+    C2 p[h], d[h];
 #pragma unroll
-    for (int q = 0; q < R; q++) v[q] = o[q];
+    for (int r = 0; r < h; r++) {
+      p[r] = cadd(v[r + 1], v[R - 1 - r]);
+      d[r] = csub(v[r + 1], v[R - 1 - r]);
+    }
+    const C2 v0 = v[0];
+#pragma unroll
+    for (int r = 0; r < h; r++) v[0] = cadd(v[0], p[r]);
+    unrolled(std::make_integer_sequence<int, h>{}, [&](auto qc) {
+      constexpr int q = decltype(qc)::value + 1;
+      C2 a = v0, b;
+      b.x = 0;
+      b.y = 0;
+      unrolled(std::make_integer_sequence<int, h>{}, [&](auto rc) {
+        constexpr int r = decltype(rc)::value;
+        constexpr T c = (T)odd_cos(R, q * (r + 1)), sn = (T)odd_sin(R, q * (r + 1));
+        a.x = fma_ct(c, p[r].x, a.x);
+        a.y = fma_ct(c, p[r].y, a.y);
+        if constexpr (r == 0) {
+          b.x = sn * d[r].x;
+          b.y = sn * d[r].y;
+        } else {
+          b.x = fma_ct(sn, d[r].x, b.x);
+          b.y = fma_ct(sn, d[r].y, b.y);
+        }
+      });
+      if (inv) {
+        b.x = -b.x;
+        b.y = -b.y;
+      }
+      v[q].x = a.x + b.y;
+      v[q].y = a.y - b.x;
+      v[R - q].x = a.x - b.y;
+      v[R - q].y = a.y + b.x;
+    });
   }
 }
 
-// One Stockham autosort stage of radix R over nrow rows of length n.
-// mbf, mns: magic numbers of n / R and Ns (fdiv).
-template <typename C2, int R>
+// One Stockham autosort stage of radix R over nrow rows of length n, held one
+// after the other (COL false) or as the columns of an n x nrow array (COL true:
+// neighbouring lanes then take neighbouring columns, so LDS reads and writes
+// stay contiguous).  mbf, mns: magic numbers of n / R (COL: nrow) and Ns (fdiv).
+template <typename C2, int R, bool COL>
 __device__ __forceinline__ void fft_stage(const C2 *in, C2 *out, int n, int nrow, int Ns,
                                           unsigned mbf, unsigned mns, const C2 *tw, bool inv) {
   const int nbf = n / R;
   const int step = n / (Ns * R);
+  const int es = COL ? nrow : 1, rs = COL ? 1 : n;  // element and row strides
   for (int w = threadIdx.x; w < nbf * nrow; w += blockDim.x) {
-    const int row = fdiv(w, mbf), j = w - row * nbf;
-    const C2 *ri = in + row * n;
-    C2 *ro = out + row * n;
+    int row, j;
+    if (COL) {
+      j = fdiv(w, mbf);
+      row = w - j * nrow;
+    } else {
+      row = fdiv(w, mbf);
+      j = w - row * nbf;
+    }
+    const C2 *ri = in + row * rs;
+    C2 *ro = out + row * rs;
     const int jq = fdiv(j, mns), k = j - jq * Ns;
     C2 v[R];
 #pragma unroll
-    for (int r = 0; r < R; r++) v[r] = ri[j + r * nbf];
+    for (int r = 0; r < R; r++) v[r] = ri[(j + r * nbf) * es];
+    if (Ns > 1) {  // the first stage's factors are 1
 #pragma unroll
-    for (int r = 1; r < R; r++) v[r] = cmul(v[r], twid(tw, r * k * step, inv));
-    small_dft<C2, R>(v, tw, n, inv);
+      for (int r = 1; r < R; r++) v[r] = cmul(v[r], twid(tw, r * k * step, inv));
+    }
+    small_dft<C2, R>(v, inv);
     const int idxD = jq * Ns * R + k;
 #pragma unroll
-    for (int r = 0; r < R; r++) ro[idxD + r * Ns] = v[r];
+    for (int r = 0; r < R; r++) ro[(idxD + r * Ns) * es] = v[r];
   }
 }
 
@@ -161,23 +274,34 @@ __device__ __forceinline__ void fft_stage(const C2 *in, C2 *out, int n, int nrow
 // register budget of every kernel that contains it (the y pass needs 94
 // VGPRs with them, 44 without), so the launchers pick the variant without
 // them whenever every radix of the plans is at most 5 (plan_big).
-template <typename C2, bool BIG>
+// X: the x transforms, whose plans do not use 6 and 8 (make_fft_dim): without
+// those stages the spread, which holds the transform beside its own registers,
+// spills less.
+template <typename C2, bool BIG, bool COL = false, bool X = false>
 __device__ __forceinline__ C2 *lds_fft(C2 *a, C2 *b, const FftPlan &p, int nrow, const C2 *tw,
                                        bool inv) {
   int Ns = 1;
+  const unsigned mrow = COL ? magic_dev(nrow) : 0u;
   for (int s = 0; s < p.nrad; s++) {
     const int R = p.rad[s];
-    const unsigned mb = p.mbf[s], mn = p.mns[s];
+    const unsigned mb = COL ? mrow : p.mbf[s], mn = p.mns[s];
     switch (R) {
-      case 2: fft_stage<C2, 2>(a, b, p.n, nrow, Ns, mb, mn, tw, inv); break;
-      case 3: fft_stage<C2, 3>(a, b, p.n, nrow, Ns, mb, mn, tw, inv); break;
-      case 4: fft_stage<C2, 4>(a, b, p.n, nrow, Ns, mb, mn, tw, inv); break;
-      case 5: fft_stage<C2, 5>(a, b, p.n, nrow, Ns, mb, mn, tw, inv); break;
+      case 2: fft_stage<C2, 2, COL>(a, b, p.n, nrow, Ns, mb, mn, tw, inv); break;
+      case 3: fft_stage<C2, 3, COL>(a, b, p.n, nrow, Ns, mb, mn, tw, inv); break;
+      case 4: fft_stage<C2, 4, COL>(a, b, p.n, nrow, Ns, mb, mn, tw, inv); break;
+      case 5: fft_stage<C2, 5, COL>(a, b, p.n, nrow, Ns, mb, mn, tw, inv); break;
+      case 6:
+        if constexpr (!X) fft_stage<C2, 6, COL>(a, b, p.n, nrow, Ns, mb, mn, tw, inv);
+        break;
+      case 8:
+        if constexpr (!X) fft_stage<C2, 8, COL>(a, b, p.n, nrow, Ns, mb, mn, tw, inv);
+        break;
+      case 10: fft_stage<C2, 10, COL>(a, b, p.n, nrow, Ns, mb, mn, tw, inv); break;
       default:
         if constexpr (BIG) {
-          if (R == 7) fft_stage<C2, 7>(a, b, p.n, nrow, Ns, mb, mn, tw, inv);
-          else if (R == 11) fft_stage<C2, 11>(a, b, p.n, nrow, Ns, mb, mn, tw, inv);
-          else fft_stage<C2, 13>(a, b, p.n, nrow, Ns, mb, mn, tw, inv);
+          if (R == 7) fft_stage<C2, 7, COL>(a, b, p.n, nrow, Ns, mb, mn, tw, inv);
+          else if (R == 11) fft_stage<C2, 11, COL>(a, b, p.n, nrow, Ns, mb, mn, tw, inv);
+          else fft_stage<C2, 13, COL>(a, b, p.n, nrow, Ns, mb, mn, tw, inv);
         }
         break;
     }
@@ -271,6 +395,10 @@ struct BrickGeom {
   int by, bz;    // rows per slab in y (even) and z
   int nby, nbz;  // slabs per axis
   float L0, L1, L2;
+  // complex half grid: element (kx, row), row = z K1 + y, at kx sk + row sr:
+  // rows of kx (1, H) for the y and z passes, planes of kx (K1 K2, 1) for the
+  // plane pass
+  int sk, sr;
 };
 
 // LDS of one slab block, all of it dynamic so that the int64 rows start at
@@ -555,7 +683,7 @@ __device__ __forceinline__ void spread_fftx_body(int bid, const int4 *__restrict
     a[e] = v;
   }
   __syncthreads();
-  C2 *res = lds_fft<C2, BIG>(a, b, p, ncx, tw, false);
+  C2 *res = lds_fft<C2, BIG, false, true>(a, b, p, ncx, tw, false);
   for (int e = tid; e < ncx * H; e += kSpreadThreads) {
     const int r = fdiv(e, mh), k = e - r * H;
     const int pz = fdiv(r, mhb), py = 2 * (r - pz * hb);
@@ -566,9 +694,9 @@ __device__ __forceinline__ void spread_fftx_body(int bid, const int4 *__restrict
     A.y = (CT)0.5 * (Z.y - Zm.y);
     B.x = (CT)0.5 * (Z.y + Zm.y);
     B.y = (CT)0.5 * (Zm.x - Z.x);
-    const size_t o = ((size_t)z * g.K1 + y) * H + k;
+    const size_t o = ((size_t)z * g.K1 + y) * g.sr + (size_t)k * g.sk;
     if (z < g.K2 && y < g.K1) out[o] = A;
-    if (z < g.K2 && y + 1 < g.K1) out[o + H] = B;
+    if (z < g.K2 && y + 1 < g.K1) out[o + g.sr] = B;
   }
 }
 template <typename CT, bool PRIO, bool BIG, bool WRAP = false>
@@ -668,7 +796,9 @@ __global__ __launch_bounds__(256) void k_gather_sorted(const int4 *__restrict__ 
 
 // x inverse: complex half rows -> real rows (C2R semantics: the imaginary
 // parts of the k = 0 and Nyquist bins are ignored).
-template <typename CT, bool BIG>
+// PLANE: the grid is in planes of kx (element (kx, row) at kx nrows + row), else
+// in rows of kx.
+template <typename CT, bool PLANE, bool BIG>
 __device__ __forceinline__ void fftx_inv_body(int bid, const typename Cx<CT>::T *__restrict__ in,
                                               int nrows, const FftPlan &p, int rb,
                                               const typename Cx<CT>::T *__restrict__ twg,
@@ -676,31 +806,44 @@ __device__ __forceinline__ void fftx_inv_body(int bid, const typename Cx<CT>::T 
   using C2 = typename Cx<CT>::T;
   extern __shared__ char smem[];
   const int n = p.n, H = n / 2 + 1;
+  const size_t sk = PLANE ? nrows : 1, sr = PLANE ? 1 : H;
   C2 *tw = reinterpret_cast<C2 *>(smem);
   C2 *a = tw + n;
   C2 *b = a + rb * n;
   staged_copy<C2>(n, threadIdx.x, blockDim.x, [&](int e) { return twg[e]; },
                   [&](int e, C2 v) { tw[e] = v; });
   const int r0 = bid * rb;
-  const unsigned mn = magic_dev(n);
+  const unsigned mn = magic_dev(n), mrb = PLANE ? magic_dev(rb) : 0u;
   struct Pair2 {
     C2 A, B;
+  };
+  // lanes along kx where a row of kx is contiguous, else along the row pairs
+  auto split = [&](int e, int &r, int &k) {
+    if (PLANE) {
+      k = fdiv(e, mrb);
+      r = e - k * rb;
+    } else {
+      r = fdiv(e, mn);
+      k = e - r * n;
+    }
   };
   staged_copy<Pair2>(
       rb * n, threadIdx.x, blockDim.x,
       [&](int e) {
-        const int r = fdiv(e, mn), k = e - r * n;
+        int r, k;
+        split(e, r, k);
         const int ra = 2 * (r0 + r), rbw = ra + 1;
         const int kk = k > n / 2 ? n - k : k;
         Pair2 q;
         q.A = C2{0, 0};
         q.B = C2{0, 0};
-        if (ra < nrows) q.A = in[(size_t)ra * H + kk];
-        if (rbw < nrows) q.B = in[(size_t)rbw * H + kk];
+        if (ra < nrows) q.A = in[ra * sr + kk * sk];
+        if (rbw < nrows) q.B = in[rbw * sr + kk * sk];
         return q;
       },
       [&](int e, Pair2 q) {
-        const int k = e - fdiv(e, mn) * n;
+        int r, k;
+        split(e, r, k);
         const bool mirror = k > n / 2;
         const int kk = mirror ? n - k : k;
         C2 A = q.A, B = q.B;
@@ -715,10 +858,10 @@ __device__ __forceinline__ void fftx_inv_body(int bid, const typename Cx<CT>::T 
         C2 Z;
         Z.x = A.x - B.y;
         Z.y = A.y + B.x;
-        a[e] = Z;
+        a[r * n + k] = Z;
       });
   __syncthreads();
-  C2 *res = lds_fft<C2, BIG>(a, b, p, rb, tw, true);
+  C2 *res = lds_fft<C2, BIG, false, true>(a, b, p, rb, tw, true);
   for (int e = threadIdx.x; e < rb * n; e += blockDim.x) {
     const int r = fdiv(e, mn), x = e - r * n;
     const int ra = 2 * (r0 + r), rbw = ra + 1;
@@ -726,13 +869,13 @@ __device__ __forceinline__ void fftx_inv_body(int bid, const typename Cx<CT>::T 
     if (rbw < nrows) phi[(size_t)rbw * n + x] = res[e].y;
   }
 }
-template <typename CT, bool PRIO, bool BIG>
+template <typename CT, bool PLANE, bool PRIO, bool BIG>
 __global__ __launch_bounds__(256) void k_fftx_inv(const typename Cx<CT>::T *__restrict__ in,
                                                   int nrows, FftPlan p, int rb,
                                                   const typename Cx<CT>::T *__restrict__ twg,
                                                   CT *__restrict__ phi) {
   if constexpr (PRIO) pme_wave_priority();
-  fftx_inv_body<CT, BIG>(blockIdx.x, in, nrows, p, rb, twg, phi);
+  fftx_inv_body<CT, PLANE, BIG>(blockIdx.x, in, nrows, p, rb, twg, phi);
 }
 
 
@@ -791,6 +934,63 @@ template <typename CT> __device__ __forceinline__ CT exp_k(CT x);
 template <> __device__ __forceinline__ float exp_k<float>(float x) { return expf(x); }
 template <> __device__ __forceinline__ double exp_k<double>(double x) { return exp(x); }
 
+// The convolution at one point: q *= the Ewald factor, with the point's energy
+// and virial terms.  Contraction is off so that both users give the same bits.
+template <typename CT, bool CALC_EV>
+__device__ __forceinline__ void conv_point(const ConvArgs &c, const CT *pre, int kx, int y, int z,
+                                           typename Cx<CT>::T &q, double (&acc)[7]) {
+#pragma clang fp contract(off)
+  if (kx == 0 && y == 0 && z == 0) {
+    q.x = 0;
+    q.y = 0;
+    return;
+  }
+  const int nf0 = c.K0 / 2 + (c.K0 % 2), nf1 = c.K1 / 2 + (c.K1 % 2), nf2 = c.K2 / 2 + (c.K2 % 2);
+  const int m0 = kx >= nf0 ? kx - c.K0 : kx;
+  const int m1 = y >= nf1 ? y - c.K1 : y;
+  const int m2 = z >= nf2 ? z - c.K2 : z;
+  const CT mh0 = (CT)c.r0 * (CT)m0, mh1 = (CT)c.r1 * (CT)m1, mh2 = (CT)c.r2 * (CT)m2;
+  const CT msq = fma_ct(mh2, mh2, fma_ct(mh1, mh1, mh0 * mh0));
+  const CT msq_inv = (CT)1 / msq;
+  const CT eterm = exp_k<CT>(-(CT)c.fac * msq) * (CT)c.piv_inv * pre[kx] * pre[c.K0 + y] *
+                   pre[c.K0 + c.K1 + z] * msq_inv;
+  if (CALC_EV) {
+    // the x half grid stands for both Hermitian halves: every kx >= 1
+    // column counts twice (the reference's mirror bookkeeping)
+    const CT mult = kx >= 1 ? (CT)2 : (CT)1;
+    const CT t1 = mult * eterm * fma_ct(q.x, q.x, q.y * q.y);
+    const CT vterm = (CT)2 * ((CT)c.fac + msq_inv);
+    const CT t2 = t1 * vterm;
+    acc[0] += (double)t1;
+    acc[1] += (double)(t1 * fma_ct(vterm * mh0, mh0, (CT)-1));
+    acc[2] += (double)(t2 * mh0 * mh1);
+    acc[3] += (double)(t2 * mh0 * mh2);
+    acc[4] += (double)(t1 * fma_ct(vterm * mh1, mh1, (CT)-1));
+    acc[5] += (double)(t2 * mh1 * mh2);
+    acc[6] += (double)(t1 * fma_ct(vterm * mh2, mh2, (CT)-1));
+  }
+  q.x *= eterm;
+  q.y *= eterm;
+}
+// This block's energy and virial partials: energy +1/2 ccelec sum, virial -1/2
+// ccelec sum.
+__device__ __forceinline__ void conv_partials(int bid, const ConvArgs &c, double (&acc)[7],
+                                              double *__restrict__ part) {
+  __shared__ double red[16 * 8];
+  for (int k = 0; k < 7; k++) {
+    double v = acc[k];
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
+    if ((threadIdx.x & 63) == 0) red[(threadIdx.x >> 6) * 8 + k] = v;
+  }
+  __syncthreads();
+  if (threadIdx.x < 7) {
+    double s = 0;
+    for (int w = 0; w < (int)(blockDim.x >> 6); w++) s += red[w * 8 + threadIdx.x];
+    part[bid * kRecipPart + threadIdx.x] =
+        threadIdx.x == 0 ? s * c.half_ccelec : -s * c.half_ccelec;
+  }
+}
+
 // z pass with the k-space convolution in the middle: block = (y, W columns).
 template <typename CT, bool CALC_EV, bool BIG>
 __device__ __forceinline__ void fftz_conv_body(int bid, typename Cx<CT>::T *__restrict__ data,
@@ -805,7 +1005,6 @@ __device__ __forceinline__ void fftz_conv_body(int bid, typename Cx<CT>::T *__re
   C2 *a = tw + n;
   C2 *b = a + W * n;
   CT *pre = reinterpret_cast<CT *>(b + W * n);
-  __shared__ double red[4 * 8];
   staged_copy<C2>(n, threadIdx.x, blockDim.x, [&](int e) { return twg[e]; },
                   [&](int e, C2 v) { tw[e] = v; });
   staged_copy<CT>(c.K0 + c.K1 + c.K2, threadIdx.x, blockDim.x, [&](int e) { return prefac[e]; },
@@ -828,41 +1027,10 @@ __device__ __forceinline__ void fftz_conv_body(int bid, typename Cx<CT>::T *__re
   __syncthreads();
   C2 *res = lds_fft<C2, BIG>(a, b, p, wc, tw, false);
   double acc[7] = {0, 0, 0, 0, 0, 0, 0};
-  const int nf0 = c.K0 / 2 + (c.K0 % 2), nf1 = c.K1 / 2 + (c.K1 % 2), nf2 = c.K2 / 2 + (c.K2 % 2);
   for (int e = threadIdx.x; e < wc * n; e += blockDim.x) {
     const int col = fdiv(e, mn), z = e - col * n;
-    const int kx = kx0 + col;
     C2 q = res[e];
-    if (kx == 0 && y == 0 && z == 0) {
-      q.x = 0;
-      q.y = 0;
-    } else {
-      const int m0 = kx >= nf0 ? kx - c.K0 : kx;
-      const int m1 = y >= nf1 ? y - c.K1 : y;
-      const int m2 = z >= nf2 ? z - c.K2 : z;
-      const CT mh0 = (CT)c.r0 * (CT)m0, mh1 = (CT)c.r1 * (CT)m1, mh2 = (CT)c.r2 * (CT)m2;
-      const CT msq = mh0 * mh0 + mh1 * mh1 + mh2 * mh2;
-      const CT msq_inv = (CT)1 / msq;
-      const CT eterm = exp_k<CT>(-(CT)c.fac * msq) * (CT)c.piv_inv * pre[kx] *
-                       pre[c.K0 + y] * pre[c.K0 + c.K1 + z] * msq_inv;
-      if (CALC_EV) {
-        // the x half grid stands for both Hermitian halves: every kx >= 1
-        // column counts twice (the reference's mirror bookkeeping)
-        const CT mult = kx >= 1 ? (CT)2 : (CT)1;
-        const CT t1 = mult * eterm * (q.x * q.x + q.y * q.y);
-        const CT vterm = (CT)2 * ((CT)c.fac + msq_inv);
-        const CT t2 = t1 * vterm;
-        acc[0] += (double)t1;
-        acc[1] += (double)(t1 * (vterm * mh0 * mh0 - (CT)1));
-        acc[2] += (double)(t2 * mh0 * mh1);
-        acc[3] += (double)(t2 * mh0 * mh2);
-        acc[4] += (double)(t1 * (vterm * mh1 * mh1 - (CT)1));
-        acc[5] += (double)(t2 * mh1 * mh2);
-        acc[6] += (double)(t1 * (vterm * mh2 * mh2 - (CT)1));
-      }
-      q.x *= eterm;
-      q.y *= eterm;
-    }
+    conv_point<CT, CALC_EV>(c, pre, kx0 + col, y, z, q, acc);
     res[e] = q;
   }
   __syncthreads();
@@ -872,21 +1040,7 @@ __device__ __forceinline__ void fftz_conv_body(int bid, typename Cx<CT>::T *__re
     const int z = fdiv(e, mw), col = e - z * W;
     if (col < wc) data[(size_t)z * zs + (size_t)y * H + kx0 + col] = out[col * n + z];
   }
-  if (CALC_EV) {
-    for (int k = 0; k < 7; k++) {
-      double v = acc[k];
-      for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-      if ((threadIdx.x & 63) == 0) red[(threadIdx.x >> 6) * 8 + k] = v;
-    }
-    __syncthreads();
-    if (threadIdx.x < 7) {
-      double s = 0;
-      for (int w = 0; w < (int)(blockDim.x >> 6); w++) s += red[w * 8 + threadIdx.x];
-      // energy +1/2 ccelec sum, virial -1/2 ccelec sum
-      part[bid * kRecipPart + threadIdx.x] =
-          threadIdx.x == 0 ? s * c.half_ccelec : -s * c.half_ccelec;
-    }
-  }
+  if constexpr (CALC_EV) conv_partials(bid, c, acc, part);
 }
 template <typename CT, bool CALC_EV, bool PRIO, bool BIG>
 __global__ __launch_bounds__(256) void k_fftz_conv(typename Cx<CT>::T *__restrict__ data, ConvArgs c,
@@ -899,6 +1053,51 @@ __global__ __launch_bounds__(256) void k_fftz_conv(typename Cx<CT>::T *__restric
 }
 
 
+// y and z transforms, convolution and their inverses of one kx plane (K1 x K2,
+// contiguous in memory) in LDS: one block per kx, one launch where the passes
+// take three.  Latency bounds those (a launch, a trip to memory each way and
+// the end of the kernel, 4-7 us each on grids this small), so for small planes
+// H blocks that do all of it win although they use few CUs; larger planes need
+// the passes' blocks (kPlaneMax).
+constexpr int kPlaneThreads = 512;
+template <typename CT, bool CALC_EV, bool PRIO, bool BIG>
+__global__ __launch_bounds__(kPlaneThreads) void k_fft_plane(
+    typename Cx<CT>::T *__restrict__ data, ConvArgs c, FftPlan py, FftPlan pz,
+    const typename Cx<CT>::T *__restrict__ twy, const typename Cx<CT>::T *__restrict__ twz,
+    const CT *__restrict__ prefac, double *__restrict__ part) {
+  using C2 = typename Cx<CT>::T;
+  if constexpr (PRIO) pme_wave_priority();
+  extern __shared__ char smem[];
+  const int K1 = c.K1, K2 = c.K2, n = K1 * K2, tid = threadIdx.x, kx = blockIdx.x;
+  C2 *a = reinterpret_cast<C2 *>(smem);
+  C2 *b = a + n;
+  C2 *ty = b + n;
+  C2 *tz = ty + K1;
+  CT *pre = reinterpret_cast<CT *>(tz + K2);
+  C2 *plane = data + (size_t)kx * n;
+  staged_copy<C2>(n, tid, kPlaneThreads, [&](int e) { return plane[e]; },
+                  [&](int e, C2 v) { a[e] = v; });
+  for (int e = tid; e < K1; e += kPlaneThreads) ty[e] = twy[e];
+  for (int e = tid; e < K2; e += kPlaneThreads) tz[e] = twz[e];
+  for (int e = tid; e < c.K0 + K1 + K2; e += kPlaneThreads) pre[e] = prefac[e];
+  __syncthreads();
+  C2 *r = lds_fft<C2, BIG>(a, b, py, K2, ty, false);
+  r = lds_fft<C2, BIG, true>(r, r == a ? b : a, pz, K1, tz, false);
+  double acc[7] = {0, 0, 0, 0, 0, 0, 0};
+  const unsigned m1 = magic_dev(K1);
+  for (int e = tid; e < n; e += kPlaneThreads) {
+    const int z = fdiv(e, m1), y = e - z * K1;
+    C2 q = r[e];
+    conv_point<CT, CALC_EV>(c, pre, kx, y, z, q, acc);
+    r[e] = q;
+  }
+  __syncthreads();
+  r = lds_fft<C2, BIG, true>(r, r == a ? b : a, pz, K1, tz, true);
+  r = lds_fft<C2, BIG>(r, r == a ? b : a, py, K2, ty, true);
+  for (int e = tid; e < n; e += kPlaneThreads) plane[e] = r[e];
+  if constexpr (CALC_EV) conv_partials(kx, c, acc, part);
+}
+
 // Launch shapes of the reciprocal passes for one system (shared by the
 // single-system launcher and the fused multi-system launch).
 template <typename CT> struct PmeShapes {
@@ -908,6 +1107,8 @@ template <typename CT> struct PmeShapes {
   bool wrap;  // an axis shorter than a slab and a stencil (in_slab)
   int ft;  // threads per block of the y, z and x-inverse passes
   size_t shs, shx, shy, shz;
+  bool plane;  // k_fft_plane instead of the y and z passes
+  size_t shp;
   ConvArgs c;
 };
 
@@ -919,12 +1120,21 @@ template <typename CT> struct PmeShapes {
 // each block walks, so one block per CU is kept, not more.  Any slab
 // shape sums every grid point exactly and pairs the same rows for the x FFT,
 // so the grid is bitwise the same.
+// Plane pass or y and z passes: planes up to 64 x 64 (chain on one stream, plane /
+// passes: 30 / 36 us at 32^3, 42 / 48 at 48^3, 56 / 63 at 64^3; 64 / 68 at 63 x
+// 98, where a call gains 1 %), and beside a pair kernel (shared) only if a
+// CU's LDS holds the plane next to sixteen pair waves' tables: otherwise its
+// blocks wait for pair waves to drain (40 MD steps, plane / passes: 2,370 / 2,667
+// us at 2,745 atoms, 3,172 / 3,485 at 11,748, 4,100 / 4,250 at 23,577; DHFR, whose
+// vdW triangle takes 5 KB a wave, 5,190 / 5,010).
+constexpr int kPlaneMax = 4096;
+constexpr size_t kPlaneLds = 144 * 1024, kCuLds = 160 * 1024;
 template <typename CT>
 // batched: the system is one of a fused batch, whose launch is filled by the
 // other systems, so its slabs are not narrowed for parallelism
 static PmeShapes<CT> pme_shapes(const NbSystem &S, int rows = kFftRowsPerBlock,
                                 int cols = kFftColsPerBlock, int threads = kFftThreads,
-                                bool batched = false) {
+                                bool batched = false, bool shared = false) {
   using C2 = typename Cx<CT>::T;
   PmeShapes<CT> P;
   if (threads < 64 || threads > 256 || threads % 64)
@@ -942,8 +1152,11 @@ static PmeShapes<CT> pme_shapes(const NbSystem &S, int rows = kFftRowsPerBlock,
   }
   if (slab_lds<C2>(K0, by, bz) > lds_cap - 2048)
     throw InvalidArgument("PME grid x dimension too large for the spread slab");
+  P.shp = (size_t)(2 * K1 * K2 + K1 + K2) * sizeof(C2) + (size_t)(K0 + K1 + K2) * sizeof(CT);
+  P.plane = !batched && K1 * K2 <= kPlaneMax && P.shp <= kPlaneLds &&
+            (!shared || P.shp + 16 * pair_wave_lds(S) <= kCuLds);
   P.bg = BrickGeom{K0, K1, K2, by, bz, (K1 + by - 1) / by, (K2 + bz - 1) / bz, (float)S.box[0],
-                   (float)S.box[1], (float)S.box[2]};
+                   (float)S.box[1], (float)S.box[2], P.plane ? K1 * K2 : 1, P.plane ? 1 : H};
   P.nslabs = P.bg.nby * P.bg.nbz;
   P.wrap = K1 < by + 3 || K2 < bz + 3;
   P.shs = slab_lds<C2>(K0, by, bz);
@@ -970,9 +1183,10 @@ template <typename CT, bool PRIO, bool BIG>
 static void recip_t(NbSystem &S, const float4 *x, int64_t *force, int stride, bool EV,
                     typename Cx<CT>::T *cgrid, CT *phi, const typename Cx<CT>::T *twx,
                     const typename Cx<CT>::T *twy, const typename Cx<CT>::T *twz, const CT *pre,
-                    hipStream_t s, bool fold) {
+                    hipStream_t s, bool fold, bool shared) {
   (void)x;
-  const PmeShapes<CT> P = pme_shapes<CT>(S);
+  const PmeShapes<CT> P =
+      pme_shapes<CT>(S, kFftRowsPerBlock, kFftColsPerBlock, kFftThreads, false, shared);
   const int K1 = S.K[1], K2 = S.K[2], H = S.K[0] / 2 + 1;
   const double qunscale = 1.0;  // sorted coordinates carry the raw charge
   hipEvent_t t0 = nullptr;
@@ -986,23 +1200,45 @@ static void recip_t(NbSystem &S, const float4 *x, int64_t *force, int stride, bo
   APO_LAUNCH_CHECK();
   S.toc(1, s, t0);
   S.tic(2, s, t0);
-  k_ffty<CT, PRIO, BIG><<<K2 * P.ncy, P.ft, P.shy, s>>>(cgrid, H, K1, P.wy, plan_of(S.fy), twy, 0);
-  APO_LAUNCH_CHECK();
-  if (K1 * P.ncz > S.part.recip_n) throw RuntimeError("reciprocal partial buffer too small");
   double *part = S.parts_ptr() + S.part.recip_off;
-  if (EV) {
-    S.part.recip_used = K1 * P.ncz;
-    k_fftz_conv<CT, true, PRIO, BIG><<<K1 * P.ncz, P.ft, P.shz, s>>>(cgrid, P.c, plan_of(S.fz), twz,
-                                                                pre, part);
+  const int nconv = P.plane ? H : K1 * P.ncz;  // rows of partials
+  if (nconv > S.part.recip_n) throw RuntimeError("reciprocal partial buffer too small");
+  if (EV) S.part.recip_used = nconv;
+  if (P.plane) {
+    auto plane = [&](auto ev) {
+      constexpr bool E = decltype(ev)::value;
+      auto *k = k_fft_plane<CT, E, PRIO, BIG>;
+      if (P.shp > 64 * 1024)
+        APO_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(k),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)P.shp));
+      k<<<H, kPlaneThreads, P.shp, s>>>(cgrid, P.c, plan_of(S.fy), plan_of(S.fz), twy, twz, pre,
+                                        part);
+    };
+    if (EV) plane(std::true_type{});
+    else plane(std::false_type{});
+    APO_LAUNCH_CHECK();
   } else {
-    k_fftz_conv<CT, false, PRIO, BIG><<<K1 * P.ncz, P.ft, P.shz, s>>>(cgrid, P.c, plan_of(S.fz), twz,
-                                                                 pre, part);
+    k_ffty<CT, PRIO, BIG><<<K2 * P.ncy, P.ft, P.shy, s>>>(cgrid, H, K1, P.wy, plan_of(S.fy), twy,
+                                                          0);
+    APO_LAUNCH_CHECK();
+    if (EV)
+      k_fftz_conv<CT, true, PRIO, BIG><<<K1 * P.ncz, P.ft, P.shz, s>>>(cgrid, P.c, plan_of(S.fz),
+                                                                       twz, pre, part);
+    else
+      k_fftz_conv<CT, false, PRIO, BIG><<<K1 * P.ncz, P.ft, P.shz, s>>>(cgrid, P.c, plan_of(S.fz),
+                                                                        twz, pre, part);
+    APO_LAUNCH_CHECK();
+    k_ffty<CT, PRIO, BIG><<<K2 * P.ncy, P.ft, P.shy, s>>>(cgrid, H, K1, P.wy, plan_of(S.fy), twy,
+                                                          1);
+    APO_LAUNCH_CHECK();
   }
-  APO_LAUNCH_CHECK();
-  k_ffty<CT, PRIO, BIG><<<K2 * P.ncy, P.ft, P.shy, s>>>(cgrid, H, K1, P.wy, plan_of(S.fy), twy, 1);
-  APO_LAUNCH_CHECK();
-  k_fftx_inv<CT, PRIO, BIG><<<(P.npair + P.rb - 1) / P.rb, P.ft, P.shx, s>>>(
-      cgrid, P.nrows, plan_of(S.fx), P.rb, twx, phi);
+  auto xinv = [&](auto pl) {
+    k_fftx_inv<CT, decltype(pl)::value, PRIO, BIG>
+        <<<(P.npair + P.rb - 1) / P.rb, P.ft, P.shx, s>>>(cgrid, P.nrows, plan_of(S.fx), P.rb, twx,
+                                                        phi);
+  };
+  if (P.plane) xinv(std::true_type{});
+  else xinv(std::false_type{});
   APO_LAUNCH_CHECK();
   S.toc(2, s, t0);
   S.tic(3, s, t0);
@@ -1015,7 +1251,7 @@ static void recip_t(NbSystem &S, const float4 *x, int64_t *force, int stride, bo
 }
 
 void recip_launch(NbSystem &S, const float4 *x, int64_t *force, int stride, bool E, bool V,
-                  hipStream_t s, bool fold) {
+                  hipStream_t s, bool fold, bool shared) {
   // the issue priority is a template parameter: as a kernel argument, every
   // wave waited for its load before issuing the kernel's own first loads
   auto run = [&](auto prio, auto big) {
@@ -1023,10 +1259,11 @@ void recip_launch(NbSystem &S, const float4 *x, int64_t *force, int stride, bool
     if (S.precision == 1)
       recip_t<double, P, B>(S, x, force, stride, E || V, S.cgrid_d.get(), S.phi_d.get(),
                             S.fx.tw64.get(), S.fy.tw64.get(), S.fz.tw64.get(), S.prefac_d.get(),
-                            s, fold);
+                            s, fold, shared);
     else
       recip_t<float, P, B>(S, x, force, stride, E || V, S.cgrid.get(), S.phi.get(),
-                           S.fx.tw.get(), S.fy.tw.get(), S.fz.tw.get(), S.prefac.get(), s, fold);
+                           S.fx.tw.get(), S.fy.tw.get(), S.fz.tw.get(), S.prefac.get(), s, fold,
+                           shared);
   };
   const bool big = plan_big(S.fx) || plan_big(S.fy) || plan_big(S.fz);
   if (S.pme_prio) {
@@ -1092,7 +1329,7 @@ __global__ __launch_bounds__(256) void kb_fftx_inv(const FftxArgs *__restrict__ 
                                                    const int *__restrict__ bstart, int nsys) {
   const int s = batch_system(bstart, nsys);
   const FftxArgs &a = tab[s];
-  fftx_inv_body<float, BIG>(blockIdx.x - bstart[s], a.cin, a.nrows, a.p, a.rb, a.tw, a.phi);
+  fftx_inv_body<float, false, BIG>(blockIdx.x - bstart[s], a.cin, a.nrows, a.p, a.rb, a.tw, a.phi);
 }
 template <bool BIG>
 __global__ __launch_bounds__(256) void kb_ffty(const FftyArgs *__restrict__ tab,

@@ -172,14 +172,17 @@ static std::vector<double> euler_moduli(int order, int K) {
   return mod;
 }
 
-static void make_fft_dim(FftDim &d, int n, hipStream_t s) {
+// The largest radices first: a stage costs a trip through LDS and a barrier.
+// xdim: the x transforms do without 6 and 8 (lds_fft).
+static void make_fft_dim(FftDim &d, int n, hipStream_t s, bool xdim) {
   d.n = n;
   d.nrad = 0;
   int m = n;
-  const int pref[] = {4, 2, 3, 5, 7, 11, 13};
+  const int pref[] = {10, 8, 6, 5, 4, 3, 2, 7, 11, 13};
   while (m > 1) {
     bool found = false;
     for (int r : pref) {
+      if (xdim && (r == 6 || r == 8)) continue;
       if (m % r == 0) {
         if (d.nrad >= 16) throw InvalidArgument("FFT size has too many factors");
         d.rad[d.nrad++] = r;
@@ -207,9 +210,9 @@ void NbSystem::setup_pme() {
   if (order != 4) throw InvalidArgument("only PME spline order 4 is supported");
   for (int d = 0; d < 3; d++)
     if (K[d] < 4 || K[d] > 1024) throw InvalidArgument("FFT grid size out of range [4, 1024]");
-  make_fft_dim(fx, K[0], 0);
-  make_fft_dim(fy, K[1], 0);
-  make_fft_dim(fz, K[2], 0);
+  make_fft_dim(fx, K[0], 0, true);
+  make_fft_dim(fy, K[1], 0, false);
+  make_fft_dim(fz, K[2], 0, false);
   size_t ng = (size_t)K[0] * K[1] * K[2];
   size_t nc = (size_t)(K[0] / 2 + 1) * K[1] * K[2];
   if (precision == 1) {
@@ -641,7 +644,7 @@ void calc_force(NbSystem &S, const float *xyzq, int flags, int64_t *force, int s
     if (with_pair) bonded_branch(sd);
     pair_branch();
   }
-  if (rec) recip_launch(S, x4, force, stride, E, V, sp, fold);
+  if (rec) recip_launch(S, x4, force, stride, E, V, sp, fold, plan.fork);
   if (own && !with_pair) {
     bonded_branch(plan.bonded2 ? S.side[1] : sp);
     if (plan.bonded2) APO_HIP(hipEventRecord(S.ev_bond, S.side[1]));
