@@ -1238,12 +1238,8 @@ static void recip_t(NbSystem &S, const float4 *x, int64_t *force, int stride, bo
   if (P.plane) {
     auto plane = [&](auto ev) {
       constexpr bool E = decltype(ev)::value;
-      auto *k = k_fft_plane<CT, E, PRIO, BIG>;
-      if (P.shp > 64 * 1024)
-        APO_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(k),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)P.shp));
-      k<<<H, kPlaneThreads, P.shp, s>>>(cgrid, P.c, plan_of(S.fy), plan_of(S.fz), twy, twz, pre,
-                                        part);
+      k_fft_plane<CT, E, PRIO, BIG><<<H, kPlaneThreads, P.shp, s>>>(
+          cgrid, P.c, plan_of(S.fy), plan_of(S.fz), twy, twz, pre, part);
     };
     if (EV) plane(std::true_type{});
     else plane(std::false_type{});
