@@ -259,19 +259,13 @@ struct SortArgs {
 };
 void launch_fill_f64(double *p, size_t n, hipStream_t s);
 void launch_fill_i32(int *p, size_t n, hipStream_t s);
-// exclusive scans, out[n] = total (also to *total_dst when given); scan2 runs
-// two independent scans in one launch
-void launch_scan(const int *in, int *out, const int *n_dev, int n_max, hipStream_t s,
-                 int *total_dst = nullptr);
-void launch_scan2(const int *in0, int *out0, const int *n0_dev, int n0_max, int *total0,
-                  const int *in1, int *out1, const int *n1_dev, int n1_max, int *total1,
-                  hipStream_t s);
 void launch_force_to_double(const int64_t *f, int natom, int stride,
                             double *out, hipStream_t s);
 void launch_add_force(const int64_t *src, int natom, int stride, int64_t *dst, hipStream_t s);
 void launch_add_energy(const double *src, double *energy, hipStream_t s);
 
-void nblist_build(NbSystem &sys, const float4 *d_xyzq, hipStream_t s, bool sizing);
+bool nblist_build(NbSystem &sys, const float4 *d_xyzq, hipStream_t s, bool sizing,
+                  int64_t *force = nullptr, size_t nforce = 0);
 void list_export_check(NbSystem &sys, hipStream_t s, bool allow_growth);
 void list_reserve(NbSystem &sys, int ncand, int nent, int nitem);
 // LDS of one pair-kernel wave (force calls).

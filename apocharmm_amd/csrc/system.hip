@@ -484,14 +484,13 @@ NbSystem *create_system(const apo_nb_params &p, const apo_nb_topology &t) {
     for (int k = 0; k < 16; k++) S->h_meta[k] = 0;
     S->col_count.reserve(S->ncol + 1);
     S->col_start.reserve(S->ncol + 1);
-    S->col_ncell.reserve(S->ncol + 1);
     S->col_cellstart.reserve(S->ncol + 1);
     S->atom_col.reserve(n);
     S->atom_slot.reserve(n);
     S->colkeys.reserve(n);
     S->zkey.reserve(n);
-    for (auto *b : {&S->icell_cnt, &S->icell_start}) b->reserve(S->ncell_cap + 1);
-    for (auto *b : {&S->grp_cnt, &S->grp_start, &S->grp_nitem, &S->grp_itemstart})
+    S->icell_start.reserve(S->ncell_cap + 1);
+    for (auto *b : {&S->grp_cnt, &S->grp_start, &S->grp_itemstart})
       b->reserve((size_t)S->ncell_cap * kGroupsPerCell + 1);
 
     // partials layout (fixed block counts -> deterministic reductions)
@@ -598,15 +597,20 @@ void calc_force(NbSystem &S, const float *xyzq, int flags, int64_t *force, int s
   bool rebuilt = false;
   if (dir || rec) {
     // both the pair kernel and PME work on the cell-sorted coordinates
+    int64_t *zero = acc ? nullptr : force;
+    const size_t nzero = acc ? 0 : 3 * (size_t)stride;
+    bool sorted = false;
     if ((flags & APO_RESET_LIST) || !S.list_valid) {
       rebuilt = true;
       S.tic(4, s, t0);
-      nblist_build(S, x4, s, false);
+      sorted = nblist_build(S, x4, s, false, zero, nzero);
       S.toc(4, s, t0);
     }
-    S.tic(7, s, t0);
-    nblist_sort_coords(S, x4, s, acc ? nullptr : force, acc ? 0 : 3 * (size_t)stride);
-    S.toc(7, s, t0);
+    if (!sorted) {
+      S.tic(7, s, t0);
+      nblist_sort_coords(S, x4, s, zero, nzero);
+      S.toc(7, s, t0);
+    }
   }
   if (plan.fork) {
     APO_HIP(hipEventRecord(S.ev_sorted, s));

@@ -90,20 +90,19 @@ struct NbSystem {
   int n_integrators = 0;
   std::vector<int> h_bonds;  // 2 * nbond, host copy for molecule grouping
   DevBuf<int> meta;   // [0] ncell [1] ncand [2] nent [3] nitem [4] maxcol
-  DevBuf<int> col_count, col_start, col_ncell, col_cellstart;
+  DevBuf<int> col_count, col_start, col_cellstart;
   DevBuf<int> atom_col, atom_slot;
   DevBuf<unsigned long long> colkeys;
   DevBuf<float> zkey;
   DevBuf<int> loc2glo, glo2loc;
   DevBuf<float4> cell_bb;  // 2 per cell: center, half extent
-  DevBuf<int> icell_cnt, icell_start;
-  DevBuf<int> cand_i, cand_j;
+  DevBuf<int> icell_start, cand_j;  // first candidate of each cell; their j cells
   DevBuf<uint32_t> cand_mask;
   // pair list: per i-group (kGroup consecutive slots of a cell) the j slots
   // with at least one live pair, packed as (candidate tile index << 5 | slot)
   // | skip-mask << 16 and padded to whole 64-lane steps; items = (group,
   // first entry, end entry, first candidate tile of the group's cell)
-  DevBuf<int> grp_cnt, grp_start, grp_nitem, grp_itemstart;
+  DevBuf<int> grp_cnt, grp_start, grp_itemstart;
   DevBuf<uint32_t> ent;
   DevBuf<int4> items;
   DevBuf<int> item_order;  // items by step count, longest first (pair-kernel order)
