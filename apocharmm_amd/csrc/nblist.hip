@@ -811,7 +811,7 @@ __global__ __launch_bounds__(kItemThreads) void k_list_guard_export(
       }
       const unsigned long long tails = __ballot(rem > 0);
       const int item = item0 + x - nf + __popcll(tails & below);
-      // groups of this round with the same remainder (isteps: power of two)
+      // the wave's 64 groups with the same remainder (isteps: power of two)
       unsigned long long peers = ~0ull;
       for (int bit = 1; bit < isteps; bit <<= 1) {
         const unsigned long long b = __ballot(rem & bit);

@@ -10,7 +10,7 @@
 //   * fr is formed in FP64 per atom (one conversion), B-splines in CT;
 //   * the charge grid is int64 fixed point (2^-40): order-independent sums;
 //   * the 3-D R2C/C2R FFT is five LDS passes of a hand-written mixed-radix
-//     (4, 2, 3, 5, 7, 11, 13) Stockham FFT: x (two real rows packed per complex
+//     (2 to 8, 10, 11, 13) Stockham FFT: x (two real rows packed per complex
 //     transform, run by the spread kernel on the rows it owns), y, [z forward
 //     -> k-space convolution + energy/virial -> z inverse] fused in one kernel,
 //     y inverse, x inverse;
@@ -1160,9 +1160,9 @@ template <typename CT> struct PmeShapes {
 // vdW triangle takes 5 KB a wave, 5,190 / 5,010).
 constexpr int kPlaneMax = 4096;
 constexpr size_t kPlaneLds = 144 * 1024, kCuLds = 160 * 1024;
-template <typename CT>
 // batched: the system is one of a fused batch, whose launch is filled by the
 // other systems, so its slabs are not narrowed for parallelism
+template <typename CT>
 static PmeShapes<CT> pme_shapes(const NbSystem &S, int rows = kFftRowsPerBlock,
                                 int cols = kFftColsPerBlock, int threads = kFftThreads,
                                 bool batched = false, bool shared = false) {
