@@ -147,6 +147,33 @@ static size_t pair_tab_lds_bytes(int mode, int ntypes, int ntab, bool energy = f
   return b;
 }
 
+// OR over the wave, as a scalar: rotations within the 16-lane rows (no LDS
+// round trips, six of which stood in front of every step's first pair), then
+// one lane of each row.
+__device__ __forceinline__ uint32_t wave_or(uint32_t v) {
+  int x = (int)v;
+  x |= __builtin_amdgcn_update_dpp(0, x, 0x128, 0xf, 0xf, true);  // row_ror:8
+  x |= __builtin_amdgcn_update_dpp(0, x, 0x124, 0xf, 0xf, true);
+  x |= __builtin_amdgcn_update_dpp(0, x, 0x122, 0xf, 0xf, true);
+  x |= __builtin_amdgcn_update_dpp(0, x, 0x121, 0xf, 0xf, true);
+  return (uint32_t)(__builtin_amdgcn_readlane(x, 0) | __builtin_amdgcn_readlane(x, 16) |
+                    __builtin_amdgcn_readlane(x, 32) | __builtin_amdgcn_readlane(x, 48));
+}
+
+// Lane k of each 16-lane row to the whole row (row_newbcast; k a constant after
+// unrolling).
+__device__ __forceinline__ int row_lane(int v, int k) {
+#define APO_ROW(K) \
+  case K: return __builtin_amdgcn_update_dpp(0, v, 0x150 + K, 0xf, 0xf, true);
+  switch (k) {
+    APO_ROW(0) APO_ROW(1) APO_ROW(2) APO_ROW(3) APO_ROW(4) APO_ROW(5) APO_ROW(6) APO_ROW(7)
+    APO_ROW(8) APO_ROW(9) APO_ROW(10) APO_ROW(11) APO_ROW(12) APO_ROW(13) APO_ROW(14)
+    APO_ROW(15)
+  }
+#undef APO_ROW
+  return v;
+}
+
 // One wave64 = one work item: an i-group of kGroup consecutive sorted slots
 // and up to kItemSteps steps of 64 packed j entries (candidate tile of the
 // i-cell, slot in that j-cell, skip mask).  Each lane holds one j
@@ -197,6 +224,12 @@ __device__ __forceinline__ void pair_body(
   double2 *sh_erfc =
       reinterpret_cast<double2 *>(smem_pair + ew_bytes + vdw_lds_bytes<T2>(TAB, ntypes));
   double2 *sh_en = sh_erfc + 3 * (P.ntab + 1);
+  // FP32 without energies: the i-charges stay in lanes (every 16-lane row holds
+  // the group's) and are multiplied through a row broadcast; as sixteen more
+  // scalars they were spilled and cost a cross-lane read per i-atom (with the
+  // scalar OR above, calls: 120.1 -> 118.2 us at 23,577 atoms on one stream,
+  // 250.8 -> 248.5 at 94k, where PME shares the chip)
+  constexpr bool QROW = sizeof(CT) == sizeof(float) && !CALC_E;
   const int nt2 = ntypes * ntypes;
   const int lane = threadIdx.x;
   const int nitem = meta[3];
@@ -239,7 +272,7 @@ __device__ __forceinline__ void pair_body(
       pix[k] = __builtin_amdgcn_readlane(pil.x, k);
       piy[k] = __builtin_amdgcn_readlane(pil.y, k);
       piz[k] = __builtin_amdgcn_readlane(pil.z, k);
-      qi[k] = charge_of<CT>(__builtin_amdgcn_readlane(pil.w, k));
+      if (!QROW) qi[k] = charge_of<CT>(__builtin_amdgcn_readlane(pil.w, k));
       const int t = __builtin_amdgcn_readlane(til, k);
       // TAB_PQA: byte offset of the type's row of (inner, outer) float4 pairs
       rowi[k] = TAB == TAB_SQUARE ? t * ntypes : (TAB == TAB_PQA ? t * ntypes * 32 : t);
@@ -248,6 +281,7 @@ __device__ __forceinline__ void pair_body(
         rhi[k] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ljl.y), k));
       }
     }
+    int qrow = pil.w;  // QROW: lane k of each row holds the charge of i-atom k
     CT fi[3 * kGroup];
 #pragma unroll
     for (int k = 0; k < 3 * kGroup; k++) fi[k] = (CT)0;
@@ -278,8 +312,7 @@ __device__ __forceinline__ void pair_body(
       uint32_t mp = m;  // PRUNE: m plus the pairs at or beyond the prune radius
       // i-atoms with no live pair in this step are skipped with a scalar branch
       uint32_t act = ~m & ((1u << kGroup) - 1u);
-      for (int off = 32; off > 0; off >>= 1) act |= __shfl_xor(act, off);
-      act = __builtin_amdgcn_readfirstlane(act);
+      act = wave_or(act);
       const CT qj = charge_of<CT>(pj.w) * qfac;
       const int tjb = tj * 32;  // TAB_PQA: byte offset of column tj
       float2 ljj = make_float2(0.f, 0.f);
@@ -302,6 +335,15 @@ __device__ __forceinline__ void pair_body(
         const CT dz = ISO ? dzu : dzu * P.sz;
         const CT r2t = dx * dx + dy * dy + dz * dz;
         if (PRUNE) mp |= (r2t < rp2t ? 0u : 1u) << k;
+        CT qq = 0;
+        if constexpr (QROW) {
+          // here, where every lane is active (the first empty asm keeps the
+          // sixteen broadcasts from being formed ahead of the loop, the second
+          // the product out of the branch)
+          asm volatile("" : "+v"(qrow));
+          qq = charge_of<CT>(row_lane(qrow, k)) * qj;
+          asm volatile("" : "+v"(qq));
+        }
         if (!(m & (1u << k)) && r2t < (ISO ? P.roff2u : P.roff2)) {
           const CT r2 = ISO ? r2t * P.s2 : r2t;
           const CT rinv = rsqrt_ct(r2);
@@ -309,7 +351,8 @@ __device__ __forceinline__ void pair_body(
           const CT rinv3 = rinv2 * rinv;
           const CT rinv6 = rinv3 * rinv3;
           // Coulomb: r dU/dr = -qq f(r) / r
-          const CT qf = qi[k] * qj * coulomb_factor(sh_ew, r2 * rinv);
+          if constexpr (!QROW) qq = qi[k] * qj;
+          const CT qf = qq * coulomb_factor(sh_ew, r2 * rinv);
           CT fv;
           if constexpr (TAB == TAB_PQA) {
             // vdW: P r^-6 - Q r^-3 - A12 r^-12 with the region's coefficients
