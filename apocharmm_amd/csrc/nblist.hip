@@ -12,7 +12,8 @@
 // Differences by design: coordinates are 32-bit fixed point per box edge, so
 // every pair uses its minimum image through integer wrap-around and a tile is
 // one cell pair (no 27 image shifts); the column sort orders (z, atom index)
-// so the list -- and every result -- is bitwise reproducible.
+// so what the list holds -- and every result -- is bitwise reproducible (only
+// the places of the cells' entry runs in their buffer vary).
 #include <algorithm>
 #include <cmath>
 
