@@ -195,7 +195,11 @@ __device__ __forceinline__ int row_lane(int v, int k) {
 // pair are dropped, and each item's surviving entries are packed to the front
 // of its own region (null entries after them, so every entry of the copy
 // stays valid) with the item's end shortened to whole steps.  One wave owns an
-// item, so the packing needs no coordination.  (The idea of pruning the list
+// item, so the packing needs no coordination.
+// Every multiply-add is written as an fma and contraction is off: left to the
+// compiler, which product of a sum it fuses differs between the lone and the
+// batched kernel (r^2 in uneven boxes), and with it the bits of a trajectory.
+// (The idea of pruning the list
 // between builds is GROMACS's dynamic pruning; the reference keeps its list.)
 template <typename CT, bool CALC_E, bool CALC_V, int TAB, bool ISO, bool PRUNE>
 __device__ __forceinline__ void pair_body(
@@ -210,6 +214,7 @@ __device__ __forceinline__ void pair_body(
     const double2 *__restrict__ erfctab, const double2 *__restrict__ vdwen,
     const double2 *__restrict__ vdwtab_e, uint32_t *__restrict__ ent_out,
     int4 *__restrict__ items_out, CT rp2t) {
+#pragma clang fp contract(off)
   static_assert(!ISO || sizeof(CT) == sizeof(float), "fixed-point-unit distances are FP32 only");
   static_assert(!PRUNE || (sizeof(CT) == sizeof(float) && !CALC_E && !CALC_V),
                 "fused pruning is an MD-step variant");
@@ -333,7 +338,7 @@ __device__ __forceinline__ void pair_body(
         const CT dx = ISO ? dxu : dxu * P.sx;
         const CT dy = ISO ? dyu : dyu * P.sy;
         const CT dz = ISO ? dzu : dzu * P.sz;
-        const CT r2t = dx * dx + dy * dy + dz * dz;
+        const CT r2t = fma(dz, dz, fma(dy, dy, dx * dx));
         if (PRUNE) mp |= (r2t < rp2t ? 0u : 1u) << k;
         CT qq = 0;
         if constexpr (QROW) {
@@ -385,7 +390,7 @@ __device__ __forceinline__ void pair_body(
             const CT t6 = fma(mo, P.roffinv3, rinv3), t12 = fma(mo, P.roffinv6, rinv6);
             const CT c6k = c.x * P.k6, c12k = c.y * P.k12;
             const CT c6 = outer ? c6k : c.x, c12 = outer ? c12k : c.y;
-            fv = c6 * t6 * rinv3 - c12 * t12 * rinv6;
+            fv = fma(c6 * t6, rinv3, -(c12 * t12 * rinv6));
           }
           const CT fij = fma(-qf, rinv, fv) * rinv2;
           // gradients per h (ISO: per fixed-point unit), scaled when flushed
@@ -433,18 +438,18 @@ __device__ __forceinline__ void pair_body(
               const double e6 = eo ? er3 - PE.roffinv3 : er3, e12 = eo ? er6 - PE.roffinv6 : er6;
               const double A6 = eo ? PE.k6 : 1.0, A12 = eo ? PE.k12 : 1.0;
               const double C6 = eo ? 0.0 : PE.dv6, C12 = eo ? 0.0 : PE.dv12;
-              ev += ce.y * (1.0 / 12.0) * (A12 * e12 * e12 + C12) -
-                    ce.x * (1.0 / 6.0) * (A6 * e6 * e6 + C6);
+              ev = fma(ce.y * (1.0 / 12.0), fma(A12 * e12, e12, C12), ev);
+              ev = fma(ce.x * (-1.0 / 6.0), fma(A6 * e6, e6, C6), ev);
             }
           }
           if (CALC_V) {
             const CT gx = fij * dx, gy = fij * dy, gz = fij * dz;
-            v0 -= gx * dx;
-            v1 -= gx * dy;
-            v2 -= gx * dz;
-            v3 -= gy * dy;
-            v4 -= gy * dz;
-            v5 -= gz * dz;
+            v0 = fma(-gx, dx, v0);
+            v1 = fma(-gx, dy, v1);
+            v2 = fma(-gx, dz, v2);
+            v3 = fma(-gy, dy, v3);
+            v4 = fma(-gy, dz, v4);
+            v5 = fma(-gz, dz, v5);
           }
         }
       }
@@ -468,12 +473,12 @@ __device__ __forceinline__ void pair_body(
       if (CALC_V) {
         // ISO: the products are in unit^2 x (energy / h^2)
         const double vs = ISO ? (double)P.s2 : 1.0;
-        acc[2] += (double)v0 * vs;
-        acc[3] += (double)v1 * vs;
-        acc[4] += (double)v2 * vs;
-        acc[5] += (double)v3 * vs;
-        acc[6] += (double)v4 * vs;
-        acc[7] += (double)v5 * vs;
+        acc[2] = fma((double)v0, vs, acc[2]);
+        acc[3] = fma((double)v1, vs, acc[3]);
+        acc[4] = fma((double)v2, vs, acc[4]);
+        acc[5] = fma((double)v3, vs, acc[5]);
+        acc[6] = fma((double)v4, vs, acc[6]);
+        acc[7] = fma((double)v5, vs, acc[7]);
       }
     }
     if (PRUNE) {
