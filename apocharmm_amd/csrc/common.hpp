@@ -206,7 +206,7 @@ template <typename CT> struct PairUnits {
   CT roff2, roff2u, flush, flush_u;
   CT ron2;
   CT k6, k12, dv6, dv12, roffinv3, roffinv6;
-  CT kappa;
+  CT kappa, kappa2, two_kappa_sqrtpi;  // NbSystem::tab_direct
   int ntab;       // intervals of the Coulomb table (ntab + 1 entries)
 };
 struct PairArgs {

@@ -1539,7 +1539,8 @@ struct LtBatch {
       batch_add_pair(pair, S, pb);
       // one layout for all: a layout every system allows (pair.hip TAB_*:
       // 4 switched-coefficient LDS table, 1 square LDS, 2 triangular LDS,
-      // 0 global), the global table if any system needs it
+      // 0 global), the global table if any system needs it, and 5 (no Coulomb
+      // table either) if any system has none
       const int m = pair_tab_lds(S);
       if (i_sys == 0) tab_mode = m;
       else if (m != tab_mode) {
@@ -1547,7 +1548,7 @@ struct LtBatch {
         // any system beyond it sends the launch to the global table
         const bool lds_ok = (m == 1 || m == 2 || m == 4) && (tab_mode == 1 || tab_mode == 2 ||
                                                              tab_mode == 4);
-        tab_mode = lds_ok ? 2 : 0;
+        tab_mode = m == 5 || tab_mode == 5 ? 5 : lds_ok ? 2 : 0;
       }
       tab_iso = (i_sys == 0 || tab_iso) && pair_tab_iso(S);
       i_sys++;

@@ -62,6 +62,17 @@ __device__ __forceinline__ double coulomb_factor(const double2 *tab, double r) {
   const double2 a = tab[3 * k], b = tab[3 * k + 1], c = tab[3 * k + 2];
   return fma(fma(fma(fma(fma(c.y, u, c.x), u, b.y), u, b.x), u, a.y), u, a.x);
 }
+// The same from libm (TAB_DIRECT).  exp's argument is formed from r^2, whose
+// rounding weighs half of r's.  Contraction is off so that the lone and the
+// batched kernel give the same bits.
+__device__ __forceinline__ float coulomb_direct(const PairUnits<float> &P, float r2, float r) {
+#pragma clang fp contract(off)
+  return fmaf(P.two_kappa_sqrtpi * r, expf(-P.kappa2 * r2), erfcf(P.kappa * r));
+}
+__device__ __forceinline__ double coulomb_direct(const PairUnits<double> &P, double r2, double r) {
+#pragma clang fp contract(off)
+  return fma(P.two_kappa_sqrtpi * r, exp(-P.kappa2 * r2), erfc(P.kappa * r));
+}
 
 __device__ __forceinline__ float rsqrt_ct(float x) { return __builtin_amdgcn_rsqf(x); }
 // hardware estimate, then one third-order step: y (1 + e/2 + 3 e^2/8) with
@@ -116,12 +127,16 @@ constexpr size_t kMaxTriLdsBytes = 32768;
 // coefficients (P, Q, A12) of the inner and outer regions per type pair
 // (NbSystem::vdwpqa) in LDS, so one table read and three multiply-adds give
 // the vdW force in either region.
-enum { TAB_GLOBAL = 0, TAB_SQUARE = 1, TAB_TRI = 2, TAB_COMBINE = 3, TAB_PQA = 4 };
-template <typename T2> static int pair_tab_mode(int ntypes, bool combine) {
+// TAB_DIRECT: TAB_GLOBAL for systems without a Coulomb table
+// (NbSystem::tab_direct).
+enum { TAB_GLOBAL = 0, TAB_SQUARE = 1, TAB_TRI = 2, TAB_COMBINE = 3, TAB_PQA = 4, TAB_DIRECT = 5 };
+template <typename T2> static int pair_tab_mode(const NbSystem &S) {
+  const int ntypes = S.ntypes;
+  if (S.tab_direct) return TAB_DIRECT;
   if (sizeof(T2) == sizeof(float2) && ntypes <= kMaxTypesPqa) return TAB_PQA;
   if (ntypes <= kMaxTypesLds) return TAB_SQUARE;
   if ((size_t)ntypes * (ntypes + 1) / 2 * sizeof(T2) <= kMaxTriLdsBytes) return TAB_TRI;
-  return combine && sizeof(T2) == sizeof(float2) ? TAB_COMBINE : TAB_GLOBAL;
+  return S.lj_combine && sizeof(T2) == sizeof(float2) ? TAB_COMBINE : TAB_GLOBAL;
 }
 // bytes of the Coulomb table, which precedes the vdW table in LDS
 template <typename CT> __host__ __device__ __forceinline__ int ew_lds_bytes(int ntab) {
@@ -182,7 +197,7 @@ __device__ __forceinline__ int row_lane(int v, int k) {
 // a live pair with them.  i-forces accumulate in 3*kGroup registers and are
 // reduced once per item; j-forces are flushed per step.
 // TAB: where the vdW table is read (TAB_GLOBAL / TAB_SQUARE / TAB_TRI /
-// TAB_COMBINE / TAB_PQA).
+// TAB_COMBINE / TAB_PQA), or TAB_DIRECT.
 // Lengths are in units of the Coulomb table's interval (PairUnits); forces are
 // scaled to A when they are flushed.
 // ISO (cubic box, mixed precision): the coordinate differences stay in
@@ -357,7 +372,11 @@ __device__ __forceinline__ void pair_body(
           const CT rinv6 = rinv3 * rinv3;
           // Coulomb: r dU/dr = -qq f(r) / r
           if constexpr (!QROW) qq = qi[k] * qj;
-          const CT qf = qq * coulomb_factor(sh_ew, r2 * rinv);
+          CT qf;
+          if constexpr (TAB == TAB_DIRECT)
+            qf = qq * coulomb_direct(P, r2, r2 * rinv);
+          else
+            qf = qq * coulomb_factor(sh_ew, r2 * rinv);
           CT fv;
           if constexpr (TAB == TAB_PQA) {
             // vdW: P r^-6 - Q r^-3 - A12 r^-12 with the region's coefficients
@@ -422,7 +441,12 @@ __device__ __forceinline__ void pair_body(
               er2 = fma(ez, ez, fma(ey, ey, ex * ex));
               erinv = rsqrt_ct(er2);
             }
-            el = fma((double)qi[k] * qje, coulomb_factor(sh_erfc, er2 * erinv) * erinv, el);
+            double g;
+            if constexpr (TAB == TAB_DIRECT)
+              g = erfc(PE.kappa * (er2 * erinv));
+            else
+              g = coulomb_factor(sh_erfc, er2 * erinv);
+            el = fma((double)qi[k] * qje, g * erinv, el);
             const double er3 = erinv * erinv * erinv, er6 = er3 * er3;
             const bool eo = er2 > PE.ron2;
             if constexpr (TAB == TAB_PQA) {
@@ -621,6 +645,8 @@ template <typename CT, bool E, bool V, bool ISO>
 static void go_pair_tab(int mode, const PairLaunch &L, const typename Vec2<CT>::T *tab,
                         const typename Vec2<CT>::T *sq, const PairUnits<CT> &P, CT qfac,
                         const PairUnits<double> &PE) {
+  if (!ISO && mode == TAB_DIRECT)
+    return go_pair<CT, E, V, TAB_DIRECT, false>(L, tab, sq, P, qfac, PE);
   if constexpr (sizeof(CT) == sizeof(float)) {
     if (mode == TAB_PQA) return go_pair<CT, E, V, TAB_PQA, ISO>(L, tab, sq, P, qfac, PE);
     if (mode == TAB_COMBINE) return go_pair<CT, E, V, TAB_COMBINE, ISO>(L, tab, sq, P, qfac, PE);
@@ -641,7 +667,7 @@ static void go_pair_iso(bool iso, int mode, const PairLaunch &L, const typename 
 // Whether the pair kernel may form distances in fixed-point units: a cubic
 // box (one unit for x, y and z), mixed precision.
 static bool pair_iso(const NbSystem &S) {
-  return S.precision == 0 && S.box[0] == S.box[1] && S.box[1] == S.box[2];
+  return S.precision == 0 && !S.tab_direct && S.box[0] == S.box[1] && S.box[1] == S.box[2];
 }
 
 // pruned: read the pruned copy; prune_out: read the build's list and write
@@ -651,7 +677,7 @@ static void launch_pair_t(NbSystem &S, const typename Vec2<CT>::T *tab,
                           const typename Vec2<CT>::T *sq, const void *ewtab,
                           const PairUnits<CT> &P, CT qfac, bool E, bool V, hipStream_t s,
                           bool pruned, bool prune_out, const PairBonded *bnd) {
-  const int mode = pair_tab_mode<typename Vec2<CT>::T>(S.ntypes, S.lj_combine);
+  const int mode = pair_tab_mode<typename Vec2<CT>::T>(S);
   pruned = pruned && !prune_out;
   const bool iso = pair_iso(S);
   PairLaunch L{S.posq.get(),
@@ -694,10 +720,8 @@ static void launch_pair_t(NbSystem &S, const typename Vec2<CT>::T *tab,
 
 size_t pair_wave_lds(const NbSystem &S) {
   return S.precision == 1
-             ? pair_tab_lds_bytes<double2>(pair_tab_mode<double2>(S.ntypes, S.lj_combine),
-                                           S.ntypes, S.tab_n)
-             : pair_tab_lds_bytes<float2>(pair_tab_mode<float2>(S.ntypes, S.lj_combine), S.ntypes,
-                                          S.tab_n);
+             ? pair_tab_lds_bytes<double2>(pair_tab_mode<double2>(S), S.ntypes, S.tab_n)
+             : pair_tab_lds_bytes<float2>(pair_tab_mode<float2>(S), S.ntypes, S.tab_n);
 }
 
 void direct_launch(NbSystem &S, const float4 *x, int64_t *force, int stride, bool E, bool V,
@@ -766,6 +790,9 @@ static void batch_pair_t(BatchLaunch<PairArgs> &b, int mode, hipStream_t s) {
                                                            b.nsys());
   else if (mode == TAB_TRI)
     kb_pair<TAB_TRI, ISO><<<b.blocks(), 64, b.lds, s>>>(b.d_args.get(), b.d_start.get(), b.nsys());
+  else if (!ISO && mode == TAB_DIRECT)
+    kb_pair<TAB_DIRECT, false><<<b.blocks(), 64, b.lds, s>>>(b.d_args.get(), b.d_start.get(),
+                                                             b.nsys());
   else if (mode == TAB_COMBINE)
     kb_pair<TAB_COMBINE, ISO><<<b.blocks(), 64, b.lds, s>>>(b.d_args.get(), b.d_start.get(), b.nsys());
   else
@@ -781,7 +808,7 @@ void batch_pair(BatchLaunch<PairArgs> &b, int mode, bool iso, hipStream_t s) {
     batch_pair_t<false>(b, mode, s);
   APO_LAUNCH_CHECK();
 }
-int pair_tab_lds(const NbSystem &S) { return pair_tab_mode<float2>(S.ntypes, S.lj_combine); }
+int pair_tab_lds(const NbSystem &S) { return pair_tab_mode<float2>(S); }
 bool pair_tab_iso(const NbSystem &S) { return pair_iso(S); }
 
 }  // namespace apo

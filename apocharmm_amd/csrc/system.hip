@@ -35,21 +35,32 @@ template <typename F> static void fit_interval(F &&fn, int deg, double *c) {
   }
 }
 
-// Interval edge: the largest power of two with k h <= 1/20 (1/8 A, 96
-// intervals at k = 0.34, r_off = 12), where the cubic's interpolation error,
-// (k h)^4 f^(4) / 3072 < 1e-8 of f(0), is well below FP32 rounding and degree 5
-// reaches 1e-12 in FP64.  At least 1/64 A (r^-12 of a pair in units of h stays
-// in FP32 range), 64 to 512 intervals (1 to 8 KB of LDS in FP32).  A power of
-// two changes no mantissa against A, so neither the unit factor's rounding nor
-// the reciprocal square root's error at the distances that dominate the force
-// moves (with h = r_off / 128 the direct forces' error was 8 % larger).
+// Interval edge: the largest power of two with k h <= 1/22 (1/8 A, 96
+// intervals at k = 0.34, r_off = 12), where the cubic's interpolation error is
+// at most 2e-8 of f(0) (1.5e-8 at k h = 0.0425), below FP32 rounding, and
+// degree 5 reaches 1.2e-12 in FP64.  At least 1/64 A (r^-12 of a pair in units of
+// h stays in FP32 range), 64 to 512 intervals (1 to 8 KB of LDS in FP32).  A
+// power of two changes no mantissa against A, so neither the unit factor's
+// rounding nor the reciprocal square root's error at the distances that
+// dominate the force moves (with h = r_off / 128 the direct forces' error was
+// 8 % larger).
+// Systems the table does not serve that well form the factor from erfc and exp
+// (tab_direct): where 512 intervals or 1/64 A do not give k h <= 1/22; beyond
+// k = 1, where a pair's f is so small that the rounding of r (2 (k r)^2 of f)
+// outweighs that of exp's argument (rms error of f over 0.8 to 9 A, table /
+// exp2 and a fitted erfc: 2.3e-8 / 2.9e-8 at k = 0.34, 9.9e-9 / 1.4e-8 at 1,
+// 5.7e-9 / 4.0e-9 at 1.6, 2.5e-9 / 1.9e-10 at 3); and beyond k r_off = 12 (r_off
+// 35 at k = 0.34), where f near r_off is below 1e-60 and the FP64 polynomials'
+// error grows against it.
 void NbSystem::make_pair_tables() {
-  int e = (int)std::min(20.0, std::max(-6.0, std::floor(std::log2(1.0 / (20.0 * kappa)))));
+  int e = (int)std::min(20.0, std::max(-6.0, std::floor(std::log2(1.0 / (22.0 * kappa)))));
   while (std::ldexp(1.0, e) * 64.0 > ctofnb) e--;
   while (e < -6 || std::ldexp(1.0, e) * 512.0 < ctofnb) e++;
   tab_h = std::ldexp(1.0, e);
   tab_n = (int)std::ceil(ctofnb / tab_h);
   const double xh = kappa * tab_h;
+  tab_direct = xh > 1.0 / 22.0 || kappa > 1.0 || kappa * ctofnb > 12.0;
+  if (tab_direct) tab_n = 0;  // one entry, not read
   std::vector<float4> t(tab_n + 1);
   std::vector<double2> td(3 * (size_t)(tab_n + 1)), te(td.size());
   for (int k = 0; k <= tab_n; k++) {
@@ -119,6 +130,8 @@ void NbSystem::make_pair_consts() {
     pu.roffinv3 = (T)(h3 / roff3);
     pu.roffinv6 = (T)(h6 / roff6);
     pu.kappa = (T)(kappa * h);
+    pu.kappa2 = (T)(kappa * h * kappa * h);
+    pu.two_kappa_sqrtpi = (T)(2.0 * kappa * h / std::sqrt(kPi));
     pu.ntab = tab_n;
   };
   units(pu_f);

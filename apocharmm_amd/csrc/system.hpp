@@ -41,6 +41,7 @@ struct NbSystem {
   // equal intervals of edge tab_h (pair.hip); cubic in FP32, degree 5 in FP64
   double tab_h = 0;
   int tab_n = 0;
+  bool tab_direct = false;  // no table: f from erfc and exp (make_pair_tables)
   DevBuf<float4> ewtab;
   DevBuf<double2> ewtab_d;  // 3 per entry
   DevBuf<double2> erfctab;  // erfc(k r) likewise, for the pair energies
