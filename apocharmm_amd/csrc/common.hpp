@@ -193,8 +193,8 @@ template <typename CT> struct PairConsts {
   CT kappa, kappa2, two_kappa_sqrtpi;
 };
 
-// Constants of the pair kernel, which works in units of h = the interval of
-// its Coulomb table (NbSystem::tab_h): a distance in these units is the table
+// Constants of the pair kernel, which works in units of h = the interval of its
+// FP32 Coulomb table (NbSystem::tab_h): a distance in these units is the table
 // index and the offset inside the interval without another multiply.
 // Lengths below are in h, energies in kcal/mol; the vdW tables the kernel
 // reads (vdwtab, vdwsq, ljtype, vdwpqa) are in the same units.
@@ -207,7 +207,9 @@ template <typename CT> struct PairUnits {
   CT ron2;
   CT k6, k12, dv6, dv12, roffinv3, roffinv6;
   CT kappa, kappa2, two_kappa_sqrtpi;  // NbSystem::tab_direct
-  int ntab;       // intervals of the Coulomb table (ntab + 1 entries)
+  int ntab;       // intervals of the FP32 Coulomb table (ntab + 1 entries)
+  double es;      // intervals of the FP64 erfc table per unit of length; their number
+  int nerfc;
 };
 struct PairArgs {
   const int4 *posq;

@@ -24,16 +24,8 @@
 namespace apo {
 
 template <typename CT> struct Vec2;
-template <> struct Vec2<float> {
-  using T = float2;
-  using Ew = float4;  // Coulomb table: kEw of these per entry
-  static constexpr int kEw = 1;
-};
-template <> struct Vec2<double> {
-  using T = double2;
-  using Ew = double2;
-  static constexpr int kEw = 3;
-};
+template <> struct Vec2<float> { using T = float2; };
+template <> struct Vec2<double> { using T = double2; };
 
 __device__ __forceinline__ unsigned long long fx_round(float v) {
   return (unsigned long long)(long long)__builtin_rintf(v * 1099511627776.0f);
@@ -42,25 +34,19 @@ __device__ __forceinline__ unsigned long long fx_round(double v) {
   return (unsigned long long)(long long)__builtin_rint(v * 1099511627776.0);
 }
 
-// Coulomb factor f(r) = erfc(k r) + 2 k r / sqrt(pi) exp(-k^2 r^2) from the
-// per-interval polynomials in LDS (NbSystem::ewtab): r in units of the
-// interval, r <= ntab + 1 (the last entry serves r that rounds up to r_off).
-// In FP32 this is one 16-byte LDS read and six instructions where exp2, rcp and
+// FP32 Coulomb factor f(r) = erfc(k r) + 2 k r / sqrt(pi) exp(-k^2 r^2) from the
+// per-interval cubics in LDS (NbSystem::ewtab): r in units of the interval, r <=
+// ntab + 1 (the last entry serves r that rounds up to r_off).
+// This is one 16-byte LDS read and six instructions where exp2, rcp and
 // a degree-8 erfc polynomial took about twenty issue slots (VALU instructions
 // of one launch at 93,984 atoms 73.2 M -> 62.9 M).  Kernel alone: 140 -> 134 us
-// there, 57 -> 49 with the virial at 26,988 atoms, FP64 with energies and virial
-// 207 -> 154 at 11,748.  What bounds it then is the latency of one pair's chain
-// (rsq, table read, cubic) over the four waves a SIMD holds.
+// there, 57 -> 49 with the virial at 26,988 atoms.  What bounds it then is the
+// latency of one pair's chain (rsq, table read, cubic) over the four waves a
+// SIMD holds.
 __device__ __forceinline__ float coulomb_factor(const float4 *tab, float r) {
   const float4 c = tab[(unsigned)r];
   const float u = __builtin_amdgcn_fractf(r);
   return fmaf(fmaf(fmaf(c.w, u, c.z), u, c.y), u, c.x);
-}
-__device__ __forceinline__ double coulomb_factor(const double2 *tab, double r) {
-  const unsigned k = (unsigned)r;
-  const double u = r - (double)k;
-  const double2 a = tab[3 * k], b = tab[3 * k + 1], c = tab[3 * k + 2];
-  return fma(fma(fma(fma(fma(c.y, u, c.x), u, b.y), u, b.x), u, a.y), u, a.x);
 }
 // The same from libm (TAB_DIRECT).  exp's argument is formed from r^2, whose
 // rounding weighs half of r's.  Contraction is off so that the lone and the
@@ -138,9 +124,13 @@ template <typename T2> static int pair_tab_mode(const NbSystem &S) {
   if ((size_t)ntypes * (ntypes + 1) / 2 * sizeof(T2) <= kMaxTriLdsBytes) return TAB_TRI;
   return S.lj_combine && sizeof(T2) == sizeof(float2) ? TAB_COMBINE : TAB_GLOBAL;
 }
-// bytes of the Coulomb table, which precedes the vdW table in LDS
+// bytes of the FP32 Coulomb table, which precedes the vdW table in LDS
 template <typename CT> __host__ __device__ __forceinline__ int ew_lds_bytes(int ntab) {
-  return (ntab + 1) * Vec2<CT>::kEw * (int)sizeof(typename Vec2<CT>::Ew);
+  return sizeof(CT) == sizeof(float) ? (ntab + 1) * (int)sizeof(float4) : 0;
+}
+// ... and of the FP64 erfc table, which follows it (FP64, and energies of either)
+template <typename CT> __host__ __device__ __forceinline__ int erfc_lds_bytes(int nerfc) {
+  return (nerfc + 1) * erfc_stride(sizeof(CT) == sizeof(double)) * (int)sizeof(CoefPair);
 }
 // bytes of the vdW table in LDS, padded to 16
 template <typename T2> __host__ __device__ __forceinline__ int vdw_lds_bytes(int mode, int ntypes) {
@@ -150,15 +140,13 @@ template <typename T2> __host__ __device__ __forceinline__ int vdw_lds_bytes(int
                                      : 0;
   return (b + 15) & ~15;
 }
-// energy calls add the erfc table and, with TAB_PQA, the vdW energies
+// energy calls add, with TAB_PQA, the vdW energies
 template <typename T2>
-static size_t pair_tab_lds_bytes(int mode, int ntypes, int ntab, bool energy = false) {
+static size_t pair_tab_lds_bytes(int mode, int ntypes, const NbSystem &S, bool energy = false) {
   using CT = std::conditional_t<sizeof(T2) == sizeof(float2), float, double>;
-  size_t b = (size_t)ew_lds_bytes<CT>(ntab) + vdw_lds_bytes<T2>(mode, ntypes);
-  if (energy) {
-    b += ew_lds_bytes<double>(ntab);
-    if (mode == TAB_PQA) b += 4 * (size_t)ntypes * ntypes * sizeof(double2);
-  }
+  size_t b = (size_t)ew_lds_bytes<CT>(S.tab_n) + vdw_lds_bytes<T2>(mode, ntypes);
+  if (energy || sizeof(CT) == sizeof(double)) b += erfc_lds_bytes<CT>(S.erfc_n);
+  if (energy && mode == TAB_PQA) b += 4 * (size_t)ntypes * ntypes * sizeof(double2);
   return b;
 }
 
@@ -198,8 +186,8 @@ __device__ __forceinline__ int row_lane(int v, int k) {
 // reduced once per item; j-forces are flushed per step.
 // TAB: where the vdW table is read (TAB_GLOBAL / TAB_SQUARE / TAB_TRI /
 // TAB_COMBINE / TAB_PQA), or TAB_DIRECT.
-// Lengths are in units of the Coulomb table's interval (PairUnits); forces are
-// scaled to A when they are flushed.
+// Lengths are in units of the FP32 Coulomb table's interval (PairUnits); forces
+// are scaled to A when they are flushed.
 // ISO (cubic box, mixed precision): the coordinate differences stay in
 // fixed-point units, r^2 is compared with the cutoff in those units and
 // converted once per pair, and the forces accumulate per unit.
@@ -221,12 +209,12 @@ __device__ __forceinline__ void pair_body(
     int bid, int nb, const int4 *__restrict__ posq, const int *__restrict__ types,
     const int4 *__restrict__ items, const int *__restrict__ iorder, const uint32_t *__restrict__ ent,
     const int *__restrict__ cand_j, const int *__restrict__ meta,
-    const typename Vec2<CT>::Ew *__restrict__ ewtab,
+    const float4 *__restrict__ ewtab,
     const typename Vec2<CT>::T *__restrict__ vdwtab, const typename Vec2<CT>::T *__restrict__ vdwsq,
     const float2 *__restrict__ ljtype, const float4 *__restrict__ vdwpqa, int ntypes,
     const PairUnits<CT> &P, CT qfac, unsigned long long *__restrict__ fsort, int ss,
     double *__restrict__ part, const PairUnits<double> &PE,
-    const double2 *__restrict__ erfctab, const double2 *__restrict__ vdwen,
+    const CoefPair *__restrict__ erfctab, const double2 *__restrict__ vdwen,
     const double2 *__restrict__ vdwtab_e, uint32_t *__restrict__ ent_out,
     int4 *__restrict__ items_out, CT rp2t) {
 #pragma clang fp contract(off)
@@ -235,15 +223,15 @@ __device__ __forceinline__ void pair_body(
                 "fused pruning is an MD-step variant");
   static_assert(TAB != TAB_PQA || sizeof(CT) == sizeof(float), "the PQA table is FP32 only");
   using T2 = typename Vec2<CT>::T;
-  using Ew = typename Vec2<CT>::Ew;
+  constexpr bool F64 = sizeof(CT) == sizeof(double);
   extern __shared__ char smem_pair[];
-  Ew *sh_ew = reinterpret_cast<Ew *>(smem_pair);
+  float4 *sh_ew = reinterpret_cast<float4 *>(smem_pair);
   const int ew_bytes = ew_lds_bytes<CT>(P.ntab);
   T2 *sh_tab = reinterpret_cast<T2 *>(smem_pair + ew_bytes);
   float4 *sh_pqa = reinterpret_cast<float4 *>(smem_pair + ew_bytes);
-  double2 *sh_erfc =
-      reinterpret_cast<double2 *>(smem_pair + ew_bytes + vdw_lds_bytes<T2>(TAB, ntypes));
-  double2 *sh_en = sh_erfc + 3 * (P.ntab + 1);
+  CoefPair *sh_erfc =
+      reinterpret_cast<CoefPair *>(smem_pair + ew_bytes + vdw_lds_bytes<T2>(TAB, ntypes));
+  double2 *sh_en = reinterpret_cast<double2 *>(sh_erfc + erfc_stride(F64) * (P.nerfc + 1));
   // FP32 without energies: the i-charges stay in lanes (every 16-lane row holds
   // the group's) and are multiplied through a row broadcast; as sixteen more
   // scalars they were spilled and cost a cross-lane read per i-atom (with the
@@ -254,7 +242,8 @@ __device__ __forceinline__ void pair_body(
   const int lane = threadIdx.x;
   const int nitem = meta[3];
   if (bid < nitem) {
-    for (int k = lane; k < (P.ntab + 1) * Vec2<CT>::kEw; k += 64) sh_ew[k] = ewtab[k];
+    if (!F64)
+      for (int k = lane; k <= P.ntab; k += 64) sh_ew[k] = ewtab[k];
     if (TAB == TAB_PQA) {
       for (int k = lane; k < 2 * nt2; k += 64) sh_pqa[k] = vdwpqa[k];
     } else if (TAB == TAB_SQUARE) {
@@ -262,11 +251,10 @@ __device__ __forceinline__ void pair_body(
     } else if (TAB == TAB_TRI) {
       for (int k = lane; k < ntypes * (ntypes + 1) / 2; k += 64) sh_tab[k] = vdwtab[k];
     }
-    if (CALC_E) {
-      for (int k = lane; k < 3 * (P.ntab + 1); k += 64) sh_erfc[k] = erfctab[k];
-      if (TAB == TAB_PQA)
-        for (int k = lane; k < 4 * nt2; k += 64) sh_en[k] = vdwen[k];
-    }
+    if (CALC_E || F64)
+      for (int k = lane; k < erfc_stride(F64) * (P.nerfc + 1); k += 64) sh_erfc[k] = erfctab[k];
+    if (CALC_E && TAB == TAB_PQA)
+      for (int k = lane; k < 4 * nt2; k += 64) sh_en[k] = vdwen[k];
     __syncthreads();
   }
   const CT flush = ISO ? P.flush_u : P.flush;
@@ -373,10 +361,16 @@ __device__ __forceinline__ void pair_body(
           // Coulomb: r dU/dr = -qq f(r) / r
           if constexpr (!QROW) qq = qi[k] * qj;
           CT qf;
-          if constexpr (TAB == TAB_DIRECT)
+          double g = 0.0;  // erfc(k r)
+          if constexpr (TAB == TAB_DIRECT) {
             qf = qq * coulomb_direct(P, r2, r2 * rinv);
-          else
+          } else if constexpr (F64) {
+            double f;
+            erfc_factors<true>(sh_erfc, r2, rinv, P.es, g, f);
+            qf = qq * f;
+          } else {
             qf = qq * coulomb_factor(sh_ew, r2 * rinv);
+          }
           CT fv;
           if constexpr (TAB == TAB_PQA) {
             // vdW: P r^-6 - Q r^-3 - A12 r^-12 with the region's coefficients
@@ -424,14 +418,13 @@ __device__ __forceinline__ void pair_body(
             // geometry: a pair energy is ~1e2 larger than the sums it
             // cancels into, and FP32 pair arithmetic (~2e-7 relative) would
             // dominate the energy error.  FP64 issue bounds this block:
-            // erfc(k r) from a degree-5 table (errors below 1e-12), the
-            // reciprocal root by one third-order step and, with TAB_PQA, one
-            // polynomial in r^-3 per region replace libm's erfc, a square root
-            // and a divide (kernel with energies and virial, alone: 616 -> 246
+            // erfc(k r) from its table (erfc_factors), the reciprocal root by
+            // one third-order step and, with TAB_PQA, one polynomial in r^-3
+            // per region replace libm's erfc, a square root and a divide (kernel with energies and virial, alone: 616 -> 246
             // us at 93,984 atoms, 191 -> 104 in DHFR, 42 -> 23 at 2,529; all
             // FP64 154 -> 68 at 11,748)
             double er2, erinv;
-            if constexpr (sizeof(CT) == sizeof(double)) {
+            if constexpr (F64) {
               er2 = r2;
               erinv = rinv;
             } else {
@@ -440,12 +433,11 @@ __device__ __forceinline__ void pair_body(
               const double ez = (double)(int)(piz[k] - pj.z) * PE.sz;
               er2 = fma(ez, ez, fma(ey, ey, ex * ex));
               erinv = rsqrt_ct(er2);
+              double f;
+              if constexpr (TAB != TAB_DIRECT)
+                erfc_factors<false>(sh_erfc, er2, erinv, PE.es, g, f);
             }
-            double g;
-            if constexpr (TAB == TAB_DIRECT)
-              g = erfc(PE.kappa * (er2 * erinv));
-            else
-              g = coulomb_factor(sh_erfc, er2 * erinv);
+            if constexpr (TAB == TAB_DIRECT) g = erfc(PE.kappa * (er2 * erinv));
             el = fma((double)qi[k] * qje, g * erinv, el);
             const double er3 = erinv * erinv * erinv, er6 = er3 * er3;
             const bool eo = er2 > PE.ron2;
@@ -534,17 +526,18 @@ __device__ __forceinline__ void pair_body(
   }
 }
 
-// energy calls in mixed precision: three waves per SIMD (168 VGPRs; 179 without
-// the bound, which leaves two)
+// Energy calls in mixed precision: three waves per SIMD (168 VGPRs; 179 without
+// the bound, which leaves two).  FP64: two (the energy and virial variant takes
+// 260 without the bound, one wave: 253 us for a call of 22,287 atoms, with it 208).
 template <typename CT, bool CALC_E, bool CALC_V, int TAB, bool ISO, bool PRUNE>
-__global__ __launch_bounds__(64, CALC_E && sizeof(CT) == sizeof(float) ? 3 : 1) void k_pair(
+__global__ __launch_bounds__(64, sizeof(CT) == sizeof(double) ? 2 : CALC_E ? 3 : 1) void k_pair(
     const int4 *__restrict__ posq, const int *__restrict__ types, const int4 *__restrict__ items,
     const int *__restrict__ iorder, const uint32_t *__restrict__ ent, const int *__restrict__ cand_j, const int *__restrict__ meta,
-    const typename Vec2<CT>::Ew *__restrict__ ewtab,
+    const float4 *__restrict__ ewtab,
     const typename Vec2<CT>::T *__restrict__ vdwtab, const typename Vec2<CT>::T *__restrict__ vdwsq,
     const float2 *__restrict__ ljtype, const float4 *__restrict__ vdwpqa, int ntypes,
     const PairUnits<CT> P, CT qfac, unsigned long long *__restrict__ fsort, int ss,
-    double *__restrict__ part, const PairUnits<double> PE, const double2 *__restrict__ erfctab,
+    double *__restrict__ part, const PairUnits<double> PE, const CoefPair *__restrict__ erfctab,
     const double2 *__restrict__ vdwen, const double2 *__restrict__ vdwtab_e,
     uint32_t *__restrict__ ent_out, int4 *__restrict__ items_out, CT rp2t, int nblocks,
     Bonded14<CT> B) {
@@ -589,14 +582,15 @@ struct PairLaunch {
   const int *iorder;
   const uint32_t *ent;
   const int *cand_j, *meta;
-  const void *ewtab;  // the precision's Coulomb table
+  const float4 *ewtab;
   const float2 *ljtype;
   const float4 *vdwpqa;
   int ntypes;
   unsigned long long *fsort;
   int ss;
   double *part;
-  const double2 *erfctab, *vdwen, *vdwtab_e;  // energy calls
+  const CoefPair *erfctab;
+  const double2 *vdwen, *vdwtab_e;  // energy calls
   int blocks;
   size_t lds;
   hipStream_t s;
@@ -621,7 +615,6 @@ template <typename CT, bool E, bool V, int TAB, bool ISO>
 static void go_pair(const PairLaunch &L, const typename Vec2<CT>::T *tab,
                     const typename Vec2<CT>::T *sq, const PairUnits<CT> &P, CT qfac,
                     const PairUnits<double> &PE) {
-  const auto *ew = static_cast<const typename Vec2<CT>::Ew *>(L.ewtab);
   Bonded14<CT> B{};
   if (!E && !V && L.bnd)
     B = bonded14_args<CT>(*L.S, L.bnd->x, L.bnd->force, L.bnd->stride, L.bnd->pairs14,
@@ -630,14 +623,14 @@ static void go_pair(const PairLaunch &L, const typename Vec2<CT>::T *tab,
   if constexpr (sizeof(CT) == sizeof(float) && !E && !V) {
     if (L.ent_out) {
       k_pair<CT, false, false, TAB, ISO, true><<<grid, 64, L.lds, L.s>>>(
-          L.posq, L.types, L.items, L.iorder, L.ent, L.cand_j, L.meta, ew, tab, sq, L.ljtype, L.vdwpqa,
+          L.posq, L.types, L.items, L.iorder, L.ent, L.cand_j, L.meta, L.ewtab, tab, sq, L.ljtype, L.vdwpqa,
           L.ntypes, P, qfac, L.fsort, L.ss, L.part, PE, L.erfctab, L.vdwen, L.vdwtab_e, L.ent_out, L.items_out,
           L.rp2t, L.blocks, B);
       return;
     }
   }
   k_pair<CT, E, V, TAB, ISO, false><<<grid, 64, L.lds, L.s>>>(
-      L.posq, L.types, L.items, L.iorder, L.ent, L.cand_j, L.meta, ew, tab, sq, L.ljtype, L.vdwpqa,
+      L.posq, L.types, L.items, L.iorder, L.ent, L.cand_j, L.meta, L.ewtab, tab, sq, L.ljtype, L.vdwpqa,
       L.ntypes, P,
       qfac, L.fsort, L.ss, L.part, PE, L.erfctab, L.vdwen, L.vdwtab_e, nullptr, nullptr, (CT)0, L.blocks, B);
 }
@@ -674,9 +667,9 @@ static bool pair_iso(const NbSystem &S) {
 // the pruned copy (mixed-precision MD steps only)
 template <typename CT>
 static void launch_pair_t(NbSystem &S, const typename Vec2<CT>::T *tab,
-                          const typename Vec2<CT>::T *sq, const void *ewtab,
-                          const PairUnits<CT> &P, CT qfac, bool E, bool V, hipStream_t s,
-                          bool pruned, bool prune_out, const PairBonded *bnd) {
+                          const typename Vec2<CT>::T *sq, const PairUnits<CT> &P, CT qfac, bool E,
+                          bool V, hipStream_t s, bool pruned, bool prune_out,
+                          const PairBonded *bnd) {
   const int mode = pair_tab_mode<typename Vec2<CT>::T>(S);
   pruned = pruned && !prune_out;
   const bool iso = pair_iso(S);
@@ -687,7 +680,7 @@ static void launch_pair_t(NbSystem &S, const typename Vec2<CT>::T *tab,
                pruned ? S.ent_p.get() : S.ent.get(),
                S.cand_j.get(),
                S.meta.get(),
-               ewtab,
+               S.ewtab.get(),
                S.ljtype.get(),
                S.vdwpqa.get(),
                S.ntypes,
@@ -698,7 +691,7 @@ static void launch_pair_t(NbSystem &S, const typename Vec2<CT>::T *tab,
                S.vdwen.get(),
                S.vdwtab_d.get(),
                S.pair_blocks,
-               pair_tab_lds_bytes<typename Vec2<CT>::T>(mode, S.ntypes, S.tab_n, E),
+               pair_tab_lds_bytes<typename Vec2<CT>::T>(mode, S.ntypes, S, E),
                s,
                prune_out ? S.ent_p.get() : nullptr,
                prune_out ? S.items_p.get() : nullptr,
@@ -720,8 +713,8 @@ static void launch_pair_t(NbSystem &S, const typename Vec2<CT>::T *tab,
 
 size_t pair_wave_lds(const NbSystem &S) {
   return S.precision == 1
-             ? pair_tab_lds_bytes<double2>(pair_tab_mode<double2>(S), S.ntypes, S.tab_n)
-             : pair_tab_lds_bytes<float2>(pair_tab_mode<float2>(S), S.ntypes, S.tab_n);
+             ? pair_tab_lds_bytes<double2>(pair_tab_mode<double2>(S), S.ntypes, S)
+             : pair_tab_lds_bytes<float2>(pair_tab_mode<float2>(S), S.ntypes, S);
 }
 
 void direct_launch(NbSystem &S, const float4 *x, int64_t *force, int stride, bool E, bool V,
@@ -730,10 +723,10 @@ void direct_launch(NbSystem &S, const float4 *x, int64_t *force, int stride, boo
   if (prune_out && (S.precision != 0 || E || V))
     throw InvalidArgument("fused list pruning runs in mixed-precision MD steps only");
   if (S.precision == 1)
-    launch_pair_t<double>(S, S.vdwtab_d.get(), S.vdwsq_d.get(), S.ewtab_d.get(), S.pu_d,
-                          kCcelec / S.tab_h, E, V, s, pruned, false, &bnd);
+    launch_pair_t<double>(S, S.vdwtab_d.get(), S.vdwsq_d.get(), S.pu_d, kCcelec / S.tab_h, E, V, s,
+                          pruned, false, &bnd);
   else
-    launch_pair_t<float>(S, S.vdwtab.get(), S.vdwsq.get(), S.ewtab.get(), S.pu_f,
+    launch_pair_t<float>(S, S.vdwtab.get(), S.vdwsq.get(), S.pu_f,
                          (float)(kCcelec / S.tab_h), E, V, s, pruned, prune_out, &bnd);
 }
 
@@ -773,12 +766,12 @@ void batch_add_pair(BatchLaunch<PairArgs> &b, NbSystem &S, int blocks) {
              reinterpret_cast<unsigned long long *>(S.fsort.get()), S.ssort};
   // LDS of every layout this system allows: the launch uses one that every
   // system of the batch allows
-  const size_t tri = pair_tab_lds_bytes<float2>(TAB_TRI, S.ntypes, S.tab_n);
-  size_t lds = pair_tab_lds_bytes<float2>(TAB_GLOBAL, S.ntypes, S.tab_n);
+  const size_t tri = pair_tab_lds_bytes<float2>(TAB_TRI, S.ntypes, S);
+  size_t lds = pair_tab_lds_bytes<float2>(TAB_GLOBAL, S.ntypes, S);
   if (tri <= lds + kMaxTriLdsBytes) lds = tri;
   for (int m : {TAB_SQUARE, TAB_PQA})
     if (S.ntypes <= (m == TAB_PQA ? kMaxTypesPqa : kMaxTypesLds))
-      lds = std::max(lds, pair_tab_lds_bytes<float2>(m, S.ntypes, S.tab_n));
+      lds = std::max(lds, pair_tab_lds_bytes<float2>(m, S.ntypes, S));
   b.add(a, blocks, lds);
 }
 template <bool ISO>

@@ -10,40 +10,22 @@
 namespace apo {
 
 // ---------------------------------------------------------------------------
-// Coulomb table of the pair kernel: f(r) = erfc(k r) + 2 k r / sqrt(pi)
-// exp(-k^2 r^2) as one polynomial per interval, interpolated at Chebyshev
-// nodes in double at set-up for the system's own k and r_off.
+// Coulomb tables of the pair kernel (coulomb_table.hpp), fitted at set-up for
+// the system's own k and r_off: f(r) = erfc(k r) + 2 k r / sqrt(pi)
+// exp(-k^2 r^2) as one cubic per interval in FP32, erfc(k r) in FP64.
 // ---------------------------------------------------------------------------
 static double coulomb_f(double x) {  // x = k r
   return std::erfc(x) + 2.0 / std::sqrt(kPi) * x * std::exp(-x * x);
 }
 
-// Coefficients c[0..deg] in u on [0, 1] of the polynomial through fn at the
-// deg + 1 Chebyshev nodes (Newton's divided differences, then expanded).
-template <typename F> static void fit_interval(F &&fn, int deg, double *c) {
-  double u[8], d[8];
-  for (int k = 0; k <= deg; k++) {
-    u[k] = 0.5 - 0.5 * std::cos(kPi * (k + 0.5) / (deg + 1));
-    d[k] = fn(u[k]);
-  }
-  for (int j = 1; j <= deg; j++)
-    for (int k = deg; k >= j; k--) d[k] = (d[k] - d[k - 1]) / (u[k] - u[k - j]);
-  for (int k = 0; k <= deg; k++) c[k] = 0.0;
-  for (int k = deg; k >= 0; k--) {  // c <- c (u - u_k) + d_k
-    for (int i = deg; i > 0; i--) c[i] = c[i - 1] - u[k] * c[i];
-    c[0] = d[k] - u[k] * c[0];
-  }
-}
-
 // Interval edge: the largest power of two with k h <= 1/22 (1/8 A, 96
 // intervals at k = 0.34, r_off = 12), where the cubic's interpolation error is
-// at most 2e-8 of f(0) (1.5e-8 at k h = 0.0425), below FP32 rounding, and
-// degree 5 reaches 1.2e-12 in FP64.  At least 1/64 A (r^-12 of a pair in units of
-// h stays in FP32 range), 64 to 512 intervals (1 to 8 KB of LDS in FP32).  A
-// power of two changes no mantissa against A, so neither the unit factor's
-// rounding nor the reciprocal square root's error at the distances that
-// dominate the force moves (with h = r_off / 128 the direct forces' error was
-// 8 % larger).
+// at most 2e-8 of f(0) (1.5e-8 at k h = 0.0425), below FP32 rounding.  At least
+// 1/64 A (r^-12 of a pair in units of h stays in FP32 range), 64 to 512
+// intervals (1 to 8 KB of LDS).  A power of two changes no mantissa against A,
+// so neither the unit factor's rounding nor the reciprocal square root's error
+// at the distances that dominate the force moves (with h = r_off / 128 the
+// direct forces' error was 8 % larger).
 // Systems the table does not serve that well form the factor from erfc and exp
 // (tab_direct): where 512 intervals or 1/64 A do not give k h <= 1/22; beyond
 // k = 1, where a pair's f is so small that the rounding of r (2 (k r)^2 of f)
@@ -62,19 +44,16 @@ void NbSystem::make_pair_tables() {
   tab_direct = xh > 1.0 / 22.0 || kappa > 1.0 || kappa * ctofnb > 12.0;
   if (tab_direct) tab_n = 0;  // one entry, not read
   std::vector<float4> t(tab_n + 1);
-  std::vector<double2> td(3 * (size_t)(tab_n + 1)), te(td.size());
   for (int k = 0; k <= tab_n; k++) {
-    auto fn = [&](double u) { return coulomb_f(xh * (k + u)); };
-    double c[6];
-    fit_interval(fn, 3, c);
+    double c[4];
+    fit_interval<double>([&](double u) { return coulomb_f(xh * (k + u)); }, 3, c);
     t[k] = make_float4((float)c[0], (float)c[1], (float)c[2], (float)c[3]);
-    fit_interval(fn, 5, c);
-    for (int i = 0; i < 3; i++) td[3 * (size_t)k + i] = make_double2(c[2 * i], c[2 * i + 1]);
-    fit_interval([&](double u) { return std::erfc(xh * (k + u)); }, 5, c);
-    for (int i = 0; i < 3; i++) te[3 * (size_t)k + i] = make_double2(c[2 * i], c[2 * i + 1]);
   }
   ewtab.upload(t, 0);
-  ewtab_d.upload(td, 0);
+  erfc_per = erfc_intervals(kappa, ctofnb);
+  const bool f64 = precision == 1;
+  const auto te = erfc_table(tab_direct ? 0.0 : kappa * ctofnb, erfc_per, f64);
+  erfc_n = (int)te.size() / erfc_stride(f64) - 1;
   erfctab.upload(te, 0);
 }
 
@@ -133,6 +112,8 @@ void NbSystem::make_pair_consts() {
     pu.kappa2 = (T)(kappa * h * kappa * h);
     pu.two_kappa_sqrtpi = (T)(2.0 * kappa * h / std::sqrt(kPi));
     pu.ntab = tab_n;
+    pu.es = erfc_per * kappa * h;
+    pu.nerfc = erfc_n;
   };
   units(pu_f);
   units(pu_d);

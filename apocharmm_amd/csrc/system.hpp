@@ -5,6 +5,7 @@
 
 #include "apocharmm_amd.h"
 #include "common.hpp"
+#include "coulomb_table.hpp"
 
 namespace apo {
 
@@ -37,14 +38,16 @@ struct NbSystem {
   int ntypes = 0;
   DevBuf<int> vdwtype;
   // Coulomb part of the pair kernel: f(r) = erfc(k r) + 2 k r / sqrt(pi)
-  // exp(-k^2 r^2), so that r dU/dr = -qq f / r, as polynomials over tab_n
-  // equal intervals of edge tab_h (pair.hip); cubic in FP32, degree 5 in FP64
+  // exp(-k^2 r^2), so that r dU/dr = -qq f / r: in FP32 cubics over tab_n equal
+  // intervals of edge tab_h, the pair kernel's length unit
   double tab_h = 0;
   int tab_n = 0;
   bool tab_direct = false;  // no table: f from erfc and exp (make_pair_tables)
   DevBuf<float4> ewtab;
-  DevBuf<double2> ewtab_d;  // 3 per entry
-  DevBuf<double2> erfctab;  // erfc(k r) likewise, for the pair energies
+  // in FP64 erfc(k r), which gives the pair energies and f (coulomb_table.hpp)
+  int erfc_n = 0;
+  double erfc_per = 0;  // intervals per unit of k r
+  DevBuf<CoefPair> erfctab;
   // vdW tables of the pair kernel, in units of tab_h (6*c6, 12*c12)
   DevBuf<float2> vdwtab;
   DevBuf<float2> vdwtab14;    // 1-4 pairs, in A

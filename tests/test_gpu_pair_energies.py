@@ -122,8 +122,10 @@ def _check(kappa, off, box, ntypes, precision):
     fm.close()
 
 
-# without a table: kappa above 1, kappa r_off above 12
-RANGE = [(0.9, 14.0), (2.0, 7.0), (3.0, 12.0), (3.0, 1.9), (5.0, 12.0), (8.0, 4.5)]
+RANGE = [(1e-4, 12.0), (0.1, 12.0), (0.34, 12.0), (0.34, 11.93), (0.34, 15.0), (0.4, 9.0),
+         (0.5, 12.0), (0.5, 1.9), (1.0, 12.0),
+         # without a table: kappa above 1, kappa r_off above 12
+         (0.9, 14.0), (2.0, 7.0), (3.0, 12.0), (3.0, 1.9), (5.0, 12.0), (8.0, 4.5)]
 
 
 @pytest.mark.parametrize("kappa,off", RANGE)
@@ -132,11 +134,14 @@ def test_pairs_over_the_range(kappa, off, precision):
     _check(kappa, off, (32.0, 32.0, 32.0), 2, precision)
 
 
-@pytest.mark.parametrize("ntypes", [24, 64, 200])
+# 2 types: switched coefficients per type pair; 24: square table; 64: triangle;
+# 200: combination rule (FP32) or the global table (FP64)
+@pytest.mark.parametrize("ntypes", [2, 24, 64, 200])
 @pytest.mark.parametrize("box", [(32.0, 32.0, 32.0), (32.0, 64.0, 32.0)])
 @pytest.mark.parametrize("precision", ["mixed", "fp64"])
 def test_pairs_of_every_layout(box, ntypes, precision):
-    _check(3.0, 12.0, box, ntypes, precision)
+    for kappa, off in ((0.34, 12.0), (3.0, 12.0)):
+        _check(kappa, off, box, ntypes, precision)
 
 
 def test_steps_and_batches_without_a_table():
