@@ -513,6 +513,32 @@ __device__ __forceinline__ void pair_body(
       }
     }
   }
+  if (CALC_E && __any(acc[0] != acc[0])) {
+    // Two atoms at one place: the third-order root and the table gave NaN for
+    // the pair, whose Coulomb energy is infinite.  The wave's items are gone
+    // through again for such pairs, here and not in the loop above, which has no
+    // registers to spare for it (50 spilled, 360 -> 463 us at 93,984 atoms).
+    bool same = false;
+    double sum = 0.0;
+#pragma unroll 1
+    for (int p = bid; p < nitem; p += nb) {
+      const int4 it = items[iorder[p]];
+#pragma unroll 1
+      for (int e0 = it.y; e0 < it.z; e0 += 64) {
+        const uint32_t e = ent[e0 + lane];
+        const int4 pj = posq[cand_j[it.w + ((e & 0xffffu) >> 5)] * kCell + (e & 31u)];
+#pragma unroll 1
+        for (int k = 0; k < kGroup; k++) {
+          const int4 pi = posq[it.x * kGroup + k];
+          if (!(e >> (16 + k) & 1u) && pi.x == pj.x && pi.y == pj.y && pi.z == pj.z) {
+            same = true;
+            sum += (double)charge_of<CT>(pi.w) * (double)charge_of<CT>(pj.w) * INFINITY;
+          }
+        }
+      }
+    }
+    if (same) acc[0] = sum;
+  }
   if (CALC_E || CALC_V) {
 #pragma unroll
     for (int k = 0; k < kPairPart; k++) {
@@ -527,8 +553,9 @@ __device__ __forceinline__ void pair_body(
 }
 
 // Energy calls in mixed precision: three waves per SIMD (168 VGPRs; 179 without
-// the bound, which leaves two).  FP64: two (the energy and virial variant takes
-// 260 without the bound, one wave: 253 us for a call of 22,287 atoms, with it 208).
+// the bound, which leaves two).  FP64: two (without the bound the energy and
+// virial variant went past 256 VGPRs to one wave: 253 us for a call of 22,287
+// atoms, with it 208).
 template <typename CT, bool CALC_E, bool CALC_V, int TAB, bool ISO, bool PRUNE>
 __global__ __launch_bounds__(64, sizeof(CT) == sizeof(double) ? 2 : CALC_E ? 3 : 1) void k_pair(
     const int4 *__restrict__ posq, const int *__restrict__ types, const int4 *__restrict__ items,

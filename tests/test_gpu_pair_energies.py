@@ -122,6 +122,22 @@ def _check(kappa, off, box, ntypes, precision):
     fm.close()
 
 
+@pytest.mark.parametrize("kappa", [0.34, 3.0])
+@pytest.mark.parametrize("precision", ["mixed", "fp64"])
+def test_atoms_at_one_place(kappa, precision):
+    """An infinite Coulomb energy of the product's sign, as 1 / r gives it."""
+    from apocharmm_amd.force_manager import ForceManager
+    print("coincident atoms", kappa, precision, flush=True)
+    spec = _spec(kappa, 12.0, (32.0, 32.0, 32.0), 2, np.random.default_rng(1))
+    fm = ForceManager(spec, precision).initialize()
+    x = torch.full((2, 4), 5.0, device="cuda")
+    for q, want in ((-Q, -np.inf), (Q, np.inf)):
+        x[0, 3], x[1, 3] = Q, q
+        fm.calcForce(x, reset=True, calcEnergy=True, terms=_lib.APO_TERM_DIRECT)
+        assert fm.getEnergyComponents()["elec"] == want
+    fm.close()
+
+
 RANGE = [(1e-4, 12.0), (0.1, 12.0), (0.34, 12.0), (0.34, 11.93), (0.34, 15.0), (0.4, 9.0),
          (0.5, 12.0), (0.5, 1.9), (1.0, 12.0),
          # without a table: kappa above 1, kappa r_off above 12
