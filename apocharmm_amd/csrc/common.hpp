@@ -303,9 +303,13 @@ void bonded_launch(NbSystem &sys, const float4 *d_xyzq, int64_t *d_force, int st
                    bool virial, bool pairs14, bool bonded, hipStream_t s);
 // fold: the gather also adds the sorted pair gradient (direct_finalize), whose
 // kernel must precede this call on the same stream; shared: the pair kernel
-// runs beside the chain
+// runs beside the chain (or may, in calls of this system with energies), which
+// decides the route of the transforms
 void recip_launch(NbSystem &sys, const float4 *d_xyzq, int64_t *d_force,
                   int stride, bool energy, bool virial, hipStream_t s, bool fold, bool shared);
+// Whether the transforms of a call that is not shared take planes that do not
+// fit in LDS beside the pair kernel's waves.
+bool pme_waits_for_pairs(const NbSystem &sys);
 // Adds up the partials the terms of this call wrote (and the self energy).
 void reduce_energy_launch(NbSystem &sys, const float4 *d_xyzq, int term_mask, bool energy,
                           bool virial, double *d_energy, double *d_virial,

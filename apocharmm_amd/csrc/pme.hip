@@ -1277,6 +1277,17 @@ static void recip_t(NbSystem &S, const float4 *x, int64_t *force, int stride, bo
   S.toc(3, s, t0);
 }
 
+bool pme_waits_for_pairs(const NbSystem &S) {
+  auto waits = [&](auto ct) {
+    using CT = decltype(ct);
+    auto plane = [&](bool shared) {
+      return pme_shapes<CT>(S, kFftRowsPerBlock, kFftColsPerBlock, kFftThreads, false, shared).plane;
+    };
+    return plane(false) && !plane(true);
+  };
+  return S.precision == 1 ? waits(double()) : waits(float());
+}
+
 void recip_launch(NbSystem &S, const float4 *x, int64_t *force, int stride, bool E, bool V,
                   hipStream_t s, bool fold, bool shared) {
   // the issue priority is a template parameter: as a kernel argument, every

@@ -536,7 +536,10 @@ void set_box(NbSystem &S, const double *b) {
 // side stream, from kForkAtoms up (one stream / fork: 127 / 131 us at 21,525
 // atoms, 146 / 148 at 28,731, 159 / 152 at 37,086, 181 / 165 at 45,852; with the
 // virial 176 / 188 at 26,988) and with energies, whose pair kernel is longer,
-// from kForkAtomsE (211 / 217, 243 / 233, 265 / 245, 287 / 279 at those sizes).  Merging saves a launch and fills the
+// from kForkAtomsE (211 / 217, 243 / 233, 265 / 245, 287 / 279 at those sizes).
+// Captured calls fork at any size, except for energies or a virial where the PME
+// branch would wait for the pair kernel all the same (pme_waits_for_pairs).
+// Merging saves a launch and fills the
 // drain of the pair items, but its latency-bound waves take pair-wave slots: in
 // captured steps it pays up to kMergeAtoms (apart / merged, 40 MD steps: 3,369 /
 // 3,186 us at 3,708 atoms, 3,324 / 3,243 at 8,061, 3,583 / 3,630 at 11,748),
@@ -544,15 +547,22 @@ void set_box(NbSystem &S, const double *b) {
 constexpr int kForkAtoms = 33000, kForkAtomsE = 25000, kMergeAtoms = 10000;
 struct BranchPlan {
   bool fork, merge, bonded2;
+  bool shared;  // recip_launch
 };
 static BranchPlan plan_branches(const NbSystem &S, hipStream_t s, bool dir, bool rec, bool bnd,
                                 bool E, bool V) {
-  BranchPlan p{false, false, false};
+  BranchPlan p{false, false, false, false};
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(s, &cap) != hipSuccess) (void)hipGetLastError();
   const bool captured = cap != hipStreamCaptureStatusNone;
+  const bool ev = E || V;
+  // the order in which energies and the virial are summed follows the route of
+  // the transforms, so with them it is a matter of the system alone
+  const bool ev_shared = S.natom >= kForkAtomsE;
   p.fork = dir && rec && !S.single_stream &&
-           (captured || S.natom >= (E ? kForkAtomsE : kForkAtoms));
+           (S.natom >= (E ? kForkAtomsE : kForkAtoms) ||
+            (captured && !(ev && !ev_shared && pme_waits_for_pairs(S))));
+  p.shared = ev ? ev_shared : p.fork;
   // kernel timers on: a launch of their own, so that slot 6 times them
   p.merge = bnd && dir && !E && !V && !S.prof_on && (!p.fork || S.natom < kMergeAtoms);
   p.bonded2 = p.fork && captured && bnd && !p.merge;
@@ -642,7 +652,7 @@ void calc_force(NbSystem &S, const float *xyzq, int flags, int64_t *force, int s
     if (with_pair) bonded_branch(sd);
     pair_branch();
   }
-  if (rec) recip_launch(S, x4, force, stride, E, V, sp, fold, plan.fork);
+  if (rec) recip_launch(S, x4, force, stride, E, V, sp, fold, plan.shared);
   if (own && !with_pair) {
     bonded_branch(plan.bonded2 ? S.side[1] : sp);
     if (plan.bonded2) APO_HIP(hipEventRecord(S.ev_bond, S.side[1]));
