@@ -756,7 +756,8 @@ __global__ __launch_bounds__(kItemThreads) void k_list_guard_export(
     const int *__restrict__ icell_start, int *__restrict__ grp_itemstart,
     int4 *__restrict__ items, int *__restrict__ order, int isteps) {
   constexpr int kW = kItemThreads / 64;
-  static_assert(kItemSteps <= 64, "one lane per item length");
+  static_assert(kItemSteps < 64 && (kItemSteps & (kItemSteps - 1)) == 0,
+                "one lane per item length from 0 to kItemSteps, lengths compared bit by bit");
   __shared__ int sh_hist[kW][64];  // [wave][length]; length isteps: the full items
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const unsigned long long below = (1ull << lane) - 1ull;
