@@ -1,4 +1,4 @@
-"""Energies and virial of one system and one list have the same bits however the
+"""Energies, virial and gradient of one system and one list have the same bits however a
 call runs: on one stream or forked, captured in a graph (replayed with eager work
 in between), with kernel timers, as a member of a batch, and for the reciprocal
 term on its own.  Their sums are ordered by the kernels' blocks, so the route of
@@ -58,11 +58,12 @@ def test_energies_and_virial_of_every_route(name, precision):
         fm.calcForce(x, calcEnergy=energy, calcVirial=virial, **kw)
 
     call()
-    want, vir = fm.getEnergyComponents(), fm.getVirial()
+    want, vir, grad = fm.getEnergyComponents(), fm.getVirial(), fm.force.clone()
     assert np.isfinite(want["epot"])
 
     def check(what, energy=True, virial=True):
         torch.cuda.synchronize()
+        assert torch.equal(fm.force, grad), what
         if energy:
             assert fm.getEnergyComponents() == want, what
         if virial:
@@ -70,6 +71,8 @@ def test_energies_and_virial_of_every_route(name, precision):
 
     call(virial=False)
     check("energies alone", virial=False)
+    call(energy=False, virial=False)
+    check("forces alone", energy=False, virial=False)
     _lib.check(_lib.lib().apo_nb_profile(fm._handle, 1))
     call()
     _lib.check(_lib.lib().apo_nb_profile(fm._handle, 0))
