@@ -1,5 +1,6 @@
 // Launches of the bonded terms and the 1-4 / exclusion pairs (bodies in
-// bonded_terms.hpp): energy and virial calls, and fused batches.
+// bonded_terms.hpp) that do not ride in the pair kernel's: energy and virial
+// calls, forked force calls from 10,000 atoms, and fused batches.
 #include "bonded_terms.hpp"
 
 namespace apo {

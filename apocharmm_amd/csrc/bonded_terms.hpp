@@ -5,9 +5,9 @@
 // and calc_14_force_kernel (src/CudaDirectForceKernels.cu:640-870): no cutoff
 // and no periodic image for these lists (ishift 13 in the reference).
 // One thread per term, FP32 (or FP64) math, int64 2^-40 atomics, per-block
-// FP64 energy/virial partials reduced later in fixed order.  Force calls run
-// them in the pair kernel's launch (pair.hip), energy and virial calls and
-// fused batches in launches of their own (bonded.hip).
+// FP64 energy/virial partials reduced later in fixed order.  They run in the pair
+// kernel's launch (pair.hip) or in launches of their own (bonded.hip), as
+// plan_branches (system.hip) decides.
 #pragma once
 
 #include <cmath>

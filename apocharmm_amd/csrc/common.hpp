@@ -236,7 +236,6 @@ struct PartLayout {
   int bond_off = 0, bond_n = 0;
   int recip_off = 0, recip_n = 0;
   int recip_used = 0;  // rows the convolution writes (recip_n are reserved)
-  int self_off = 0, self_n = 0;
   int total = 0;
 };
 

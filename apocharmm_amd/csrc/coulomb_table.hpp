@@ -5,7 +5,6 @@
 //        = erfc(k r) + 2 k r / sqrt(pi) exp(-k^2 r^2)
 #pragma once
 
-#include <algorithm>
 #include <cmath>
 #include <vector>
 

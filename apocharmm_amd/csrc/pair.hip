@@ -39,10 +39,10 @@ __device__ __forceinline__ unsigned long long fx_round(double v) {
 // ntab + 1 (the last entry serves r that rounds up to r_off).
 // This is one 16-byte LDS read and six instructions where exp2, rcp and
 // a degree-8 erfc polynomial took about twenty issue slots (VALU instructions
-// of one launch at 93,984 atoms 73.2 M -> 62.9 M).  Kernel alone: 140 -> 134 us
-// there, 57 -> 49 with the virial at 26,988 atoms.  What bounds it then is the
-// latency of one pair's chain (rsq, table read, cubic) over the four waves a
-// SIMD holds.
+// per launch of the 98,304-atom step 71.8 M -> 60.1 M, the charges' row broadcast
+// below included).  Kernel alone: 140 -> 134 us at 93,984 atoms, 57 -> 49 with
+// the virial at 26,988.  What bounds it then is the latency of one pair's chain
+// (rsq, table read, cubic) over the four waves a SIMD holds: VALU 69 % busy.
 __device__ __forceinline__ float coulomb_factor(const float4 *tab, float r) {
   const float4 c = tab[(unsigned)r];
   const float u = __builtin_amdgcn_fractf(r);
@@ -420,9 +420,10 @@ __device__ __forceinline__ void pair_body(
             // dominate the energy error.  FP64 issue bounds this block:
             // erfc(k r) from its table (erfc_factors), the reciprocal root by
             // one third-order step and, with TAB_PQA, one polynomial in r^-3
-            // per region replace libm's erfc, a square root and a divide (kernel with energies and virial, alone: 616 -> 246
-            // us at 93,984 atoms, 191 -> 104 in DHFR, 42 -> 23 at 2,529; all
-            // FP64 154 -> 68 at 11,748)
+            // per region replace libm's erfc, a square root and a divide
+            // (kernel with energies and virial, alone: 616 -> 271 us at 93,984
+            // atoms, 191 -> 112 in DHFR, 42 -> 24 at 2,529; all FP64, whose
+            // forces left libm too, 207 -> 71 at 11,748)
             double er2, erinv;
             if constexpr (F64) {
               er2 = r2;

@@ -270,10 +270,10 @@ __device__ __forceinline__ void fft_stage(const C2 *in, C2 *out, int n, int nrow
 // Returns the buffer holding the result.
 // Always inlined: as a called function it makes every caller allocate the
 // callee's worst-case register budget (262 VGPRs, one wave per SIMD).
-// BIG: the plan may hold radices 7, 11 or 13.  Their generic DFT sets the
-// register budget of every kernel that contains it (the y pass needs 94
-// VGPRs with them, 44 without), so the launchers pick the variant without
-// them whenever every radix of the plans is at most 5 (plan_big).
+// BIG: the plan may hold radices 7, 11 or 13.  Their stages set the register
+// budget of every kernel that contains them (y pass 64 VGPRs with them,
+// 45 without), so the launchers pick the variant without them whenever no
+// plan has such a radix (plan_big).
 // X: the x transforms, whose plans do not use 6 and 8 (make_fft_dim): without
 // those stages the spread, which holds the transform beside its own registers,
 // spills less.
@@ -340,16 +340,6 @@ __device__ __forceinline__ void staged_copy(int total, int tid, int nthreads, Lo
 // ---------------------------------------------------------------------------
 // B-splines and fractional coordinates
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ void frac_coord(float x, double inv_len, int K, int &ix, double &w) {
-  const double ww = (double)x * inv_len + 2.0;
-  double fr = (double)K * (ww - (floor(ww + 0.5) - 0.5));
-  // fr = K is the periodic image of 0; non-finite input maps to 0 so every
-  // grid index stays in range
-  if (!(fr >= 0.0 && fr < (double)K)) fr = 0.0;
-  ix = (int)fr;
-  w = fr - (double)ix;
-}
-
 // Order-4 Cardinal B-spline weights (and derivatives) at offset w.
 template <typename CT>
 __device__ __forceinline__ void bspline4(CT w, CT (&th)[4], CT (&dth)[4]) {
@@ -482,13 +472,6 @@ __device__ __forceinline__ Theta6 theta6_coef(int t) {
 }
 __device__ __forceinline__ double theta6(const Theta6 &c, double w) {
   return fma(fma(fma(c.c3, w, c.c2), w, c.c1), w, c.c0);
-}
-
-__device__ __forceinline__ double readlane_f64(double v, int k) {
-  const long long b = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_readlane((int)(b & 0xffffffffll), k);
-  const int hi = __builtin_amdgcn_readlane((int)(b >> 32), k);
-  return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
 }
 
 // Whether stencil row p >= -3 (from the slab's first row) lies in a slab of B
@@ -1399,7 +1382,7 @@ struct PmeBatch {
   BatchLaunch<FftzArgs> fz;
   BatchLaunch<GatherArgs> gather;
   int ft = kFftThreads;  // threads per block of the y, z and x-inverse passes
-  bool big = false;      // some system's plans need radices above 5 (plan_big)
+  bool big = false;      // some system's plans need radix 7, 11 or 13 (plan_big)
   bool wrap = false;     // some system's spread wraps (PmeShapes::wrap)
 };
 

@@ -499,7 +499,6 @@ NbSystem *create_system(const apo_nb_params &p, const apo_nb_topology &t) {
     // for the worst case W = 1 (the reduction reads the rows written)
     S->zconv_blocks = S->K[1] * (S->K[0] / 2 + 1);
     L.recip_off = off; L.recip_n = S->zconv_blocks; off += L.recip_n * kRecipPart;
-    L.self_off = off; L.self_n = std::max(1, (n + 255) / 256); off += L.self_n;
     L.total = off;
     S->parts.reserve(off);
     S->red_sums.reserve(reduce_sums_size(L, n));
@@ -523,11 +522,11 @@ void set_box(NbSystem &S, const double *b) {
 
 // How a call runs its three branches: the pair kernel, the PME chain and the
 // bonded and 1-4 terms.
-//  * one_stream: one after the other on the caller's stream (small eager calls);
-//  * otherwise the PME chain stays on the caller's stream, behind the sort, so
-//    that the spread's blocks are resident before the pair kernel on the side
-//    stream takes the wave slots (the other way round the spread starved:
-//    force call 277 -> 253 us at 93,984 atoms);
+//  * without fork one after the other on the caller's stream (small eager calls);
+//  * fork: the PME chain stays on the caller's stream, behind the sort, so that
+//    the spread's blocks are resident before the pair kernel on the side stream
+//    takes the wave slots (the other way round the spread starved: force call
+//    277 -> 253 us at 93,984 atoms);
 //  * merge: the bonded terms' blocks run in the pair kernel's launch;
 //  * bonded2: they have a side stream of their own (captured calls, where the
 //    events cost the host nothing).
@@ -539,11 +538,11 @@ void set_box(NbSystem &S, const double *b) {
 // from kForkAtomsE (211 / 217, 243 / 233, 265 / 245, 287 / 279 at those sizes).
 // Captured calls fork at any size, except for energies or a virial where the PME
 // branch would wait for the pair kernel all the same (pme_waits_for_pairs).
-// Merging saves a launch and fills the
-// drain of the pair items, but its latency-bound waves take pair-wave slots: in
-// captured steps it pays up to kMergeAtoms (apart / merged, 40 MD steps: 3,369 /
-// 3,186 us at 3,708 atoms, 3,324 / 3,243 at 8,061, 3,583 / 3,630 at 11,748),
-// on one stream at every size (130 -> 128 us at 23,558).
+// Merging saves a launch and fills the drain of the pair items, but its
+// latency-bound waves take pair-wave slots: in captured steps it pays up to
+// kMergeAtoms (apart / merged, 40 MD steps: 3,369 / 3,186 us at 3,708 atoms,
+// 3,324 / 3,243 at 8,061, 3,583 / 3,630 at 11,748), on one stream at every size
+// (130 -> 128 us at 23,558).
 constexpr int kForkAtoms = 33000, kForkAtomsE = 25000, kMergeAtoms = 10000;
 struct BranchPlan {
   bool fork, merge, bonded2;

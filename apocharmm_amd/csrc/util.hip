@@ -1,4 +1,4 @@
-// Small device utilities: fills, single-block scans, fixed-point conversion
+// Small device utilities: fills, fixed-point conversion
 // and the final fixed-order energy/virial reduction (self energy included).
 #include <algorithm>
 #include <cmath>
