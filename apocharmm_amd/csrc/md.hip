@@ -1171,10 +1171,11 @@ struct LtSystem {
         builds_triggered++;
         steps_since_rebuild = 0;
       }
-      // prune on the schedule, and whenever the pruned copy belongs to an
-      // earlier build (a rebuild outside this integrator, a fused batch)
+      // prune on the schedule, which starts anew at every build (as in
+      // run_cycle), and whenever the pruned copy belongs to an earlier build (a
+      // rebuild outside this integrator, a fused batch)
       const bool prune = !rebuild && prune_every > 0 &&
-                         (steps_since_rebuild % prune_every == 0 ||
+                         (steps_since_rebuild % nbfreq % prune_every == 0 ||
                           nb->pruned_build != nb->builds_queued);
       const bool com = comfreq > 0 && step % (unsigned long long)comfreq == 0;
       // centre-of-mass removal only touches the half-step displacements, so
