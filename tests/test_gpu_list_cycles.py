@@ -1,6 +1,6 @@
-"""List cycles run as recorded graphs or step by step: every mix of the two has to
-give the trajectory of eager stepping bit for bit, also where the prune interval
-does not divide the list interval."""
+"""List cycles run as recorded graphs or, the first time at given launch constants,
+step by step: every mix of the two has to give the trajectory of eager stepping
+bit for bit, also where the prune interval does not divide the list interval."""
 import numpy as np
 import pytest
 
@@ -39,3 +39,8 @@ def _run(pieces, prune, comfreq, graph=True, setting=0):
 @pytest.mark.parametrize("pieces", [(5 * NB,), (NB,) * 5, (NB, 3 * NB, NB), (2 * NB, 3 * NB)])
 def test_stepped_and_recorded_cycles(pieces, prune, comfreq):
     assert _run(pieces, prune, comfreq) == _run(pieces, prune, comfreq, graph=False)
+
+
+def test_the_trial_of_launch_settings():
+    # 16 trial cycles, then one step by step, then recorded ones
+    assert _run((20 * NB,), 4, 0, setting=None) == _run((20 * NB,), 4, 0, graph=False)
