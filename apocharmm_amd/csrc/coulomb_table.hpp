@@ -10,23 +10,29 @@
 
 namespace apo {
 
-// Coefficients c[0..deg] in u on [0, 1] of the polynomial through fn at the
-// deg + 1 Chebyshev nodes (Newton's divided differences, then expanded).
-template <typename T, typename F> void fit_interval(F &&fn, int deg, T *c) {
-  T u[16], d[16];
-  const T pi = std::acos((T)-1);
-  for (int k = 0; k <= deg; k++) {
-    u[k] = (T)0.5 - (T)0.5 * std::cos(pi * (k + (T)0.5) / (deg + 1));
-    d[k] = fn(u[k]);
+// Polynomials of degree deg through the deg + 1 Chebyshev nodes of [0, 1].
+template <typename T> struct IntervalFit {
+  int deg;
+  T u[16];
+  explicit IntervalFit(int degree) : deg(degree) {
+    const T pi = std::acos((T)-1);
+    for (int k = 0; k <= deg; k++)
+      u[k] = (T)0.5 - (T)0.5 * std::cos(pi * (k + (T)0.5) / (deg + 1));
   }
-  for (int j = 1; j <= deg; j++)
-    for (int k = deg; k >= j; k--) d[k] = (d[k] - d[k - 1]) / (u[k] - u[k - j]);
-  for (int k = 0; k <= deg; k++) c[k] = 0;
-  for (int k = deg; k >= 0; k--) {  // c <- c (u - u_k) + d_k
-    for (int i = deg; i > 0; i--) c[i] = c[i - 1] - u[k] * c[i];
-    c[0] = d[k] - u[k] * c[0];
+  // Coefficients c[0..deg] in u of the one through fn (Newton's divided
+  // differences, then expanded).
+  template <typename F> void operator()(F &&fn, T *c) const {
+    T d[16];
+    for (int k = 0; k <= deg; k++) d[k] = fn(u[k]);
+    for (int j = 1; j <= deg; j++)
+      for (int k = deg; k >= j; k--) d[k] = (d[k] - d[k - 1]) / (u[k] - u[k - j]);
+    for (int k = 0; k <= deg; k++) c[k] = 0;
+    for (int k = deg; k >= 0; k--) {  // c <- c (u - u_k) + d_k
+      for (int i = deg; i > 0; i--) c[i] = c[i - 1] - u[k] * c[i];
+      c[0] = d[k] - u[k] * c[0];
+    }
   }
-}
+};
 
 // ---- FP64: g, and f from its value and derivative ---------------------------
 // Polynomials on intervals of k r = 1/16, of degree 11 where f is wanted too
@@ -60,10 +66,10 @@ inline std::vector<CoefPair> erfc_table(double xmax, double per, bool force) {
   std::vector<CoefPair> c((size_t)(n + 1) * erfc_stride(force));
   // extended precision: f multiplies the derivative by r in intervals, and with
   // it the rounding of the fitted values
+  const IntervalFit<long double> fit(deg);
   long double p[kErfcDegF + 1];
   for (int k = 0; k <= n; k++) {
-    fit_interval<long double>([&](long double u) { return std::erfc((k + u) / (long double)per); },
-                              deg, p);
+    fit([&](long double u) { return std::erfc((k + u) / (long double)per); }, p);
     for (int i = 0; i < deg; i += 2)
       c[(size_t)k * erfc_stride(force) + i / 2] = CoefPair{(double)p[i], (double)p[i + 1]};
   }

@@ -44,9 +44,10 @@ void NbSystem::make_pair_tables() {
   tab_direct = xh > 1.0 / 22.0 || kappa > 1.0 || kappa * ctofnb > 12.0;
   if (tab_direct) tab_n = 0;  // one entry, not read
   std::vector<float4> t(tab_n + 1);
+  const IntervalFit<double> fit(3);
   for (int k = 0; k <= tab_n; k++) {
     double c[4];
-    fit_interval<double>([&](double u) { return coulomb_f(xh * (k + u)); }, 3, c);
+    fit([&](double u) { return coulomb_f(xh * (k + u)); }, c);
     t[k] = make_float4((float)c[0], (float)c[1], (float)c[2], (float)c[3]);
   }
   ewtab.upload(t, 0);
